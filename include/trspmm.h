@@ -381,7 +381,9 @@ void trs_plan_free(trs_plan* p);
  * Execution.
  * ------------------------------------------------------------------------------------------- */
 /* Bytes of device workspace trs_spmm_f16 needs for feature width K (0 when none): the partial
- * slots of split rows and, for K >= 128, the plan's staged hot B rows (option hot_rows). */
+ * slots of split rows and, for K >= 128, the plan's staged hot B rows (option hot_rows).  For K that 8
+ * does not divide the staged rows (odd K >= 65, even K >= 104) are optional: a workspace that only
+ * holds the partial slots is accepted, and the call then runs without them, the same bits. */
 int64_t trs_spmm_workspace_bytes(const trs_plan* p, int32_t K);
 
 /* C[m, K] (float32, row stride ldc) = A_plan (m x n) * B[n, K] (fp16, row stride ldb).
@@ -395,7 +397,8 @@ int trs_spmm_f16(const trs_plan* p, const uint16_t* B, int64_t ldb, int32_t K, f
  * the reference.  The workspace (partial slots, staged hot rows) comes from a static device array of
  * TRS_NOALLOC_SCRATCH_BYTES,
  * which every GPU the library runs on holds until the process ends; the call allocates nothing.
- * Plans whose trs_spmm_workspace_bytes(p, K) exceeds that size are refused with TRS_EINVAL.  All
+ * Plans whose trs_spmm_workspace_bytes(p, K), without optional staged rows, exceeds that size are
+ * refused with TRS_EINVAL.  All
  * calls on one GPU share its array: calls that overlap on one GPU race (serialise them).  Same
  * kernels and arguments as trs_spmm_f16, so the output is bitwise equal to it.  The first call on
  * each device looks the array's address up (hipGetSymbolAddress): make that call outside stream
@@ -415,7 +418,8 @@ int trs_sddmm_f16(const trs_plan* p, const uint16_t* X, int64_t ldx, const uint1
 /* Bytes of device workspace trs_sddmm_f16_ws uses at feature width K: from K = 128, an output
  * buffer for the plan's split part (XCD sub-rows of its long rows, merged into place at the end of
  * the call) and the plan's staged hot Y rows (plan option hot_rows); 0 when the plan or K uses
- * neither.  No reference counterpart. */
+ * neither.  For K that 8 does not divide the staged rows (K >= 121) are optional, as for the SpMM.
+ * No reference counterpart. */
 int64_t trs_sddmm_workspace_bytes(const trs_plan* p, int32_t K);
 
 /* trs_sddmm_f16 with a workspace of trs_sddmm_workspace_bytes(p, K) bytes (fewer: TRS_EINVAL):

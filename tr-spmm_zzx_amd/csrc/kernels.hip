@@ -4,7 +4,7 @@
 //   k_spmm_tasks    residual CSR.  A "lane group" of LPG lanes owns one task: a run of whole rows
 //                   (the entries streamed flat, rows flushed as their end is crossed) or one piece
 //                   of a long row.  Each lane holds VEC consecutive features (8, 4, 2 or 1:
-//                   16-, 8-, 4- or 2-byte loads, by K and alignment), so one B row of K fp16 is
+//                   16-, 8-, 4- or 2-byte loads, by K; any alignment), so one B row of K fp16 is
 //                   fetched by K/VEC lanes; U nonzeros are in flight per lane; narrow groups are
 //                   held to 2 or 4 waves per SIMD by dynamic LDS.  fp32 accumulation.  Replaces the reference residual kernels
 //                   (TR-source/SpMM/mGCNkernel.cu:976-1171, spmm_utils/compute.h:27-240), which
@@ -18,12 +18,12 @@
 //                   (mGCNkernel_online.cu:54-241, 812-933) and the add kernel (:1314-1324).
 // SDDMM (no reference counterpart):
 //   k_sddmm_tasks   residual entries: one lane group per task, per-entry dot products reduced
-//                   across the group; 16-, 8-, 4- or 2-byte loads of X and Y by K and alignment.
+//                   across the group; 16-, 8-, 4- or 2-byte loads of X and Y by K, any alignment.
 //   k_sddmm_mfma32  one wave per dense 16x16 tile: D = X[16 window rows] . Y[16 tile columns]^T
 //                   accumulated over K with gfx950's v_mfma_f32_16x16x32_f16 (both operands
 //                   contiguous in K, 16-byte loads straight from global), sampled at the tile's
-//                   stored entries; k_sddmm_mfma is the same with v_mfma_f32_16x16x16_f16 for K
-//                   that is not a multiple of 8.
+//                   stored entries; k_sddmm_mfma is the same with v_mfma_f32_16x16x16_f16 for
+//                   K < 8.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -47,8 +47,16 @@ typedef _Float16 half8_t __attribute__((ext_vector_type(8)));
 typedef _Float16 half16_t __attribute__((ext_vector_type(16)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
+// The same vectors at any element address: a global load or store of 4, 8 or 16 bytes needs no more
+// than its element's alignment on gfx950 (one instruction either way), so rows of any width and
+// leading dimension are read and written at full vector width.
+typedef half2_t half2_u __attribute__((aligned(2)));
+typedef half4_t half4_u __attribute__((aligned(2)));
+typedef half8_t half8_u __attribute__((aligned(2)));
+typedef float2_t float2_u __attribute__((aligned(4)));
+typedef float4_t float4_u __attribute__((aligned(4)));
 
-bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
+[[maybe_unused]] bool aligned16(const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
 // ------------------------------------------------------------------------------------------------
 // SpMM / SDDMM kernels and their launchers (the width parts only).
@@ -61,10 +69,10 @@ struct BFrag;
 template <>
 struct BFrag<8> {
   half8_t v;
-  __device__ __forceinline__ void load(const uint16_t* p) { v = *reinterpret_cast<const half8_t*>(p); }
+  __device__ __forceinline__ void load(const uint16_t* p) { v = *reinterpret_cast<const half8_u*>(p); }
   // non-temporal: the line is not kept in the caches for later readers
   __device__ __forceinline__ void load_nt(const uint16_t* p) {
-    v = __builtin_nontemporal_load(reinterpret_cast<const half8_t*>(p));
+    v = __builtin_nontemporal_load(reinterpret_cast<const half8_u*>(p));
   }
   __device__ __forceinline__ void zero() { v = half8_t{0, 0, 0, 0, 0, 0, 0, 0}; }
   __device__ __forceinline__ void fma(float (&acc)[8], float a) const {
@@ -83,7 +91,7 @@ struct BFrag<8> {
 template <>
 struct BFrag<4> {
   half4_t v;
-  __device__ __forceinline__ void load(const uint16_t* p) { v = *reinterpret_cast<const half4_t*>(p); }
+  __device__ __forceinline__ void load(const uint16_t* p) { v = *reinterpret_cast<const half4_u*>(p); }
   __device__ __forceinline__ void zero() { v = half4_t{0, 0, 0, 0}; }
   __device__ __forceinline__ void fma(float (&acc)[4], float a) const {
 #pragma unroll
@@ -100,7 +108,7 @@ struct BFrag<4> {
 template <>
 struct BFrag<2> {
   half2_t v;
-  __device__ __forceinline__ void load(const uint16_t* p) { v = *reinterpret_cast<const half2_t*>(p); }
+  __device__ __forceinline__ void load(const uint16_t* p) { v = *reinterpret_cast<const half2_u*>(p); }
   __device__ __forceinline__ void zero() { v = half2_t{0, 0}; }
   __device__ __forceinline__ void fma(float (&acc)[2], float a) const {
     acc[0] = __builtin_fmaf(a, (float)v[0], acc[0]);
@@ -123,25 +131,56 @@ __device__ __forceinline__ void store_vec(float* dst, const float (&acc)[VEC]) {
   if constexpr (VEC == 8) {
     const float4_t lo{acc[0], acc[1], acc[2], acc[3]}, hi{acc[4], acc[5], acc[6], acc[7]};
     if constexpr (NT) {
-      __builtin_nontemporal_store(lo, reinterpret_cast<float4_t*>(dst));
-      __builtin_nontemporal_store(hi, reinterpret_cast<float4_t*>(dst) + 1);
+      __builtin_nontemporal_store(lo, reinterpret_cast<float4_u*>(dst));
+      __builtin_nontemporal_store(hi, reinterpret_cast<float4_u*>(dst) + 1);
     } else {
-      reinterpret_cast<float4_t*>(dst)[0] = lo;
-      reinterpret_cast<float4_t*>(dst)[1] = hi;
+      reinterpret_cast<float4_u*>(dst)[0] = lo;
+      reinterpret_cast<float4_u*>(dst)[1] = hi;
     }
   } else if constexpr (VEC == 4) {
     const float4_t v{acc[0], acc[1], acc[2], acc[3]};
-    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<float4_t*>(dst));
-    else reinterpret_cast<float4_t*>(dst)[0] = v;
+    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<float4_u*>(dst));
+    else reinterpret_cast<float4_u*>(dst)[0] = v;
   } else if constexpr (VEC == 2) {
     const float2_t v{acc[0], acc[1]};
-    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<float2_t*>(dst));
-    else reinterpret_cast<float2_t*>(dst)[0] = v;
+    if constexpr (NT) __builtin_nontemporal_store(v, reinterpret_cast<float2_u*>(dst));
+    else reinterpret_cast<float2_u*>(dst)[0] = v;
   } else {
     if constexpr (NT) __builtin_nontemporal_store(acc[0], dst);
     else dst[0] = acc[0];
   }
 }
+
+// Which elements of a lane's window are its own, as masks of the fragment's 32-bit words: all but the
+// first `skip`, which belong to the lane before.
+template <int VEC>
+struct OwnElements {
+  uint32_t mask[VEC / 2 > 0 ? VEC / 2 : 1];
+  __device__ __forceinline__ explicit OwnElements(int skip) {
+#pragma unroll
+    for (int j = 0; j < VEC / 2; ++j)
+      mask[j] = skip <= 2 * j ? 0xffffffffu : skip == 2 * j + 1 ? 0xffff0000u : 0u;
+  }
+  // b with zeros in place of the others' elements
+  __device__ __forceinline__ void keep(BFrag<VEC>& b) const {
+    if constexpr (VEC > 1) {
+      typedef uint32_t words_t __attribute__((ext_vector_type(VEC / 2)));
+      words_t w = __builtin_bit_cast(words_t, b.v);
+      if constexpr (VEC == 2) {
+        w &= mask[0];
+      } else {
+#pragma unroll
+        for (int j = 0; j < VEC / 2; ++j) w[j] &= mask[j];
+      }
+      b.v = __builtin_bit_cast(decltype(b.v), w);
+    }
+  }
+};
+
+// First feature of the VEC-wide window that covers feature f0 < K without leaving the row: f0 itself,
+// or K - VEC where [f0, f0 + VEC) would pass the row's end (the launchers take VEC <= K).
+template <int VEC>
+__device__ __forceinline__ int row_window(int f0, int K) { return f0 < K - VEC ? f0 : K - VEC; }
 
 // Element offset of row `row` (validated non-negative) in an operand with leading dimension ld
 // (the host guarantees ld < 2^31): one 32 x 32 -> 64-bit multiply per gather.
@@ -386,6 +425,7 @@ constexpr int kNtStores = 2;
 constexpr int kStageMax = 256;
 constexpr int kStageSpan = kStageMax + 8;
 typedef int32_t int4_t __attribute__((ext_vector_type(4)));
+typedef int4_t int4_u __attribute__((aligned(2)));
 
 template <int LPG>
 __device__ __forceinline__ void stage_stream(const int32_t* __restrict__ col, const uint16_t* __restrict__ val,
@@ -504,10 +544,14 @@ __device__ __forceinline__ void spmm_tasks_run(const DevicePlan& P, int block, i
   __syncthreads();
   if (!valid) return;
 
-  const int f = blockIdx.y * (LPG * VEC) + li * VEC;
-  const bool active = f < K;
-  const uint16_t* __restrict__ Bf = B + (active ? f : 0);
-  const uint16_t* __restrict__ Hf = HOT ? P.hot_b + (active ? f : 0) : nullptr;
+  // lane li holds features [f, f + VEC); the last lane of a width that VEC does not divide holds the
+  // last VEC features instead, the same sums in the same order as its neighbour's where they overlap
+  // (both store the same values)
+  const int f0 = blockIdx.y * (LPG * VEC) + li * VEC;
+  const bool active = f0 < K;
+  const int f = active ? row_window<VEC>(f0, K) : 0;
+  const uint16_t* __restrict__ Bf = B + f;
+  const uint16_t* __restrict__ Hf = HOT ? P.hot_b + f : nullptr;
   float acc[VEC];
   zero_acc(acc);
   // one batch: column ids and values (from LDS when staged) and its B gathers
@@ -599,8 +643,9 @@ __device__ __forceinline__ void fixup_narrow(const DevicePlan& P, int block, int
   const int lane = threadIdx.x & 63;
   const int id = (block * 4 + (threadIdx.x >> 6)) * GPW + lane / LPG;
   if (id >= P.nfixups) return;
-  const int f = blockIdx.y * (LPG * VEC) + (lane % LPG) * VEC;
-  if (f >= K) return;
+  const int f0 = blockIdx.y * (LPG * VEC) + (lane % LPG) * VEC;
+  if (f0 >= K) return;
+  const int f = row_window<VEC>(f0, K);
   const Fixup x = P.fixups[id];
   float acc[VEC];
   zero_acc(acc);
@@ -633,11 +678,12 @@ __device__ __forceinline__ void fixup_wide(const DevicePlan& P, int block, int K
   __shared__ float red[G][LPG * VEC];
   const int g = threadIdx.x / LPG;
   const int li = threadIdx.x % LPG;
-  const int f = blockIdx.y * (LPG * VEC) + li * VEC;
+  const int f0 = blockIdx.y * (LPG * VEC) + li * VEC;
+  const int f = row_window<VEC>(f0, K);
   const Fixup x = P.wfixups[block];
   float acc[VEC];
   zero_acc(acc);
-  if (f < K) {
+  if (f0 < K) {
     for (int s = g; s < x.slots; s += G) {
       const float* src = partial + (int64_t)P.slot_list[x.slot_begin + s] * K + f;
 #pragma unroll
@@ -653,7 +699,7 @@ __device__ __forceinline__ void fixup_wide(const DevicePlan& P, int block, int K
       for (int i = 0; i < VEC; ++i) red[g][li * VEC + i] += red[g + h][li * VEC + i];
     __syncthreads();
   }
-  if (g == 0 && f < K) {
+  if (g == 0 && f0 < K) {
 #pragma unroll
     for (int i = 0; i < VEC; ++i) acc[i] = red[0][li * VEC + i];
     store_vec<VEC>(C + (int64_t)x.row * ldc + f, acc);
@@ -668,6 +714,34 @@ __global__ __launch_bounds__(256) void k_spmm_fixup(DevicePlan P, int K, float* 
                                                     const float* __restrict__ partial) {
   if ((int)blockIdx.x < P.nwfixups) fixup_wide<VEC, LPG>(P, blockIdx.x, K, C, ldc, partial);
   else fixup_narrow<VEC, LPG>(P, (int)blockIdx.x - P.nwfixups, K, C, ldc, partial);
+}
+
+// Features [f, f + VEC) of B row c into LDS at dst: zeros for an
+// empty column slot (c < 0) or past the row's end, which a lane at the end of a width that VEC does
+// not divide reads as the row's last VEC features, shifted back.
+template <int VEC>
+__device__ __forceinline__ void stage_fragment(const uint16_t* __restrict__ B, int64_t ldb, int c, int f, int K,
+                                               _Float16* dst) {
+  typedef _Float16 frag_t __attribute__((ext_vector_type(VEC)));
+  BFrag<VEC> b;
+  if (c >= 0 && f < K) {
+    const int w = row_window<VEC>(f, K);
+    b.load(B + row_offset(c, ldb) + w);
+    if constexpr (VEC > 1) {
+      if (w != f) {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i) dst[i] = (_Float16)0;
+#pragma unroll
+        for (int i = 0; i < VEC; ++i)
+          if (i >= f - w) dst[i - (f - w)] = b.v[i];
+        return;
+      }
+    }
+  } else {
+    b.zero();
+  }
+  if constexpr (VEC > 1) *reinterpret_cast<frag_t*>(dst) = b.v;
+  else dst[0] = b.v;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -714,13 +788,7 @@ void k_spmm_mfma_win(DevicePlan P, const uint16_t* __restrict__ B, int64_t ldb, 
       const int k = idx / per_row;
       const int ff = (idx % per_row) * VEC;
       const int c = P.tile_cols[t * 16 + k];
-      BFrag<VEC> b;
-      if (c >= 0 && fbase + ff < K) b.load(B + row_offset(c, ldb) + fbase + ff);
-      else b.zero();
-      if constexpr (VEC == 8) *reinterpret_cast<half8_t*>(bst + k * KCB + ff) = b.v;
-      else if constexpr (VEC == 4) *reinterpret_cast<half4_t*>(bst + k * KCB + ff) = b.v;
-      else if constexpr (VEC == 2) *reinterpret_cast<half2_t*>(bst + k * KCB + ff) = b.v;
-      else bst[k * KCB + ff] = b.v;
+      stage_fragment<VEC>(B, ldb, c, fbase + ff, K, bst + k * KCB + ff);
     }
     __syncthreads();
 #pragma unroll
@@ -755,13 +823,7 @@ void k_spmm_mfma_win(DevicePlan P, const uint16_t* __restrict__ B, int64_t ldb, 
           const int ff = (i2 % per_row) * VEC;
           const int c = P.quad_cols[(int64_t)q * 64 + k];
           const int f = fbase + 64 * j + ff;
-          BFrag<VEC> b;
-          if (c >= 0 && f < K) b.load(B + row_offset(c, ldb) + f);
-          else b.zero();
-          if constexpr (VEC == 8) *reinterpret_cast<half8_t*>(bst + k * QS + ff) = b.v;
-          else if constexpr (VEC == 4) *reinterpret_cast<half4_t*>(bst + k * QS + ff) = b.v;
-          else if constexpr (VEC == 2) *reinterpret_cast<half2_t*>(bst + k * QS + ff) = b.v;
-          else bst[k * QS + ff] = b.v;
+          stage_fragment<VEC>(B, ldb, c, f, K, bst + k * QS + ff);
         }
         __syncthreads();
         if (wave + 4 * j < ntn) {
@@ -792,7 +854,8 @@ void k_spmm_mfma_win(DevicePlan P, const uint16_t* __restrict__ B, int64_t ldb, 
   const int groups = 256 / gs;     // threads past groups * gs sit this phase out
   const int g = threadIdx.x / gs;
   const int ff = (threadIdx.x % gs) * VEC;
-  const int f = fbase + ff;
+  const int f0 = fbase + ff;
+  const int f = row_window<VEC>(f0, K);
   for (int rl = g; g < groups && rl < 16; rl += groups) {
     const int row = w.row0 + rl;
     if (row >= P.m) break;
@@ -801,9 +864,18 @@ void k_spmm_mfma_win(DevicePlan P, const uint16_t* __restrict__ B, int64_t ldb, 
     // pipelined batches of 4 entries (same-box A/B on SBM against 8 unpipelined / 8 pipelined /
     // 4 unpipelined: K=64 0.230 vs 0.246 / 0.257 / 0.248 ms, K=128 0.430 vs 0.462 / 0.479 /
     // 0.468, K=256 0.909 vs 0.938 / 0.922 / 1.037)
-    accumulate_row<VEC, 4, false, true>(P.col, P.val, B + (f < K ? f : 0), ldb, P.rowptr[row], P.rowptr[row + 1],
+    accumulate_row<VEC, 4, false, true>(P.col, P.val, B + f, ldb, P.rowptr[row], P.rowptr[row + 1],
                                         racc);
-    if (f >= K) continue;
+    if (f0 >= K) continue;
+    if constexpr (VEC > 1) {
+      // the row's last VEC features: those from f0 on are this thread's
+      if (f != f0) {
+#pragma unroll
+        for (int i = 0; i < VEC; ++i)
+          if (f + i >= f0) C[(int64_t)row * ldc + f + i] = racc[i] + otile[rl * KCP + f + i - fbase];
+        continue;
+      }
+    }
     const float* src = otile + rl * KCP + ff;
     if constexpr (VEC == 8) {
       const float4_t lo = reinterpret_cast<const float4_t*>(src)[0];
@@ -883,13 +955,15 @@ __device__ __forceinline__ float reduce_scatter(float (&v)[U], int li) {
 // acc: add to the outputs instead of writing them (a later feature pass of the same entries).
 // HOT: P.col is the hot-renumbered copy and negative ids gather Y rows from the staged rows
 // P.hot_b.
+// RAG: VEC does not divide K: the lane at the end of a row reads the row's last VEC features and
+// zeroes those of the lane before in both operands (in one alone, 0 x Inf would be NaN).
 // Static LDS of k_sddmm_tasks<.., LPG, .., LS>: the row-pointer slices and, when staged, the
 // column id slices (the arrays it declares; checked there).
 constexpr size_t sddmm_static_lds(int lpg, bool ls) {
   return (size_t)4 * (64 / lpg) * (kTaskRows + 1) * 4 + (ls ? (size_t)4 * (64 / lpg) * kStageSpan * 4 : 16);
 }
 
-template <int VEC, int LPG, int U, bool LS, bool SPF = false, bool NTO = false, bool HOT = false>
+template <int VEC, int LPG, int U, bool LS, bool SPF, bool NTO, bool HOT, bool RAG>
 __device__ __forceinline__ void sddmm_tasks_run(const DevicePlan& P, int block, int nblocks,
                                                 const uint16_t* __restrict__ X, int64_t ldx,
                                                 const uint16_t* __restrict__ Y, int64_t ldy, int K,
@@ -982,12 +1056,16 @@ __device__ __forceinline__ void sddmm_tasks_run(const DevicePlan& P, int block, 
     for (int i = 0; i < U; ++i) s[i] = 0.f;
     for (int f0 = 0; f0 < K; f0 += FPP) {
       const int f = f0 + li * VEC;
+      // (the last feature pass of a wide row may be narrower than VEC: its window then starts in the
+      // pass before, at w < 0; lanes past K read the first window and own nothing of it)
+      const int w = RAG ? row_window<VEC>(f < K ? f : 0, K) : f < K ? f : 0;
+      const OwnElements<VEC> own(f < K ? f - w : VEC);
       // all Y gathers first, unconditional so they issue back to back (lanes past K read features
       // [0, VEC) and padded slots repeat the last entry; both are discarded), then one X fetch per
       // distinct row of the chunk; the fragment each entry uses is selected in registers
       BFrag<VEC> x[U], y[U];
-      const uint16_t* __restrict__ Yf = Y + (f < K ? f : 0);
-      const uint16_t* __restrict__ Hf = HOT ? P.hot_b + (f < K ? f : 0) : nullptr;
+      const uint16_t* __restrict__ Yf = Y + w;
+      const uint16_t* __restrict__ Hf = HOT ? P.hot_b + w : nullptr;
 #pragma unroll
       for (int i = 0; i < U; ++i) y[i].load(gather_addr<HOT>(Yf, ldy, Hf, P.hot_ld, cc[i]));
       if constexpr (PFC) {
@@ -1002,11 +1080,18 @@ __device__ __forceinline__ void sddmm_tasks_run(const DevicePlan& P, int block, 
 #pragma unroll
       for (int i = 0; i < U; ++i) {
         if (f < K && p + i < t.nz_end && (i == 0 ? !reuse : rr[i] != rr[i - 1])) {
-          const uint16_t* xp = X + (int64_t)(P.sub_row ? P.sub_row[rr[i]] : rr[i]) * ldx + f;
-          if constexpr (VEC == 8) x[i].load_nt(xp);
+          const uint16_t* xp = X + (int64_t)(P.sub_row ? P.sub_row[rr[i]] : rr[i]) * ldx + w;
+          if constexpr (VEC == 8 && !RAG) x[i].load_nt(xp);
           else x[i].load(xp);
         } else {
           x[i].zero();
+        }
+      }
+      if constexpr (RAG) {
+#pragma unroll
+        for (int i = 0; i < U; ++i) {   // (masked where loaded, each X fetch would be waited for there)
+          own.keep(x[i]);
+          own.keep(y[i]);
         }
       }
       BFrag<VEC> xe = reuse ? xc : x[0];
@@ -1040,14 +1125,14 @@ __device__ __forceinline__ void sddmm_tasks_run(const DevicePlan& P, int block, 
 
 // Main part (Pm, the first gm workgroups, into out_m) and split part (Px, the rest, into out_x) in
 // one launch, as k_spmm_tasks (gm a multiple of kXcds where a split part follows).
-template <int VEC, int LPG, int U, bool LS, bool SPF = false, bool NTO = false, bool HOT = false>
+template <int VEC, int LPG, int U, bool LS, bool SPF, bool NTO, bool HOT, bool RAG>
 __global__ __launch_bounds__(256) void k_sddmm_tasks(DevicePlan Pm, DevicePlan Px, int gm,
                                                      const uint16_t* __restrict__ X, int64_t ldx,
                                                      const uint16_t* __restrict__ Y, int64_t ldy, int K,
                                                      float* __restrict__ out_m, float* __restrict__ out_x, int acc) {
   const int b = (int)blockIdx.x;
-  if (b < gm) sddmm_tasks_run<VEC, LPG, U, LS, SPF, NTO, HOT>(Pm, b, gm, X, ldx, Y, ldy, K, out_m, acc);
-  else sddmm_tasks_run<VEC, LPG, U, LS, SPF, NTO, HOT>(Px, b - gm, (int)gridDim.x - gm, X, ldx, Y, ldy, K, out_x, acc);
+  if (b < gm) sddmm_tasks_run<VEC, LPG, U, LS, SPF, NTO, HOT, RAG>(Pm, b, gm, X, ldx, Y, ldy, K, out_m, acc);
+  else sddmm_tasks_run<VEC, LPG, U, LS, SPF, NTO, HOT, RAG>(Px, b - gm, (int)gridDim.x - gm, X, ldx, Y, ldy, K, out_x, acc);
 }
 
 // The split rows' outputs into place (one workgroup per merge task): contiguous stores, reads from
@@ -1124,12 +1209,12 @@ __global__ __launch_bounds__(256) void k_sddmm_mfma(DevicePlan P, const uint16_t
   }
 }
 
-// SDDMM over dense tiles with gfx950's v_mfma_f32_16x16x32_f16, K % 8 == 0 and 16-byte aligned
-// rows: lane l supplies 8 consecutive features (one 16-byte load) of X row row0 + l % 16 as A and of
+// SDDMM over dense tiles with gfx950's v_mfma_f32_16x16x32_f16, K >= 8 and rows of any alignment: lane l supplies 8 consecutive features (one 16-byte load) of X row row0 + l % 16 as A and of
 // Y row col_{l % 16} as B, for the feature group 8 (l / 16) of each 32-feature step.  A and B use
 // the same lane/element -> feature assignment, so D[r][c] = X[r] . Y[c] whatever order the
 // instruction sums its 32 products in.  The loads of up to 4 steps (128 features) are issued
-// before their MFMAs.  Features past K read feature 0 and are zeroed in both operands.
+// before their MFMAs.  Features past K read feature 0 and are zeroed in both operands; the lane at the end of a
+// K that 8 does not divide reads the row's last 8 features and zeroes the others' in both.
 __global__ __launch_bounds__(256) void k_sddmm_mfma32(DevicePlan P, const uint16_t* __restrict__ X, int64_t ldx,
                                                       const uint16_t* __restrict__ Y, int64_t ldy, int K,
                                                       float* __restrict__ out) {
@@ -1149,15 +1234,22 @@ __global__ __launch_bounds__(256) void k_sddmm_mfma32(DevicePlan P, const uint16
 #pragma unroll
     for (int i = 0; i < SPC; ++i) {
       const int k = k0 + 32 * i + fq;
-      const int kk = k < K ? k : 0;
-      a[i] = *reinterpret_cast<const half8_t*>(xp + kk);
-      b[i] = *reinterpret_cast<const half8_t*>(yp + kk);
+      const int kk = k < K ? row_window<8>(k, K) : 0;
+      a[i] = *reinterpret_cast<const half8_u*>(xp + kk);
+      b[i] = *reinterpret_cast<const half8_u*>(yp + kk);
     }
 #pragma unroll
     for (int i = 0; i < SPC; ++i) {
-      const bool in = k0 + 32 * i + fq < K;
-      const half8_t z{0, 0, 0, 0, 0, 0, 0, 0};
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(in ? a[i] : z, in ? b[i] : z, acc, 0, 0, 0);
+      // features of this step that are this lane's: none past the row's end, and the last ones of
+      // the row's last window
+      const int k = k0 + 32 * i + fq;
+      const int skip = k < K ? k - row_window<8>(k, K) : 8;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        a[i][j] = j < skip ? (_Float16)0 : a[i][j];
+        b[i][j] = j < skip ? (_Float16)0 : b[i][j];
+      }
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[i], acc, 0, 0, 0);
     }
   }
   const int32_t* pos = P.tile_pos + (int64_t)t * 256;
@@ -1204,29 +1296,31 @@ void launch_tasks(dim3 grid, int gm, int waves, hipStream_t s, const DevicePlan&
                      occupancy_pad(tasks_static_lds(LPG, LS), waves), s, p, x, gm, B, ldb, K, C, ldc, partial);
 }
 
-// Staged hot rows: dst[r][0, K) = B[rows[r]][0, K) for r < nhot, 16 bytes per thread (K % 8 == 0,
-// 16-byte aligned rows).
+// Staged hot rows: dst[r][0, K) = B[rows[r]][0, K) for r < nhot (row stride hld), 16 bytes per
+// thread (K >= 8; the last chunk of a row is its last 8 features).
 __global__ __launch_bounds__(256) void k_stage_hot_rows(const uint16_t* __restrict__ B, int64_t ldb, int K,
                                                         const int32_t* __restrict__ rows, int32_t nhot,
-                                                        uint16_t* __restrict__ dst) {
-  const int chunks = K >> 3;
+                                                        uint16_t* __restrict__ dst, int hld) {
+  const int chunks = (K + 7) >> 3;
   const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (t >= (int64_t)nhot * chunks) return;
   const int r = (int)(t / chunks), c = (int)(t - (int64_t)r * chunks);
-  const int4_t v = *reinterpret_cast<const int4_t*>(B + row_offset(rows[r], ldb) + c * 8);
-  *reinterpret_cast<int4_t*>(dst + (int64_t)r * K + c * 8) = v;
+  const int f = row_window<8>(c * 8, K);
+  const int4_t v = *reinterpret_cast<const int4_u*>(B + row_offset(rows[r], ldb) + f);
+  *reinterpret_cast<int4_u*>(dst + (int64_t)r * hld + f) = v;
 }
 
 // Copies the plan's hot rows of B (K features) into hot and returns the view whose task kernels
 // read the renumbered columns and the staged rows.
 DevicePlan hot_view(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, uint16_t* hot, hipStream_t s) {
-  const int64_t threads = (int64_t)p.nhot * (K >> 3);
+  const int64_t threads = (int64_t)p.nhot * ((K + 7) >> 3);
+  const int hld = hot_row_stride(K);
   hipLaunchKernelGGL(k_stage_hot_rows, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, B, ldb, K,
-                     p.hot_rows, p.nhot, hot);
+                     p.hot_rows, p.nhot, hot, hld);
   DevicePlan v = p;
   v.col = p.hot_col;
   v.hot_b = hot;
-  v.hot_ld = K;
+  v.hot_ld = hld;
   return v;
 }
 
@@ -1237,19 +1331,6 @@ int lanes_for(int K, int vec) {
   return l;
 }
 
-// Narrow loads of a width just past a power of two leave most lanes of a wide group idle: the
-// group width (>= 16 lanes) with the fewest lane slots over all feature passes (ties to fewer
-// passes), taken when it saves at least a fifth of the slots of `lpg` lanes.
-int fewer_lane_slots(int K, int vec, int lpg) {
-  const int slots0 = (K + lpg * vec - 1) / (lpg * vec) * lpg;
-  int best = lpg, best_slots = slots0;
-  for (int l = lpg / 2; l >= 16; l >>= 1) {
-    const int slots = (K + l * vec - 1) / (l * vec) * l;
-    if (slots < best_slots) best = l, best_slots = slots;
-  }
-  return best_slots * 5 <= slots0 * 4 ? best : lpg;
-}
-
 template <int VEC>
 hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
                            float* partial, uint16_t* hot, hipStream_t s, hipEvent_t* ev) {
@@ -1258,10 +1339,6 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
   // a plan may ask for fewer lanes per group: several feature passes, each gathering a narrower
   // slice of B (smaller working set per pass)
   while (p.feature_lanes > 0 && lpg > p.feature_lanes && lpg > 1) lpg >>= 1;
-  // (same-box A/B on R-MAT: K=66 2.25 ms in one pass of 64 lanes -> 1.93 in three of 16, K=130
-  // 4.59 -> 3.21, K=65 3.14 -> 2.42, K=81 3.20 -> 2.78, K=33 1.47 -> 1.35; grid+hubs K=66 1.99 ->
-  // 2.07, K=33 1.41 -> 1.46.  K=97, an eighth fewer slots in seven passes: 3.25 -> 3.33)
-  if (p.feature_lanes <= 0 && VEC <= 2) lpg = fewer_lane_slots(K, VEC, lpg);
   // passes of at most 128 features for 16-byte loads: each pass gathers 256-byte slices of B
   // rows, twice as many of which fit an XCD's L2 as whole 512-byte rows (R-MAT 2^20, K = 256:
   // 1.730 ms in one pass of 32 lanes, 1.522 in two of 16, 1.837 in four of 8; K = 128 in two
@@ -1275,7 +1352,7 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
   const int passes = (K + fpp - 1) / fpp;
   // staged hot rows for the staged-stream kernel of 16-lane groups (256-byte gathers); the window
   // kernel keeps reading B through the plain column ids
-  const bool hot_on = VEC == 8 && lpg == 16 && hot != nullptr && hot_buffer_bytes(p, K) > 0 &&
+  const bool hot_on = VEC == 8 && lpg == 16 && hot != nullptr && hot_buffer_bytes(p, K, false) > 0 &&
                       p.task_max <= kStageMax && p.stage >= 0 &&
                       (p.x_ntasks == 0 || p.x_task_max <= kStageMax);
   const DevicePlan tp = hot_on ? hot_view(p, B, ldb, K, hot, s) : p;
@@ -1344,7 +1421,14 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     }                                                                                                     \
     break;                                                                                                \
   }
-    switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) TRS_TASKS(16) TRS_TASKS(32) TRS_TASKS(64) }
+    // 4- and 2-byte loads serve K <= 8 in groups of 4 lanes, 8-byte ones K <= 64 in 4 or 16 lanes
+    if constexpr (VEC < 4) {
+      switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) }
+    } else if constexpr (VEC < 8) {
+      switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) TRS_TASKS(16) }
+    } else {
+      switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) TRS_TASKS(16) TRS_TASKS(32) TRS_TASKS(64) }
+    }
 #undef TRS_TASKS
 #undef TRS_TASKS_NT
   };
@@ -1377,7 +1461,13 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     const int gpb = 4 * (64 / lpg);
     dim3 grid(p.nwfixups + (p.nfixups + gpb - 1) / gpb, passes);
 #define TRS_FIX(L) case L: hipLaunchKernelGGL((k_spmm_fixup<VEC, L>), grid, dim3(256), 0, s, p, K, C, ldc, partial); break;
-    switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) TRS_FIX(16) TRS_FIX(32) TRS_FIX(64) }
+    if constexpr (VEC < 4) {
+      switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) }
+    } else if constexpr (VEC < 8) {
+      switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) TRS_FIX(16) }
+    } else {
+      switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) TRS_FIX(16) TRS_FIX(32) TRS_FIX(64) }
+    }
 #undef TRS_FIX
   }
   if (ev) (void)hipEventRecord(ev[3], s);
@@ -1389,7 +1479,7 @@ hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx,
                             int K, float* out, uint16_t* hot, float* xbuf, hipStream_t s, hipEvent_t* ev) {
   if (ev) (void)hipEventRecord(ev[0], s);
   // staged hot Y rows (all K features, once per call) for the passes run by 16-lane groups
-  const bool hot_on = VEC == 8 && hot != nullptr && hot_buffer_bytes(p, K) > 0;
+  const bool hot_on = VEC == 8 && hot != nullptr && hot_buffer_bytes(p, K, true) > 0;
   const DevicePlan hp = hot_on ? hot_view(p, Y, ldy, K, hot, s) : p;
   // the split part writes its own buffer (then merged) where the workspace holds one
   bool merge_on = p.x_ntasks > 0 && xbuf != nullptr && merge_buffer_bytes(p, K) > 0;
@@ -1405,12 +1495,8 @@ hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx,
     const int acc = f0 > 0 ? 1 : 0;
     DevicePlan pp = p;
     int lpg = lanes_for(Kp, VEC);
-    // fewer lanes than features: the kernel loops over feature chunks per batch (no second walk
-    // of the entries), so narrow loads take the group width with the fewest lane slots (same-box
-    // A/B on R-MAT: K=66 1.49 ms with 64 lanes -> 0.91 with 16, K=82 1.50 -> 0.99, K=130 2.00 ->
-    // 1.72, K=33 1.40 -> 0.73, K=65 1.87 -> 1.20)
+    // a plan may ask for fewer lanes: the kernel then loops over feature chunks per batch
     while (p.feature_lanes > 0 && lpg > p.feature_lanes && lpg > 1) lpg >>= 1;
-    if (p.feature_lanes <= 0 && VEC <= 2) lpg = fewer_lane_slots(Kp, VEC, lpg);
     // at least 8 lanes, so that a group writes 8 consecutive sums (32 bytes) per store and the
     // outputs stream; lanes past K add zeros (R-MAT K=4 0.329 -> 0.258 ms, K=2 0.327 -> 0.259,
     // K=1 0.467 -> 0.260)
@@ -1435,33 +1521,34 @@ hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx,
     // 16-byte runs, as 4-lane groups write at K=16, lose: 0.418 -> 0.469)
     const bool ls = p.task_max <= kStageMax && p.stage >= 0 && (x.ntasks <= 0 || x.task_max <= kStageMax);
     const bool nto = (p.streaming & 2) != 0;
+    const bool rag = VEC > 1 && Kp % VEC != 0;
     // occupancy: uncapped unless the plan asks (option occupancy: waves per SIMD, held by unused
     // dynamic LDS)
     const int waves = p.occupancy > 0 ? p.occupancy : 0;
-#define TRS_SD_LAUNCH(VV, LL, UU, LSV, ...)                                                               \
-  hipLaunchKernelGGL((k_sddmm_tasks<VV, LL, UU, LSV, ##__VA_ARGS__>), grid, dim3(256),                    \
+#define TRS_SD_LAUNCH(LL, UU, LSV, SPFV, NTOV, HOTV, RAGV)                                                \
+  hipLaunchKernelGGL((k_sddmm_tasks<VEC, LL, UU, LSV, SPFV, NTOV, HOTV, RAGV>), grid, dim3(256),          \
                      occupancy_pad(sddmm_static_lds(LL, LSV), waves), s, p, x, gm, Xp, ldx, Yp, ldy, Kp, out, xout, acc)
-#define TRS_SD_U(L, U)                                                                                     \
-    constexpr bool nt_ok = (U < L ? U : L) >= 8;                                                           \
-    if constexpr (L == 16) {                                                                               \
-      if (VEC == 8 && p.hot_b != nullptr) {                                                                \
-        if (ls) {                                                                                          \
-          if (nt_ok && nto) TRS_SD_LAUNCH(VEC, L, U, true, false, nt_ok, VEC == 8);                        \
-          else TRS_SD_LAUNCH(VEC, L, U, true, false, false, VEC == 8);                                     \
-        } else {                                                                                           \
-          if (nt_ok && nto) TRS_SD_LAUNCH(VEC, L, U, false, false, nt_ok, VEC == 8);                       \
-          else TRS_SD_LAUNCH(VEC, L, U, false, false, false, VEC == 8);                                    \
-        }                                                                                                  \
-        break;                                                                                             \
-      }                                                                                                    \
-      if (ls) {                                                                                            \
-        if (nt_ok && nto) TRS_SD_LAUNCH(VEC, L, U, true, false, nt_ok);                                    \
-        else TRS_SD_LAUNCH(VEC, L, U, true);                                                               \
-        break;                                                                                             \
-      }                                                                                                    \
-    }                                                                                                      \
-    if (nt_ok && nto) TRS_SD_LAUNCH(VEC, L, U, false, (L <= 8), nt_ok);                                    \
-    else TRS_SD_LAUNCH(VEC, L, U, false, (L <= 8));
+#define TRS_SD_NTO(L, U, LSV, SPFV, HOTV, RAGV)                                                           \
+    if (nt_ok && nto) TRS_SD_LAUNCH(L, U, LSV, SPFV, nt_ok, HOTV, RAGV);                                  \
+    else TRS_SD_LAUNCH(L, U, LSV, SPFV, false, HOTV, RAGV);
+#define TRS_SD_U(L, U)                                                                                    \
+    constexpr bool nt_ok = (U < L ? U : L) >= 8;                                                          \
+    if constexpr (L == 16) {                                                                              \
+      if (VEC == 8 && p.hot_b != nullptr) {                                                               \
+        if (ls && rag) { TRS_SD_NTO(L, U, true, false, (VEC == 8), (VEC == 8)) }                          \
+        else if (ls) { TRS_SD_NTO(L, U, true, false, (VEC == 8), false) }                                 \
+        else if (rag) { TRS_SD_NTO(L, U, false, false, (VEC == 8), (VEC == 8)) }                          \
+        else { TRS_SD_NTO(L, U, false, false, (VEC == 8), false) }                                        \
+        break;                                                                                            \
+      }                                                                                                   \
+      if (ls) {                                                                                           \
+        if (rag) { TRS_SD_NTO(L, U, true, false, false, (VEC > 1)) }                                        \
+        else { TRS_SD_NTO(L, U, true, false, false, false) }                                              \
+        break;                                                                                            \
+      }                                                                                                   \
+    }                                                                                                     \
+    if (rag) { TRS_SD_NTO(L, U, false, (L <= 8), false, (VEC > 1)) }                                        \
+    else { TRS_SD_NTO(L, U, false, (L <= 8), false, false) }
     // entries in flight per lane group: 4 where a 16-lane group's 16-byte loads cover 128 features,
     // 8 elsewhere (same-box A/B on the R-MAT 2^20 pattern, 8 -> 4: K = 128 0.726 -> 0.705 ms, K = 256
     // (two passes of 128) 1.544 -> 1.482; K = 96 0.689 -> 0.720, K = 32 0.380 -> 0.488)
@@ -1474,9 +1561,17 @@ hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx,
       TRS_SD_U(L, 8)                                                                                       \
     }                                                                                                      \
     break;
-    switch (lpg) { TRS_SD(1) TRS_SD(2) TRS_SD(4) TRS_SD(8) TRS_SD(16) TRS_SD(32) TRS_SD(64) }
+    // loads narrower than 16 bytes serve K <= 64, at most 16 lanes of 8 bytes, 8 of 4 or 2 bytes
+    if constexpr (VEC < 4) {
+      switch (lpg) { TRS_SD(1) TRS_SD(2) TRS_SD(4) TRS_SD(8) }
+    } else if constexpr (VEC < 8) {
+      switch (lpg) { TRS_SD(1) TRS_SD(2) TRS_SD(4) TRS_SD(8) TRS_SD(16) }
+    } else {
+      switch (lpg) { TRS_SD(1) TRS_SD(2) TRS_SD(4) TRS_SD(8) TRS_SD(16) TRS_SD(32) TRS_SD(64) }
+    }
 #undef TRS_SD
 #undef TRS_SD_U
+#undef TRS_SD_NTO
 #undef TRS_SD_LAUNCH
     };
     DevicePlan none = pp;
@@ -1528,7 +1623,7 @@ hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx,
   if (p.ntiles > 0 && p.tile_pos) {
     const bool v4 = K % 4 == 0 && ldx % 4 == 0 && ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 7) == 0 &&
                     (reinterpret_cast<uintptr_t>(Y) & 7) == 0;
-    const bool v8 = K % 8 == 0 && ldx % 8 == 0 && ldy % 8 == 0 && aligned16(X) && aligned16(Y);
+    const bool v8 = K >= 8;
     dim3 grid((p.ntiles + 3) / 4);
     // 16x16x32 with 16-byte loads issued ahead (same-box A/B on SBM 1M: K=128 0.174 -> 0.116 ms,
     // K=256 0.314 -> 0.205 ms; K=32 unchanged)
@@ -1902,27 +1997,25 @@ hipError_t launch_spmm(const DevicePlan& p, const uint16_t* B, int64_t ldb, int 
   // loads, 0.273 with four lanes of 4-byte loads (below); K=4 0.515 -> 0.220), and K=16 runs best
   // as 4 lanes of 8-byte loads (R-MAT 0.436 ms with 2 lanes of 16-byte loads, 0.324; grid+hubs
   // 0.368 -> 0.307)
-  const bool v8 = K > 16 && K % 8 == 0 && ldb % 8 == 0 && ldc % 4 == 0 && aligned16(B) && aligned16(C) &&
-                  (partial == nullptr || aligned16(partial));
-  // 8-byte loads when rows are only 8-byte aligned (K % 4 == 0): R-MAT K=100 3.22 ms with 2-byte
-  // loads
-  const bool v4 = K > 8 && K % 4 == 0 && ldb % 4 == 0 && ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(B) & 7) == 0 &&
-                  aligned16(C) && (partial == nullptr || aligned16(partial));
-  // 4-byte loads for even widths that 8-byte loads cannot serve (same-box A/B against 2-byte
-  // loads, R-MAT: K=10 0.438 -> 0.346 ms, K=18 0.776 -> 0.612, K=30 0.828 -> 0.641, K=98 3.245 ->
-  // 2.313; SBM K=18 0.295 -> 0.208).  K=12 and 16 stay on 8-byte loads in 4-lane groups (R-MAT
-  // K=16 0.318 vs 0.333 ms with 4-byte loads in 8-lane groups)
-  // K = 6 and 8 too, in groups of 4 lanes (R-MAT K=6 0.297 -> 0.253 ms, K=8 0.283 -> 0.273; SBM,
-  // whose window kernel stages B rows with the same loads, K=6 0.189 -> 0.144, K=8 0.180 ->
-  // 0.145; grid+hubs K=8 0.241 -> 0.245).  K=4 stays on 2-byte loads (R-MAT 0.219 vs 0.233)
-  const bool v2 = (K > 8 || K == 6 || K == 8) && !(v8 || v4) && K % 2 == 0 && ldb % 2 == 0 && ldc % 2 == 0 &&
-                  (reinterpret_cast<uintptr_t>(B) & 3) == 0 && (reinterpret_cast<uintptr_t>(C) & 7) == 0 &&
-                  (partial == nullptr || aligned16(partial));
+  // Load width by K alone: a row of any alignment is read with whole vectors (see half8_u), the last
+  // lane taking the row's last VEC features.  16-byte loads from K = 17 on, where 3 lanes of a group
+  // have work (K = 16 is faster as 4 lanes of 8 bytes: R-MAT 2^20 0.436 -> 0.324 ms, and K = 8 as 4
+  // lanes of 4 bytes: 0.545 -> 0.273; K = 4 as 4 lanes of 2 bytes: 0.233 -> 0.219).  With narrower
+  // loads for the widths that 8, 4 or 2 do not divide, and 2-byte ones for odd ones, R-MAT 2^20 took
+  // (us, narrow -> this): K = 5 310 -> 244, 7 336 -> 262, 13 348 -> 289, 17 580 -> 379, 18 385 ->
+  // 312, 28 460 -> 371, 31 643 -> 458, 65 1755 -> 643, 97 2198 -> 724, 100 942 -> 644, 127 2425 -> 814,
+  // 130 2122 -> 1333, 255 4436 -> 1618; SBM 250K nodes K = 17 76 -> 43, 65 169 -> 95, 127 240 -> 132.
+  // K = 33..64 off the 16-byte grid keep 8-byte loads in 16-lane groups, whose staged stream holds
+  // more entries in flight than 8-lane groups held to 2 waves: K = 33 595 (16-byte) / 454, 41 622 /
+  // 464, 52 568 / 442, 63 696 / 518 (2-byte loads before: 992, 1013, 440 with 8 bytes, 1130); grid of
+  // 4M nodes with hubs K = 41 760 / 700; on the grid 16-byte loads stay (K = 64 457 us).
+  const bool rows16 = K % 8 == 0 && ldb % 8 == 0 && aligned16(B);
+  const bool v8 = K > 16 && (K <= 32 || K > 64 || rows16), v4 = K > 8, v2 = K > 4;
   // (the staged hot rows need 16-byte aligned rows in the buffer too)
   if (hot != nullptr && !aligned16(hot)) hot = nullptr;
-  if (v2) return spmm_width<2>(p, B, ldb, K, C, ldc, partial, nullptr, stream, ev);
   return v8 ? spmm_width<8>(p, B, ldb, K, C, ldc, partial, hot, stream, ev)
        : v4 ? spmm_width<4>(p, B, ldb, K, C, ldc, partial, nullptr, stream, ev)
+       : v2 ? spmm_width<2>(p, B, ldb, K, C, ldc, partial, nullptr, stream, ev)
             : spmm_width<1>(p, B, ldb, K, C, ldc, partial, nullptr, stream, ev);
 }
 
@@ -1932,18 +2025,18 @@ hipError_t launch_sddmm(const DevicePlan& p, const uint16_t* X, int64_t ldx, con
   // 16-byte loads per task, 0.331), and up to K=64 8-byte loads are faster than 16-byte ones
   // (same-box A/B on R-MAT: K=32 0.468 -> 0.430 ms, K=64 0.550 -> 0.503; K=128 1.038 vs 1.080
   // with 8-byte loads, so 16-byte loads from K=72 on)
-  const bool v8 = K > 64 && K % 8 == 0 && ldx % 8 == 0 && ldy % 8 == 0 && aligned16(X) && aligned16(Y);
-  const bool v4 = K > 8 && K % 4 == 0 && ldx % 4 == 0 && ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 7) == 0 &&
-                  (reinterpret_cast<uintptr_t>(Y) & 7) == 0;
-  // 4-byte loads for K = 9..16 (8-lane groups, whose outputs go out in 32-byte runs; R-MAT K=16
-  // 0.418 -> 0.334 ms, K=12 0.408 -> 0.287) and for other even widths that 8-byte loads cannot
-  // serve (K=18 0.743 -> 0.431 ms, K=66 1.866 -> 1.479, K=130 2.350 -> 1.993 with 2-byte loads)
-  const bool v2 = K > 8 && (K <= 16 || !(v8 || v4)) && K % 2 == 0 && ldx % 2 == 0 && ldy % 2 == 0 &&
-                  (reinterpret_cast<uintptr_t>(X) & 3) == 0 && (reinterpret_cast<uintptr_t>(Y) & 3) == 0;
+  // Load width by K alone, as in launch_spmm: 8 lanes of 2 bytes to K = 8 and of 4 bytes to K = 16
+  // (outputs in 32-byte runs; R-MAT 2^20 K = 16 0.418 -> 0.334 ms, K = 12 0.408 -> 0.287), 8-byte loads
+  // to K = 64 (K = 32 0.468 -> 0.430 against 16-byte loads, K = 64 0.550 -> 0.503; K = 33 598 / 605 us, 52
+  // 477 / 582), 16-byte loads above.  With narrower loads for the widths that the vector does not
+  // divide the pattern took (us, narrow -> this): K = 9 393 -> 293, 13 396 -> 303, 17 706 -> 356, 31 712 ->
+  // 404, 33 702 -> 508, 63 1447 -> 567, 65 1173 -> 724, 97 2003 -> 779, 98 1508 -> 753, 100 905 -> 753,
+  // 127 2058 -> 944, 130 1657 -> 1484, 255 3692 -> 1809.
+  const bool v8 = K > 64, v4 = K > 16, v2 = K > 8;
   if (hot != nullptr && !aligned16(hot)) hot = nullptr;
-  if (v2) return sddmm_width<2>(p, X, ldx, Y, ldy, K, out, nullptr, xbuf, stream, ev);
   return v8 ? sddmm_width<8>(p, X, ldx, Y, ldy, K, out, hot, xbuf, stream, ev)
        : v4 ? sddmm_width<4>(p, X, ldx, Y, ldy, K, out, nullptr, xbuf, stream, ev)
+       : v2 ? sddmm_width<2>(p, X, ldx, Y, ldy, K, out, nullptr, xbuf, stream, ev)
             : sddmm_width<1>(p, X, ldx, Y, ldy, K, out, nullptr, xbuf, stream, ev);
 }
 #endif  // TRS_KERNEL_PART == 0

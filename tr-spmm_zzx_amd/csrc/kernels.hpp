@@ -128,10 +128,23 @@ constexpr int kSddmmMergeMinK = 128;
 inline int64_t merge_buffer_bytes(const DevicePlan& p, int K) {
   return p.nmerge > 0 && K >= kSddmmMergeMinK ? p.x_entries * 4 : 0;
 }
+// Widths that 8 does not divide stage their hot rows padded to whole cache lines, so that most gathers
+// are aligned again.  A staged row pays where an unaligned one is dear: odd widths (rows off the
+// 4-byte grid) from the first 16-lane width on, even ones where a row spans three lines, and the
+// SDDMM, which waits on its reductions besides, only near 256 bytes.  R-MAT 2^20, unstaged -> staged:
+// SpMM K = 65 684 -> 643 us, 81 859 -> 805, 127 1156 -> 817, 100 661 -> 644, 110 734 -> 684 (2^18
+// nodes: 65 187 -> 175, 127 224 -> 192, 100 151 -> 157: the copy's own 5 us); SDDMM K = 101 802 ->
+// 815, 107 839 -> 828, 121 900 -> 856, 127 1544 -> 945 (2^18: 101 190 -> 201, 121 196 -> 203, 127
+// 259 -> 206).
+inline bool stages_hot_rows(int K, bool sddmm) {
+  if (K % 8 == 0) return K >= kHotMinK;
+  return K >= (sddmm ? 121 : K % 2 != 0 ? 65 : 104);
+}
+inline int hot_row_stride(int K) { return K % 8 == 0 ? K : (K + 63) / 64 * 64; }
 // Bytes of the staged-row buffer of plan p at width K (0 when the plan or K does not stage).
-inline int64_t hot_buffer_bytes(const DevicePlan& p, int K) {
-  if (p.nhot <= 0 || K < kHotMinK || K % 8 != 0) return 0;
-  return (int64_t)p.nhot * K * 2;
+inline int64_t hot_buffer_bytes(const DevicePlan& p, int K, bool sddmm) {
+  if (p.nhot <= 0 || !stages_hot_rows(K, sddmm)) return 0;
+  return (int64_t)p.nhot * hot_row_stride(K) * 2;
 }
 // Column histogram of col[0, total) into counts[n] (ids outside [0, n) are skipped), counted in
 // `copies` histograms counts[k * n .. (k + 1) * n) (all zeroed by the caller) and summed into the

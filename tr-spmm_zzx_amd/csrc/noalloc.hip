@@ -22,6 +22,7 @@
 
 namespace trs {
 void set_error(const std::string& msg);
+int64_t spmm_least_workspace(const trs_plan* p, int32_t K);
 }
 
 namespace {
@@ -66,18 +67,19 @@ extern "C" int trs_spmm_f16_noalloc(const trs_plan* p, const uint16_t* B, int64_
                                     int64_t ldc, void* stream) {
   if (!p) return fail(TRS_EINVAL, "NULL plan");
   if (K < 0) return fail(TRS_EINVAL, "K must be non-negative");
-  const int64_t need = trs_spmm_workspace_bytes(p, K);
+  const int64_t need = trs::spmm_least_workspace(p, K);
   if (need > kScratchBytes)
     return fail(TRS_EINVAL, "trs_spmm_f16_noalloc: the plan's workspace needs " + std::to_string(need) +
                                 " bytes at K = " + std::to_string(K) + ", more than the " +
                                 std::to_string(kScratchBytes) +
                                 "-byte scratch array holds; call trs_spmm_f16 with a workspace instead");
   void* ws = nullptr;
-  if (need > 0) {
+  const bool use = trs_spmm_workspace_bytes(p, K) > 0;
+  if (use) {
     const int rc = scratch_address(&ws);
     if (rc) return rc;
   }
   // trs_spmm_f16 checks the plan's device against the current one (whose scratch address this is)
   // before it launches anything
-  return trs_spmm_f16(p, B, ldb, K, C, ldc, ws, need, stream);
+  return trs_spmm_f16(p, B, ldb, K, C, ldc, ws, use ? kScratchBytes : 0, stream);
 }

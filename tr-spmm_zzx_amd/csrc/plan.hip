@@ -34,6 +34,7 @@ thread_local std::string g_error;
 
 namespace trs {
 void set_error(const std::string& msg) { g_error = msg; }
+int64_t spmm_least_workspace(const trs_plan* p, int32_t K);
 }  // namespace trs
 
 struct trs_plan {
@@ -2375,20 +2376,24 @@ static int64_t partial_region_bytes(const trs_plan* p, int32_t K) {
 
 int64_t trs_spmm_workspace_bytes(const trs_plan* p, int32_t K) {
   if (!p || K <= 0 || p->csr_only) return 0;
-  const int64_t hot = trs::hot_buffer_bytes(p->dp, K);
+  const int64_t hot = trs::hot_buffer_bytes(p->dp, K, false);
   const int64_t partial = partial_region_bytes(p, K);
   return hot > 0 ? ((partial + 255) & ~int64_t(255)) + hot : partial;
 }
 
+// The staged rows of a width that 8 does not divide are left out where the workspace has no room
+// for them.
+static bool staging_is_optional(int32_t K) { return K % 8 != 0; }
+
 // SDDMM workspace: the split part's output buffer, then (256-byte aligned) the staged hot rows.
 static int64_t merge_region_bytes(const trs_plan* p, int32_t K) {
   const int64_t b = trs::merge_buffer_bytes(p->dp, K);
-  return trs::hot_buffer_bytes(p->dp, K) > 0 ? (b + 255) & ~int64_t(255) : b;
+  return trs::hot_buffer_bytes(p->dp, K, true) > 0 ? (b + 255) & ~int64_t(255) : b;
 }
 
 int64_t trs_sddmm_workspace_bytes(const trs_plan* p, int32_t K) {
   if (!p || K <= 0 || !p->csr_only) return 0;
-  return merge_region_bytes(p, K) + trs::hot_buffer_bytes(p->dp, K);
+  return merge_region_bytes(p, K) + trs::hot_buffer_bytes(p->dp, K, true);
 }
 
 static int check_call(const trs_plan* p, int32_t K) {
@@ -2409,11 +2414,11 @@ static int spmm_impl(const trs_plan* p, const uint16_t* B, int64_t ldb, int32_t 
   if (!C || (p->dp.n > 0 && !B) || ldb < K || ldc < K)
     return report(fail(TRS_EINVAL, "trs_spmm_f16: NULL operand or leading dimension < K"));
   if (ldb > INT32_MAX) return report(fail(TRS_ERANGE, "trs_spmm_f16: leading dimension of B beyond 2^31 - 1"));
-  const int64_t need = trs_spmm_workspace_bytes(p, K);
+  const int64_t need = trs::spmm_least_workspace(p, K);
   if (ws_bytes < need || (need > 0 && !ws))
     return report(fail(TRS_EINVAL, "trs_spmm_f16: workspace smaller than trs_spmm_workspace_bytes"));
   const int64_t partial = partial_region_bytes(p, K);
-  uint16_t* hot = trs::hot_buffer_bytes(p->dp, K) > 0
+  uint16_t* hot = ws && trs::hot_buffer_bytes(p->dp, K, false) > 0 && ws_bytes >= trs_spmm_workspace_bytes(p, K)
                       ? reinterpret_cast<uint16_t*>(static_cast<unsigned char*>(ws) + ((partial + 255) & ~int64_t(255)))
                       : nullptr;
   const hipError_t e = trs::launch_spmm(p->dp, B, ldb, K, C, ldc, static_cast<float*>(ws), hot,
@@ -2492,11 +2497,12 @@ static int sddmm_impl(const trs_plan* p, const uint16_t* X, int64_t ldx, const u
   if (!X || !Y || ldx < K || ldy < K)
     return report(fail(TRS_EINVAL, "trs_sddmm_f16: NULL operand or leading dimension < K"));
   if (ldy > INT32_MAX) return report(fail(TRS_ERANGE, "trs_sddmm_f16: leading dimension of Y beyond 2^31 - 1"));
-  const int64_t need = trs_sddmm_workspace_bytes(p, K);
+  const int64_t full = trs_sddmm_workspace_bytes(p, K);
+  const int64_t need = staging_is_optional(K) ? trs::merge_buffer_bytes(p->dp, K) : full;
   if (ws && ws_bytes < need)
     return report(fail(TRS_EINVAL, "trs_sddmm_f16_ws: workspace smaller than trs_sddmm_workspace_bytes"));
   float* xbuf = ws && trs::merge_buffer_bytes(p->dp, K) > 0 ? static_cast<float*>(ws) : nullptr;
-  uint16_t* hot = ws && trs::hot_buffer_bytes(p->dp, K) > 0
+  uint16_t* hot = ws && trs::hot_buffer_bytes(p->dp, K, true) > 0 && ws_bytes >= full
                       ? reinterpret_cast<uint16_t*>(static_cast<unsigned char*>(ws) + merge_region_bytes(p, K))
                       : nullptr;
   const hipError_t e =
@@ -2539,3 +2545,9 @@ int trs_sddmm_f16_kernel_ms(const trs_plan* p, const uint16_t* X, int64_t ldx, c
 }
 
 }  // extern "C"
+
+// The workspace that trs_spmm_f16 asks for at least.
+int64_t trs::spmm_least_workspace(const trs_plan* p, int32_t K) {
+  if (!p || K <= 0 || p->csr_only || !staging_is_optional(K)) return trs_spmm_workspace_bytes(p, K);
+  return partial_region_bytes(p, K);
+}
