@@ -1576,7 +1576,7 @@ hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx,
     };
     DevicePlan none = pp;
     none.ntasks = 0;
-    if (lpg <= 8 && p.nnarrow_tasks > 0) {
+    if (lpg <= 8 && p.nnarrow_tasks > 0 && K <= fpass) {   // (a later pass adds to where the first wrote)
       // lane groups of <= 8 lanes: the unsplit layout of every row in pieces of S entries, every
       // output written in place (no split part, nothing to merge)
       DevicePlan v = pp;
