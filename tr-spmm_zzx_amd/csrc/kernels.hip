@@ -719,15 +719,17 @@ __global__ __launch_bounds__(256) void k_spmm_fixup(DevicePlan P, int K, float* 
 // Features [f, f + VEC) of B row c into LDS at dst: zeros for an
 // empty column slot (c < 0) or past the row's end, which a lane at the end of a width that VEC does
 // not divide reads as the row's last VEC features, shifted back.
-template <int VEC>
+// RAG: VEC does not divide K (a kernel of its own: with these branches in it the window kernel takes
+// 8% longer at aligned widths, SBM of 250K nodes K = 128 98 -> 106 us).
+template <int VEC, bool RAG>
 __device__ __forceinline__ void stage_fragment(const uint16_t* __restrict__ B, int64_t ldb, int c, int f, int K,
                                                _Float16* dst) {
   typedef _Float16 frag_t __attribute__((ext_vector_type(VEC)));
   BFrag<VEC> b;
   if (c >= 0 && f < K) {
-    const int w = row_window<VEC>(f, K);
+    const int w = RAG ? row_window<VEC>(f, K) : f;
     b.load(B + row_offset(c, ldb) + w);
-    if constexpr (VEC > 1) {
+    if constexpr (RAG) {
       if (w != f) {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) dst[i] = (_Float16)0;
@@ -753,7 +755,7 @@ __device__ __forceinline__ void stage_fragment(const uint16_t* __restrict__ B, i
 // Here A = the 16x16 tile (window row x tile column), B = gathered B rows (tile column x feature).
 // Occupancy floor: the register budget of 6 waves per SIMD (the compiler settles at 5 otherwise;
 // measured: 5 waves cost 6% on SBM K=128 and 4% at K=256, 0.963 vs 0.924 ms).
-template <int VEC, int NTILE>
+template <int VEC, int NTILE, bool RAG>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(6)))
 void k_spmm_mfma_win(DevicePlan P, const uint16_t* __restrict__ B, int64_t ldb, int K, float* __restrict__ C,
                      int64_t ldc, int KC) {
@@ -788,7 +790,7 @@ void k_spmm_mfma_win(DevicePlan P, const uint16_t* __restrict__ B, int64_t ldb, 
       const int k = idx / per_row;
       const int ff = (idx % per_row) * VEC;
       const int c = P.tile_cols[t * 16 + k];
-      stage_fragment<VEC>(B, ldb, c, fbase + ff, K, bst + k * KCB + ff);
+      stage_fragment<VEC, RAG>(B, ldb, c, fbase + ff, K, bst + k * KCB + ff);
     }
     __syncthreads();
 #pragma unroll
@@ -823,7 +825,7 @@ void k_spmm_mfma_win(DevicePlan P, const uint16_t* __restrict__ B, int64_t ldb, 
           const int ff = (i2 % per_row) * VEC;
           const int c = P.quad_cols[(int64_t)q * 64 + k];
           const int f = fbase + 64 * j + ff;
-          stage_fragment<VEC>(B, ldb, c, f, K, bst + k * QS + ff);
+          stage_fragment<VEC, RAG>(B, ldb, c, f, K, bst + k * QS + ff);
         }
         __syncthreads();
         if (wave + 4 * j < ntn) {
@@ -855,7 +857,7 @@ void k_spmm_mfma_win(DevicePlan P, const uint16_t* __restrict__ B, int64_t ldb, 
   const int g = threadIdx.x / gs;
   const int ff = (threadIdx.x % gs) * VEC;
   const int f0 = fbase + ff;
-  const int f = row_window<VEC>(f0, K);
+  const int f = RAG ? row_window<VEC>(f0, K) : f0 < K ? f0 : 0;
   for (int rl = g; g < groups && rl < 16; rl += groups) {
     const int row = w.row0 + rl;
     if (row >= P.m) break;
@@ -867,7 +869,7 @@ void k_spmm_mfma_win(DevicePlan P, const uint16_t* __restrict__ B, int64_t ldb, 
     accumulate_row<VEC, 4, false, true>(P.col, P.val, B + f, ldb, P.rowptr[row], P.rowptr[row + 1],
                                         racc);
     if (f0 >= K) continue;
-    if constexpr (VEC > 1) {
+    if constexpr (RAG) {
       // the row's last VEC features: those from f0 on are this thread's
       if (f != f0) {
 #pragma unroll
@@ -1214,7 +1216,8 @@ __global__ __launch_bounds__(256) void k_sddmm_mfma(DevicePlan P, const uint16_t
 // the same lane/element -> feature assignment, so D[r][c] = X[r] . Y[c] whatever order the
 // instruction sums its 32 products in.  The loads of up to 4 steps (128 features) are issued
 // before their MFMAs.  Features past K read feature 0 and are zeroed in both operands; the lane at the end of a
-// K that 8 does not divide reads the row's last 8 features and zeroes the others' in both.
+// K that 8 does not divide (RAG) reads the row's last 8 features and zeroes the others' in both.
+template <bool RAG>
 __global__ __launch_bounds__(256) void k_sddmm_mfma32(DevicePlan P, const uint16_t* __restrict__ X, int64_t ldx,
                                                       const uint16_t* __restrict__ Y, int64_t ldy, int K,
                                                       float* __restrict__ out) {
@@ -1234,22 +1237,28 @@ __global__ __launch_bounds__(256) void k_sddmm_mfma32(DevicePlan P, const uint16
 #pragma unroll
     for (int i = 0; i < SPC; ++i) {
       const int k = k0 + 32 * i + fq;
-      const int kk = k < K ? row_window<8>(k, K) : 0;
+      const int kk = k >= K ? 0 : RAG ? row_window<8>(k, K) : k;
       a[i] = *reinterpret_cast<const half8_u*>(xp + kk);
       b[i] = *reinterpret_cast<const half8_u*>(yp + kk);
     }
 #pragma unroll
     for (int i = 0; i < SPC; ++i) {
-      // features of this step that are this lane's: none past the row's end, and the last ones of
-      // the row's last window
       const int k = k0 + 32 * i + fq;
-      const int skip = k < K ? k - row_window<8>(k, K) : 8;
+      if constexpr (RAG) {
+        // features of this step that are this lane's: none past the row's end, and the last ones of
+        // the row's last window
+        const int skip = k < K ? k - row_window<8>(k, K) : 8;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        a[i][j] = j < skip ? (_Float16)0 : a[i][j];
-        b[i][j] = j < skip ? (_Float16)0 : b[i][j];
+        for (int j = 0; j < 8; ++j) {
+          a[i][j] = j < skip ? (_Float16)0 : a[i][j];
+          b[i][j] = j < skip ? (_Float16)0 : b[i][j];
+        }
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[i], acc, 0, 0, 0);
+      } else {
+        const bool in = k < K;
+        const half8_t z{0, 0, 0, 0, 0, 0, 0, 0};
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(in ? a[i] : z, in ? b[i] : z, acc, 0, 0, 0);
       }
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[i], b[i], acc, 0, 0, 0);
     }
   }
   const int32_t* pos = P.tile_pos + (int64_t)t * 256;
@@ -1421,9 +1430,9 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     }                                                                                                     \
     break;                                                                                                \
   }
-    // 4- and 2-byte loads serve K <= 8 in groups of 4 lanes, 8-byte ones K <= 64 in 4 or 16 lanes
+    // 4- and 2-byte loads serve K <= 8 in groups of 4 or 8 lanes, 8-byte ones K <= 64 in 4 or 16 lanes
     if constexpr (VEC < 4) {
-      switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) }
+      switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) }
     } else if constexpr (VEC < 8) {
       switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) TRS_TASKS(16) }
     } else {
@@ -1453,8 +1462,15 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     const int cw = KC < 64 ? KC : 64;
     const size_t stage = std::max<size_t>((size_t)16 * (KC + 8), p.nquads > 0 ? (size_t)64 * (cw + 8) : 0);
     const size_t shm = (size_t)16 * (KC + 4) * 4 + stage * 2;
-    if (KC <= 64) hipLaunchKernelGGL((k_spmm_mfma_win<VEC, 1>), grid, dim3(256), shm, s, p, B, ldb, K, C, ldc, KC);
-    else hipLaunchKernelGGL((k_spmm_mfma_win<VEC, 2>), grid, dim3(256), shm, s, p, B, ldb, K, C, ldc, KC);
+#define TRS_WIN(NTILE, RAG) \
+    hipLaunchKernelGGL((k_spmm_mfma_win<VEC, NTILE, RAG>), grid, dim3(256), shm, s, p, B, ldb, K, C, ldc, KC)
+    const bool rag = VEC > 1 && K % VEC != 0;
+    if (KC <= 64) {
+      if (rag) TRS_WIN(1, (VEC > 1)); else TRS_WIN(1, false);
+    } else if constexpr (VEC == 8) {
+      if (rag) TRS_WIN(2, true); else TRS_WIN(2, false);
+    }
+#undef TRS_WIN
   }
   if (ev) (void)hipEventRecord(ev[2], s);
   if (p.nfixups > 0 || p.nwfixups > 0) {
@@ -1462,7 +1478,7 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     dim3 grid(p.nwfixups + (p.nfixups + gpb - 1) / gpb, passes);
 #define TRS_FIX(L) case L: hipLaunchKernelGGL((k_spmm_fixup<VEC, L>), grid, dim3(256), 0, s, p, K, C, ldc, partial); break;
     if constexpr (VEC < 4) {
-      switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) }
+      switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) }
     } else if constexpr (VEC < 8) {
       switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) TRS_FIX(16) }
     } else {
@@ -1627,7 +1643,8 @@ hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx,
     dim3 grid((p.ntiles + 3) / 4);
     // 16x16x32 with 16-byte loads issued ahead (same-box A/B on SBM 1M: K=128 0.174 -> 0.116 ms,
     // K=256 0.314 -> 0.205 ms; K=32 unchanged)
-    if (v8) hipLaunchKernelGGL(k_sddmm_mfma32, grid, dim3(256), 0, s, p, X, ldx, Y, ldy, K, out);
+    if (v8 && K % 8 != 0) hipLaunchKernelGGL(k_sddmm_mfma32<true>, grid, dim3(256), 0, s, p, X, ldx, Y, ldy, K, out);
+    else if (v8) hipLaunchKernelGGL(k_sddmm_mfma32<false>, grid, dim3(256), 0, s, p, X, ldx, Y, ldy, K, out);
     else if (v4) hipLaunchKernelGGL((k_sddmm_mfma<true>), grid, dim3(256), 0, s, p, X, ldx, Y, ldy, K, out);
     else hipLaunchKernelGGL((k_sddmm_mfma<false>), grid, dim3(256), 0, s, p, X, ldx, Y, ldy, K, out);
   }
@@ -2010,7 +2027,10 @@ hipError_t launch_spmm(const DevicePlan& p, const uint16_t* B, int64_t ldb, int 
   // 464, 52 568 / 442, 63 696 / 518 (2-byte loads before: 992, 1013, 440 with 8 bytes, 1130); grid of
   // 4M nodes with hubs K = 41 760 / 700; on the grid 16-byte loads stay (K = 64 457 us).
   const bool rows16 = K % 8 == 0 && ldb % 8 == 0 && aligned16(B);
-  const bool v8 = K > 16 && (K <= 32 || K > 64 || rows16), v4 = K > 8, v2 = K > 4;
+  // K = 5 and 7 stay on 8 lanes of 2 bytes over short rows (grid of 2M nodes K = 7: 109 us, 127 with 4-byte
+  // loads; R-MAT, whose tasks are long, 336 / 262)
+  const bool v8 = K > 16 && (K <= 32 || K > 64 || rows16), v4 = K > 8,
+             v2 = K > 4 && (K % 2 == 0 || K > 8 || p.task_nnz >= 64);
   // (the staged hot rows need 16-byte aligned rows in the buffer too)
   if (hot != nullptr && !aligned16(hot)) hot = nullptr;
   return v8 ? spmm_width<8>(p, B, ldb, K, C, ldc, partial, hot, stream, ev)
