@@ -1340,6 +1340,30 @@ int lanes_for(int K, int vec) {
   return l;
 }
 
+// The MFMA windows with B rows staged VEC features per load.
+template <int VEC>
+void launch_windows_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
+                        hipStream_t s) {
+  const int kc16 = ((K + 15) / 16) * 16;
+  // at most 128 features per workgroup: wider B slices in flight per window cost L2 capacity
+  // (SBM 1M, K = 256: 0.912 ms with 256 features per workgroup, 0.871 with two of 128)
+  const int KC = kc16 < 128 ? kc16 : 128;
+  dim3 grid(p.nmwin, (K + KC - 1) / KC);
+  // staging space: 16 dense-tile B rows of KC features, or a quad's 64 rows of min(KC, 64)
+  const int cw = KC < 64 ? KC : 64;
+  const size_t stage = std::max<size_t>((size_t)16 * (KC + 8), p.nquads > 0 ? (size_t)64 * (cw + 8) : 0);
+  const size_t shm = (size_t)16 * (KC + 4) * 4 + stage * 2;
+#define TRS_WIN(NTILE, RAG) \
+  hipLaunchKernelGGL((k_spmm_mfma_win<VEC, NTILE, RAG>), grid, dim3(256), shm, s, p, B, ldb, K, C, ldc, KC)
+  const bool rag = VEC > 1 && K % VEC != 0;
+  if (KC <= 64) {
+    if (rag) TRS_WIN(1, (VEC > 1)); else TRS_WIN(1, false);
+  } else if constexpr (VEC == 8) {
+    if (rag) TRS_WIN(2, true); else TRS_WIN(2, false);
+  }
+#undef TRS_WIN
+}
+
 template <int VEC>
 hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
                            float* partial, uint16_t* hot, hipStream_t s, hipEvent_t* ev) {
@@ -1452,26 +1476,7 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     run_tasks(tp, xv);
   }
   if (ev) (void)hipEventRecord(ev[1], s);
-  if (p.nmwin > 0) {
-    const int kc16 = ((K + 15) / 16) * 16;
-    // at most 128 features per workgroup: wider B slices in flight per window cost L2 capacity
-    // (SBM 1M, K = 256: 0.912 ms with 256 features per workgroup, 0.871 with two of 128)
-    const int KC = kc16 < 128 ? kc16 : 128;
-    dim3 grid(p.nmwin, (K + KC - 1) / KC);
-    // staging space: 16 dense-tile B rows of KC features, or a quad's 64 rows of min(KC, 64)
-    const int cw = KC < 64 ? KC : 64;
-    const size_t stage = std::max<size_t>((size_t)16 * (KC + 8), p.nquads > 0 ? (size_t)64 * (cw + 8) : 0);
-    const size_t shm = (size_t)16 * (KC + 4) * 4 + stage * 2;
-#define TRS_WIN(NTILE, RAG) \
-    hipLaunchKernelGGL((k_spmm_mfma_win<VEC, NTILE, RAG>), grid, dim3(256), shm, s, p, B, ldb, K, C, ldc, KC)
-    const bool rag = VEC > 1 && K % VEC != 0;
-    if (KC <= 64) {
-      if (rag) TRS_WIN(1, (VEC > 1)); else TRS_WIN(1, false);
-    } else if constexpr (VEC == 8) {
-      if (rag) TRS_WIN(2, true); else TRS_WIN(2, false);
-    }
-#undef TRS_WIN
-  }
+  launch_spmm_windows(p, B, ldb, K, C, ldc, s);
   if (ev) (void)hipEventRecord(ev[2], s);
   if (p.nfixups > 0 || p.nwfixups > 0) {
     const int gpb = 4 * (64 / lpg);
@@ -1888,6 +1893,8 @@ template <int VEC>
 hipError_t spmm_width(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
                       float* partial, uint16_t* hot, hipStream_t s, hipEvent_t* ev);
 template <int VEC>
+void windows_width(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc, hipStream_t s);
+template <int VEC>
 hipError_t sddmm_width(const DevicePlan& p, const uint16_t* X, int64_t ldx, const uint16_t* Y, int64_t ldy, int K,
                        float* out, uint16_t* hot, float* xbuf, hipStream_t s, hipEvent_t* ev);
 #if TRS_KERNEL_PART > 0
@@ -1895,6 +1902,10 @@ template <int VEC>
 hipError_t spmm_width(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
                       float* partial, uint16_t* hot, hipStream_t s, hipEvent_t* ev) {
   return launch_spmm_vec<VEC>(p, B, ldb, K, C, ldc, partial, hot, s, ev);
+}
+template <int VEC>
+void windows_width(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc, hipStream_t s) {
+  launch_windows_vec<VEC>(p, B, ldb, K, C, ldc, s);
 }
 template <int VEC>
 hipError_t sddmm_width(const DevicePlan& p, const uint16_t* X, int64_t ldx, const uint16_t* Y, int64_t ldy, int K,
@@ -1905,6 +1916,8 @@ hipError_t sddmm_width(const DevicePlan& p, const uint16_t* X, int64_t ldx, cons
 #define TRS_WIDTH_INSTANCES(PREFIX, V)                                                                       \
   PREFIX template hipError_t spmm_width<V>(const DevicePlan&, const uint16_t*, int64_t, int, float*, int64_t, \
                                            float*, uint16_t*, hipStream_t, hipEvent_t*);                      \
+  PREFIX template void windows_width<V>(const DevicePlan&, const uint16_t*, int64_t, int, float*, int64_t,    \
+                                        hipStream_t);                                                         \
   PREFIX template hipError_t sddmm_width<V>(const DevicePlan&, const uint16_t*, int64_t, const uint16_t*,     \
                                             int64_t, int, float*, uint16_t*, float*, hipStream_t, hipEvent_t*);
 #if TRS_KERNEL_PART > 0
@@ -2006,6 +2019,21 @@ hipError_t launch_place_entries(const PlaceEntries& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
+void launch_spmm_windows(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
+                         hipStream_t stream) {
+  if (p.nmwin <= 0) return;
+  // B rows are staged with 16-byte loads where the task kernel takes 8-byte ones (K = 40 / 50 / 64 on SBM of
+  // 250K nodes: 59 / 70 / 56 us, 62 / 74 / 65 with 8-byte loads), but for odd rows of about that width (K =
+  // 31 / 33 / 41: 57 / 65 / 69, 55 / 62 / 66)
+  if (K > 16 && !(K % 2 != 0 && K > 24 && K <= 64)) windows_width<8>(p, B, ldb, K, C, ldc, stream);
+  else if (K > 8) windows_width<4>(p, B, ldb, K, C, ldc, stream);
+  else if (K > 4) windows_width<2>(p, B, ldb, K, C, ldc, stream);
+  else windows_width<1>(p, B, ldb, K, C, ldc, stream);
+}
+
+// Bytes a call reads and writes at least (entries, B, C) past which its gathers wait on HBM.
+constexpr int64_t kBeyondMall = 320'000'000;
+
 hipError_t launch_spmm(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
                        float* partial, uint16_t* hot, hipStream_t stream, hipEvent_t* ev) {
   // wide loads only where they leave at least 4 lanes per group (whose column/value loads are
@@ -2025,11 +2053,16 @@ hipError_t launch_spmm(const DevicePlan& p, const uint16_t* B, int64_t ldb, int 
   // K = 33..64 off the 16-byte grid keep 8-byte loads in 16-lane groups, whose staged stream holds
   // more entries in flight than 8-lane groups held to 2 waves: K = 33 595 (16-byte) / 454, 41 622 /
   // 464, 52 568 / 442, 63 696 / 518 (2-byte loads before: 992, 1013, 440 with 8 bytes, 1130); grid of
-  // 4M nodes with hubs K = 41 760 / 700; on the grid 16-byte loads stay (K = 64 457 us).
-  const bool rows16 = K % 8 == 0 && ldb % 8 == 0 && aligned16(B);
+  // 4M nodes with hubs K = 41 760 / 700.  On the 16-byte grid they do so where the call's operands are
+  // well beyond the 256 MB MALL, where the gathers wait on HBM (R-MAT 2^20 with 31M entries K = 40 / 48
+  // / 56 / 64 505 / 507 / 564 / 459 -> 410 / 410 / 438 / 419 us, grid of 4M nodes K = 40 / 56 / 64 622 /
+  // 753 / 588 -> 606 / 735 / 572), and not below (grid of 640K nodes K = 48 / 64 74 / 71 -> 83 / 83,
+  // R-MAT 2^18 K = 64 112 -> 122).
   // K = 5 and 7 stay on 8 lanes of 2 bytes over short rows (grid of 2M nodes K = 7: 109 us, 127 with 4-byte
   // loads; R-MAT, whose tasks are long, 336 / 262)
-  const bool v8 = K > 16 && (K <= 32 || K > 64 || rows16), v4 = K > 8,
+  const bool aligned = K % 8 == 0 && ldb % 8 == 0 && aligned16(B);
+  const int64_t touched = p.nnz_csr * 6 + (int64_t)p.m * K * 4 + (int64_t)p.n * K * 2;
+  const bool v8 = K > 16 && (K <= 32 || K > 64 || (aligned && touched < kBeyondMall)), v4 = K > 8,
              v2 = K > 4 && (K % 2 == 0 || K > 8 || p.task_nnz >= 64);
   // (the staged hot rows need 16-byte aligned rows in the buffer too)
   if (hot != nullptr && !aligned16(hot)) hot = nullptr;

@@ -230,6 +230,9 @@ hipError_t launch_gather_group_tiles(const int32_t* ids, int32_t nids, const int
 // the three kernels.
 hipError_t launch_spmm(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
                        float* partial, uint16_t* hot, hipStream_t stream, hipEvent_t* ev = nullptr);
+// The plan's MFMA windows (a part of launch_spmm).
+void launch_spmm_windows(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
+                         hipStream_t stream);
 // out[0, n) = 0 with a kernel (not a memset node: callers may capture the stream in a graph).
 hipError_t launch_zero_fill(float* out, int64_t n, hipStream_t stream);
 // hot: as for launch_spmm, Y rows.  xbuf: the split part's own output buffer
