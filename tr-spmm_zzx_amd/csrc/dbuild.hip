@@ -45,7 +45,8 @@ namespace {
 
 using u64 = unsigned long long;
 
-constexpr int kSmallU = 8192;       // windows with more distinct columns take the workgroup kernel
+constexpr int kSmallU = 2048;       // windows with more distinct columns take the workgroup kernel
+constexpr int kNarrowU = 1024;      // windows of at most this many, the narrow launch of the wave kernel
 constexpr int kBlockWaves = 8;      // waves of that kernel
 constexpr int kLdsUnits = 65536;    // most units whose order it keeps in LDS (16-bit indices; the
                                     // device's LDS per workgroup may allow fewer)
@@ -916,16 +917,18 @@ __device__ void plan_window(const Build& B, int32_t w, P* perm, uint32_t* taken,
   }
 }
 
-// Windows of at most kSmallU distinct columns, one wave each (workgroups of one wave); matched
-// pairs go to the window's part of B.pairs.
+// Windows of (LO, CAP] distinct columns, CAP <= kSmallU, one wave each (workgroups of one wave); matched
+// pairs go to the window's part of B.pairs.  The LDS is sized by CAP, so that the many narrow windows
+// run 32 to a CU, not the 8 that kSmallU leaves room for (R-MAT 2^18: 1200 us in one launch -> 325 in two).
+template <int LO, int CAP>
 __global__ __launch_bounds__(64) void k_plan_small(Build B) {
   const int32_t w = blockIdx.x;
   const int32_t ub = B.ubase[w], U = B.ubase[w + 1] - ub;
-  if (U > kSmallU) return;
-  __shared__ uint16_t perm[kSmallU / 2 + 1];
-  __shared__ uint8_t unnz[kSmallU / 2 + 1];
-  __shared__ uint8_t leaf[kSmallU / 2 + 1];
-  __shared__ uint32_t taken[kSmallU / 64 + 2];
+  if ((LO > 0 && U <= LO) || U > CAP) return;
+  __shared__ uint16_t perm[CAP / 2 + 1];
+  __shared__ uint8_t unnz[CAP / 2 + 1];
+  __shared__ uint8_t leaf[CAP / 2 + 1];
+  __shared__ uint32_t taken[CAP / 64 + 2];
   __shared__ int LR[256];
   __shared__ int GB[512];
   __shared__ WinShared sh;
@@ -1141,29 +1144,51 @@ __global__ __launch_bounds__(256) void k_fill_groups(Build B, Out O, int64_t ite
   const int32_t w = O.s_win[g];
   const int32_t ub = B.ubase[w];
   const int32_t* gl = B.gl + ub + 4 * w + (int64_t)(g - B.wgroups[w]) * 4;
+  // all four members' masks and first positions at once (an absent member reads the window's first
+  // column), then the row's entries: three round trips behind the group's, where a member at a time
+  // took up to sixteen (R-MAT 2^18: 550 us -> 327)
+  int32_t m[4], first[4];
+  uint32_t mask[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) m[q] = gl[q];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int32_t u = ub + max(m[q], 0);
+    mask[q] = B.umask[u];
+    first[q] = B.ufirst[u];
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q)
+    if (q % ws == lr) O.s_col[(int64_t)g * 4 + q] = m[q] >= 0 ? B.ucol[ub + m[q]] : -1;
   uint32_t present = 0;
   int kept = 0;
-  float v[2] = {0.f, 0.f};
-  int p[2] = {-1, -1};
+  int p0 = -1, p1 = -1;
+  int32_t s0 = 0, s1 = 0;   // sorted positions of the row's first two members
+#pragma unroll
   for (int q = 0; q < 4; ++q) {
-    const int32_t m = gl[q];
-    if (lr == 0) O.s_col[(int64_t)g * 4 + q] = m >= 0 ? B.ucol[ub + m] : -1;
-    if (m < 0 || !((B.umask[ub + m] >> lr) & 1u)) continue;
+    if (m[q] < 0 || !((mask[q] >> lr) & 1u)) continue;
     present |= 1u << q;
-    const int32_t e = entry_of(B, ub + m, lr);
-    if (kept < 2) {
-      v[kept] = B.val[e];
-      p[kept] = q;
+    const int32_t at = first[q] + popc32(mask[q] & ((1u << lr) - 1u));
+    if (kept == 0) {
+      p0 = q;
+      s0 = at;
+    } else if (kept == 1) {
+      p1 = q;
+      s1 = at;
     } else {
-      B.spill[e] = 1;
+      B.spill[B.s_e[at]] = 1;
     }
     ++kept;
   }
+  float2 v{0.f, 0.f};
+  if (kept > 0) {
+    const int32_t e0 = B.s_e[s0], e1 = kept > 1 ? B.s_e[s1] : -1;
+    v.x = B.val[e0];
+    if (kept > 1) v.y = B.val[e1];
+  }
   O.s_mask[t] = (uint8_t)present;
-  O.s_val[2 * t] = v[0];
-  O.s_val[2 * t + 1] = v[1];
-  O.s_pos[2 * t] = (int8_t)p[0];
-  O.s_pos[2 * t + 1] = (int8_t)p[1];
+  reinterpret_cast<float2*>(O.s_val)[t] = v;
+  reinterpret_cast<uint16_t*>(O.s_pos)[t] = (uint16_t)((uint32_t)(p0 & 0xff) | ((uint32_t)(p1 & 0xff) << 8));
 }
 
 // block_online.cpp:190-210 (g window-local, gend the window's group count)
@@ -1174,8 +1199,10 @@ __device__ __forceinline__ void load_chunk(const Out& O, int64_t gb, int g, int 
   p1 = 1;
   if (g >= gend || lr >= ws) return;
   const int64_t b = ((gb + g) * ws + lr) * 2;
-  const int q0 = O.s_pos[b], q1 = O.s_pos[b + 1];
-  const float a0 = O.s_val[b], a1 = O.s_val[b + 1];
+  const uint32_t pp = *reinterpret_cast<const uint16_t*>(O.s_pos + b);   // (b is even)
+  const int q0 = (int8_t)(pp & 0xff), q1 = (int8_t)(pp >> 8);
+  const float2 av = *reinterpret_cast<const float2*>(O.s_val + b);
+  const float a0 = av.x, a1 = av.y;
   if (q0 < 0 && q1 < 0) return;
   if (q0 >= 0 && q1 >= 0) {
     if (q0 <= q1) {
@@ -1197,35 +1224,44 @@ __device__ __forceinline__ void load_chunk(const Out& O, int64_t gb, int g, int 
 
 __device__ __forceinline__ uint16_t f16_bits(float f) { return trs::half_bits_of(__float_as_uint(f)); }
 
-// Tile t: 4 groups of its window (block_online.cpp:796-841).
+// Tile t: 4 groups of its window (block_online.cpp:796-841), one thread per pair of rows rg, rg + 8, so
+// that a tile's threads read neighbouring rows of its groups and write one run of its packed values
+// (one thread per tile, 32 bytes to a store instruction of 64 lanes 256 bytes apart: R-MAT 2^18 711 us ->
+// 163).
 __global__ __launch_bounds__(256) void k_fill_tiles(Build B, Out O, int32_t ntiles) {
-  const int32_t t = (int32_t)(blockIdx.x * 256 + threadIdx.x);
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int32_t t = (int32_t)(i >> 3);
+  const int rg = (int)(i & 7);
   if (t >= ntiles) return;
   const int ws = B.ws;
   const int32_t w = window_of(B.wtiles, B.nwin, t);
   const int32_t gb = B.wgroups[w], G = B.wgroups[w + 1] - gb;
   const int base = (t - B.wtiles[w]) * 4;
-  O.tile_win[t] = w;
-  O.tile_group[t] = gb + base;
-  for (int k = 0; k < 16; ++k) {
-    const int g = base + k / 4;
-    O.tile_cols[(int64_t)t * 16 + k] = g < G ? O.s_col[((int64_t)gb + g) * 4 + k % 4] : -1;
+  if (rg == 0) {
+    O.tile_win[t] = w;
+    O.tile_group[t] = gb + base;
   }
-  for (int rg = 0; rg < 8; ++rg) {
-    float a[16];
-    uint32_t meta = 0;
-    for (int c = 0; c < 4; ++c) {
-      int p0, p1;
-      load_chunk(O, gb, base + c, G, rg, ws, a[4 * c], a[4 * c + 1], p0, p1);
-      meta |= ((uint32_t)(p0 & 3) | ((uint32_t)(p1 & 3) << 2)) << (4 * c);
-      load_chunk(O, gb, base + c, G, rg + 8, ws, a[4 * c + 2], a[4 * c + 3], p0, p1);
-      meta |= ((uint32_t)(p0 & 3) | ((uint32_t)(p1 & 3) << 2)) << (16 + 4 * c);
-    }
-    O.packed_meta[(int64_t)t * 8 + rg] = (int32_t)meta;
-    for (int j = 0; j < 8; ++j)
-      O.packed_a[((int64_t)t * 8 + rg) * 8 + j] =
-          (int32_t)((uint32_t)f16_bits(a[2 * j]) | ((uint32_t)f16_bits(a[2 * j + 1]) << 16));
+  const int g = base + rg / 2;   // columns 2 rg and 2 rg + 1 of the tile
+  int2 c{-1, -1};
+  if (g < G) c = *reinterpret_cast<const int2*>(O.s_col + ((int64_t)gb + g) * 4 + 2 * (rg & 1));
+  reinterpret_cast<int2*>(O.tile_cols)[i] = c;
+  float a[16];
+  uint32_t meta = 0;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    int p0, p1;
+    load_chunk(O, gb, base + k, G, rg, ws, a[4 * k], a[4 * k + 1], p0, p1);
+    meta |= ((uint32_t)(p0 & 3) | ((uint32_t)(p1 & 3) << 2)) << (4 * k);
+    load_chunk(O, gb, base + k, G, rg + 8, ws, a[4 * k + 2], a[4 * k + 3], p0, p1);
+    meta |= ((uint32_t)(p0 & 3) | ((uint32_t)(p1 & 3) << 2)) << (16 + 4 * k);
   }
+  O.packed_meta[i] = (int32_t)meta;
+  int32_t h[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) h[j] = (int32_t)((uint32_t)f16_bits(a[2 * j]) | ((uint32_t)f16_bits(a[2 * j + 1]) << 16));
+  int4* dst = reinterpret_cast<int4*>(O.packed_a + i * 8);
+  dst[0] = make_int4(h[0], h[1], h[2], h[3]);
+  dst[1] = make_int4(h[4], h[5], h[6], h[7]);
 }
 
 // Residual parts of row r (block_online.cpp:397-439, :705-733): entries of the window's residual
@@ -1480,7 +1516,8 @@ int trs_build_online_device(const int32_t* rowptr, const int32_t* col, const flo
     return fail(TRS_EDEVICE, "hipMemsetAsync failed");
   if (W > 0) {
     hipLaunchKernelGGL(k_list_large, dim3(grid_of(W)), dim3(256), 0, s, B, big, nbig_d);
-    hipLaunchKernelGGL(k_plan_small, dim3(W), dim3(64), 0, s, B);
+    hipLaunchKernelGGL((k_plan_small<kNarrowU, kSmallU>), dim3(W), dim3(64), 0, s, B);
+    hipLaunchKernelGGL((k_plan_small<0, kNarrowU>), dim3(W), dim3(64), 0, s, B);
     int32_t nbig = 0;
     if (hipMemcpyAsync(&nbig, nbig_d, 4, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
       return fail(TRS_EDEVICE, std::string("trs_build_online_device: ") + hipGetErrorString(hipGetLastError()));
@@ -1615,7 +1652,7 @@ int trs_build_online_device(const int32_t* rowptr, const int32_t* col, const flo
     hipLaunchKernelGGL(k_group_windows, dim3(grid_of(G)), dim3(256), 0, s, B, O, (int32_t)G);
     hipLaunchKernelGGL(k_fill_groups, dim3(grid_of(G * ws)), dim3(256), 0, s, B, O, G * ws);
   }
-  if (T > 0) hipLaunchKernelGGL(k_fill_tiles, dim3(grid_of(T)), dim3(256), 0, s, B, O, (int32_t)T);
+  if (T > 0) hipLaunchKernelGGL(k_fill_tiles, dim3(grid_of(T * 8)), dim3(256), 0, s, B, O, (int32_t)T);
   hipLaunchKernelGGL(k_fill_residual, dim3(grid_of(std::max(rows, 1))), dim3(256), 0, s, B, O);
   if (scan(B.spill, nnz, B.spill_at, bsum2, s) != hipSuccess) return fail_f(TRS_EDEVICE, "scan failed");
   int32_t nsp = 0;

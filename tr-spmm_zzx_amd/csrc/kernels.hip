@@ -1664,7 +1664,9 @@ hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx,
 #if TRS_KERNEL_PART == 0
 
 // One workgroup per tile, one thread per (row, column) slot: binary search of the column in the
-// CSR row (columns ascending) and mark the entry; an entry counts when its flag was clear.
+// CSR row (columns ascending) and mark the entry; an entry counts when its flag was clear.  The count
+// takes one atomic per workgroup: with one per entry, all on one address, SBM of 1M nodes (62.5K tiles,
+// 7.2M entries) took 2880 us, now 750.
 __global__ __launch_bounds__(256) void k_mark_tile_entries(const TileEntries* __restrict__ tiles, int32_t m,
                                                            const int32_t* __restrict__ rowptr,
                                                            const int32_t* __restrict__ col,
@@ -1674,19 +1676,23 @@ __global__ __launch_bounds__(256) void k_mark_tile_entries(const TileEntries* __
   const TileEntries& t = tiles[blockIdx.x];
   const int r = threadIdx.x >> 4, k = threadIdx.x & 15;
   const int row = t.row0 + r;
-  if (!((t.present[r >> 2] >> ((r & 3) * 16 + k)) & 1) || row >= m) return;
-  const int32_t c = t.cols[k];
-  int lo = rowptr[row], hi = rowptr[row + 1];
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (col[mid] < c) lo = mid + 1;
-    else hi = mid;
+  int fresh = 0;
+  if (((t.present[r >> 2] >> ((r & 3) * 16 + k)) & 1) && row < m) {
+    const int32_t c = t.cols[k];
+    int lo = rowptr[row], hi = rowptr[row + 1];
+    while (lo < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (col[mid] < c) lo = mid + 1;
+      else hi = mid;
+    }
+    if (lo < rowptr[row + 1] && col[lo] == c) {
+      const uint32_t bit = 1u << ((lo & 3) * 8);
+      fresh = !(atomicOr(flag_words + (lo >> 2), bit) & bit);
+      if (tile_pos) tile_pos[(int64_t)blockIdx.x * 256 + threadIdx.x] = lo;
+    }
   }
-  if (lo < rowptr[row + 1] && col[lo] == c) {
-    const uint32_t bit = 1u << ((lo & 3) * 8);
-    if (!(atomicOr(flag_words + (lo >> 2), bit) & bit)) atomicAdd(marked, 1u);
-    if (tile_pos) tile_pos[(int64_t)blockIdx.x * 256 + threadIdx.x] = lo;
-  }
+  const int n = __syncthreads_count(fresh);
+  if (threadIdx.x == 0 && n > 0) atomicAdd(marked, (uint32_t)n);
 }
 
 // Bits of `mask` below this lane.
@@ -1695,7 +1701,10 @@ __device__ __forceinline__ int lanes_below(uint64_t mask) {
 }
 
 // One wave per CSR row: 64 entries at a time, destinations from wave ballots, so each row keeps its
-// column order.
+// column order.  The columns and values of kPlaceAhead steps are loaded before the first is placed: a hub
+// row is one wave's chain of steps, and with one step's loads in flight its round trips were the kernel's
+// time (R-MAT 2^18 475 us -> 257; grid of 4M nodes, hubs of 100K entries, 2771 -> 1755).
+constexpr int kPlaceAhead = 8;
 __global__ __launch_bounds__(256) void k_place_entries(const PlaceEntries a) {
   const int row = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
@@ -1706,39 +1715,73 @@ __global__ __launch_bounds__(256) void k_place_entries(const PlaceEntries a) {
     int cur[kXcds];
 #pragma unroll
     for (int x = 0; x < kXcds; ++x) cur[x] = a.cursor[si * kXcds + x];
-    for (int p = b; p < e; p += 64) {
-      const int q = p + lane;
-      const bool in = q < e;
-      const int32_t c = in ? a.col[q] : 0;
-      const int xq = xcd_of_column(c);
-      int dst = 0;
+    for (int p0 = b; p0 < e; p0 += 64 * kPlaceAhead) {
+      int32_t cs[kPlaceAhead];
+      float vs[kPlaceAhead];
 #pragma unroll
-      for (int x = 0; x < kXcds; ++x) {
-        const uint64_t mask = __ballot(in && xq == x);
-        if (in && xq == x) dst = cur[x] + lanes_below(mask);
-        cur[x] += __popcll(mask);
+      for (int k = 0; k < kPlaceAhead; ++k) {   // steps past the row read its last entry
+        const int q = min(p0 + k * 64 + lane, e - 1);
+        cs[k] = a.col[q];
+        vs[k] = a.val_out ? a.val[q] : 0.f;
       }
-      if (in) {
-        a.col_out[dst] = c;
-        if (a.val_out) a.val_out[dst] = half_bits_of(__builtin_bit_cast(uint32_t, a.val[q]));
-        if (a.x_pos) a.x_pos[dst - a.x_base] = q;
-        if (a.x_src) a.x_src[a.merge_off[si] + (q - b)] = (int32_t)(dst - a.x_base);
+#pragma unroll
+      for (int k = 0; k < kPlaceAhead; ++k) {
+        const int q = p0 + k * 64 + lane;
+        if (p0 + k * 64 >= e) break;
+        const bool in = q < e;
+        const int32_t c = cs[k];
+        const int xq = xcd_of_column(c);
+        int dst = 0;
+#pragma unroll
+        for (int x = 0; x < kXcds; ++x) {
+          const uint64_t mask = __ballot(in && xq == x);
+          if (in && xq == x) dst = cur[x] + lanes_below(mask);
+          cur[x] += __popcll(mask);
+        }
+        if (in) {
+          a.col_out[dst] = c;
+          if (a.val_out) a.val_out[dst] = half_bits_of(__builtin_bit_cast(uint32_t, vs[k]));
+          if (a.x_pos) a.x_pos[dst - a.x_base] = q;
+          if (a.x_src) a.x_src[a.merge_off[si] + (q - b)] = (int32_t)(dst - a.x_base);
+        }
       }
     }
     if (a.compact) return;
   }
   int out = a.main_rowptr[row];
-  for (int p = b; p < e; p += 64) {
-    const int q = p + lane;
-    const bool keep = q < e && !(a.flag && a.flag[q]);
+  auto place = [&](int q, bool keep, int32_t c, float v) {
     const uint64_t mask = __ballot(keep);
     if (keep) {
       const int dst = out + lanes_below(mask);
-      a.col_out[dst] = a.col[q];
-      if (a.val_out) a.val_out[dst] = half_bits_of(__builtin_bit_cast(uint32_t, a.val[q]));
+      a.col_out[dst] = c;
+      if (a.val_out) a.val_out[dst] = half_bits_of(__builtin_bit_cast(uint32_t, v));
       if (a.res_pos) a.res_pos[dst] = q;
     }
     out += __popcll(mask);
+  };
+  int p0 = b;
+  for (; e - p0 > 64; p0 += 64 * kPlaceAhead) {
+    int32_t cs[kPlaceAhead];
+    float vs[kPlaceAhead];
+    uint8_t fs[kPlaceAhead];
+#pragma unroll
+    for (int k = 0; k < kPlaceAhead; ++k) {
+      const int q = min(p0 + k * 64 + lane, e - 1);
+      cs[k] = a.col[q];
+      vs[k] = a.val_out ? a.val[q] : 0.f;
+      fs[k] = a.flag ? a.flag[q] : (uint8_t)0;
+    }
+#pragma unroll
+    for (int k = 0; k < kPlaceAhead; ++k) {
+      if (p0 + k * 64 >= e) break;
+      const int q = p0 + k * 64 + lane;
+      place(q, q < e && !fs[k], cs[k], vs[k]);
+    }
+  }
+  if (p0 < e) {   // at most one step (most rows are no longer)
+    const int q = p0 + lane;
+    const bool keep = q < e && !(a.flag && a.flag[q]);
+    place(q, keep, keep ? a.col[q] : 0, keep && a.val_out ? a.val[q] : 0.f);
   }
 }
 
@@ -1753,6 +1796,36 @@ __global__ __launch_bounds__(256) void k_count_columns(const int32_t* __restrict
     const int32_t c = col[e];
     if (c >= 0 && c < n) atomicAdd(&h[c], 1);
   }
+}
+
+// The same with the counters in LDS: workgroup (r, g) counts the entries of group g of the list that lie in
+// columns [r * kCountSpan, (r + 1) * kCountSpan) and writes them to copy g of the histogram, every counter
+// once.  The list is read once per range of columns, from the L2s and the MALL for the most part, where
+// global atomics take 14 G a second whatever their spread: R-MAT 2^18 (7.9M entries, 8 ranges) 575 us ->
+// 43, R-MAT 2^20 (31M, 32 ranges) 2673 -> 462.
+__global__ __launch_bounds__(1024) void k_count_columns_lds(const int32_t* __restrict__ col, int64_t total, int32_t n,
+                                                            int32_t* __restrict__ counts) {
+  extern __shared__ int32_t hist[];   // kCountSpan counters
+  const int32_t lo = (int32_t)blockIdx.x * kCountSpan;
+  const int32_t span = min(kCountSpan, n - lo);
+  for (int32_t i = threadIdx.x; i < span; i += 1024) hist[i] = 0;
+  __syncthreads();
+  const int64_t per = (total + gridDim.y - 1) / gridDim.y;
+  const int64_t b = per * blockIdx.y, e = min(b + per, total);
+  constexpr int AHEAD = 8;
+  for (int64_t p = b + threadIdx.x; p < e; p += 1024 * AHEAD) {
+    int32_t c[AHEAD];
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) c[k] = p + k * 1024 < e ? col[p + k * 1024] : -1;
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) {
+      const uint32_t i = (uint32_t)(c[k] - lo);
+      if (c[k] >= lo && i < (uint32_t)span) atomicAdd(&hist[i], 1);
+    }
+  }
+  __syncthreads();
+  int32_t* out = counts + (int64_t)blockIdx.y * n + lo;
+  for (int32_t i = threadIdx.x; i < span; i += 1024) out[i] = hist[i];
 }
 
 // counts[c] = sum of the copies' counts of column c (copy 0 is counts itself).
@@ -1810,12 +1883,21 @@ __global__ __launch_bounds__(256) void k_split_stats(const int32_t* __restrict__
   const int32_t* c = col + start[i];
   const int32_t n = len[i];
   int32_t k[kXcds] = {};
-  for (int32_t q = l; q < n; q += 64) {
-    const int32_t v = c[q];
-    const int x = xcd_of_column(v);
+  // eight steps' columns loaded at once, as in k_place_entries (R-MAT 2^18 360 us -> 295)
+  constexpr int kAhead = 8;
+  for (int32_t q0 = l; q0 < n; q0 += 64 * kAhead) {
+    int32_t vs[kAhead];
 #pragma unroll
-    for (int y = 0; y < kXcds; ++y) k[y] += x == y;
-    if (seen) __hip_atomic_store(seen + v, (uint8_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int i = 0; i < kAhead; ++i) vs[i] = c[min(q0 + i * 64, n - 1)];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      if (q0 + i * 64 >= n) break;
+      const int32_t v = vs[i];
+      const int x = xcd_of_column(v);
+#pragma unroll
+      for (int y = 0; y < kXcds; ++y) k[y] += x == y;
+      if (seen) __hip_atomic_store(seen + v, (uint8_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
   }
 #pragma unroll
   for (int y = 0; y < kXcds; ++y) {
@@ -1944,7 +2026,15 @@ hipError_t launch_count_columns(const int32_t* col, int64_t total, int32_t n, in
                                 hipStream_t stream) {
   if (total <= 0 || n <= 0) return hipSuccess;
   if (copies < 1) copies = 1;
-  hipLaunchKernelGGL(k_count_columns, dim3(stride_grid(total)), dim3(256), 0, stream, col, total, n, counts, copies);
+  if (counts_in_lds(n)) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(k_count_columns_lds),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, kCountSpan * 4);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(k_count_columns_lds, dim3((unsigned)((n + kCountSpan - 1) / kCountSpan), (unsigned)copies),
+                       dim3(1024), kCountSpan * 4, stream, col, total, n, counts);
+  } else {
+    hipLaunchKernelGGL(k_count_columns, dim3(stride_grid(total)), dim3(256), 0, stream, col, total, n, counts, copies);
+  }
   if (copies > 1) hipLaunchKernelGGL(k_sum_copies, dim3(stride_grid(n)), dim3(256), 0, stream, counts, n, copies);
   return hipGetLastError();
 }

@@ -147,8 +147,21 @@ inline int64_t hot_buffer_bytes(const DevicePlan& p, int K, bool sddmm) {
   return (int64_t)p.nhot * hot_row_stride(K) * 2;
 }
 // Column histogram of col[0, total) into counts[n] (ids outside [0, n) are skipped), counted in
-// `copies` histograms counts[k * n .. (k + 1) * n) (all zeroed by the caller) and summed into the
-// first; and the renumbering hot_col[e] = rank[col[e]] >= 0 ? ~rank[col[e]] : col[e].
+// `copies` histograms counts[k * n .. (k + 1) * n) and summed into the first (all zeroed by the caller,
+// unless counts_in_lds(n): then every counter is written); and the renumbering hot_col[e] = rank[col[e]] >= 0 ? ~rank[col[e]] : col[e].
+// Up to 32 ranges of kCountSpan columns are counted in LDS (128 KB a workgroup); the list is read once a
+// range, so past that many the global atomics, spread over as many columns, cost less (grid of 4M nodes, 128
+// ranges: 23M entries in 293 us with atomics).
+constexpr int32_t kCountSpan = 32768;
+constexpr int kCountRanges = 32;
+inline bool counts_in_lds(int32_t n) { return n <= kCountSpan * kCountRanges; }
+// Copies for a list of `total` entries over n columns counted in LDS: a workgroup to every CU, of at least
+// 8192 entries each.
+inline int lds_count_copies(int64_t total, int32_t n) {
+  const int64_t ranges = (n + kCountSpan - 1) / kCountSpan;
+  const int64_t most = 256 / ranges, fit = total / 8192;
+  return (int)(fit < 1 ? 1 : fit < most ? fit : most);
+}
 hipError_t launch_count_columns(const int32_t* col, int64_t total, int32_t n, int32_t* counts, int copies,
                                 hipStream_t stream);
 hipError_t launch_renumber_hot(const int32_t* col, int64_t total, int32_t n, const int32_t* rank, int32_t* hot_col,

@@ -1421,7 +1421,9 @@ Status stage_hot_rows(trs_plan* P, int64_t total, const trs_plan_options& opt) {
   // far more columns than entries, whose columns are mostly unused anyway
   if (want <= 0 || (int64_t)n > kHotMaxColumnsPerEntry * total) return Status{};
   // histogram copies against atomic contention on hot columns, within kCountCopyBytes
-  const int copies = (int)std::max<int64_t>(1, std::min<int64_t>(kCountCopies, kCountCopyBytes / ((int64_t)n * 4)));
+  const bool in_lds = trs::counts_in_lds(n);
+  const int copies = in_lds ? trs::lds_count_copies(total, n)
+                            : (int)std::max<int64_t>(1, std::min<int64_t>(kCountCopies, kCountCopyBytes / ((int64_t)n * 4)));
   int32_t* counts = nullptr;
   if (hipMalloc(&counts, (size_t)n * 4 * copies) != hipSuccess) {
     (void)hipGetLastError();
@@ -1432,7 +1434,7 @@ Status stage_hot_rows(trs_plan* P, int64_t total, const trs_plan_options& opt) {
     return st;
   };
   std::vector<int32_t> cnt((size_t)n);
-  if (hipMemset(counts, 0, (size_t)n * 4 * copies) != hipSuccess ||
+  if ((!in_lds && hipMemset(counts, 0, (size_t)n * 4 * copies) != hipSuccess) ||
       trs::launch_count_columns(d.col, total, n, counts, copies, nullptr) != hipSuccess ||
       trs::launch_uncount_windows(d.mwin, d.nmwin, d.m, d.rowptr, d.col, n, counts, nullptr) != hipSuccess ||
       hipMemcpy(cnt.data(), counts, (size_t)n * 4, hipMemcpyDeviceToHost) != hipSuccess)
