@@ -1407,7 +1407,10 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     // (K = 32: R-MAT 0.311 -> 0.303 ms, grid+hubs 0.393 -> 0.383; 8-lane groups at K = 64 gain
     // 0.6% on R-MAT and lose 2% on grid+hubs with 16, and keep 8).  With 16-byte loads the two
     // parts then took batches of their own (split_batch): the main part 3 at >= 16 lanes, 8 at 8
-    // lanes and 32 at 4 lanes, the split part 8, 16 and 16
+    // lanes and 32 at 4 lanes, the split part 8, 16 and 16.  8-byte loads in 16-lane groups (K = 33..64)
+    // take 8 in both parts (main / split 4 / 4, 4 / 8, 6 / 8, 8 / 8: R-MAT 2^20 K = 48 410 / 378 / 371
+    // / 372 us, K = 64 418 / 384 / 376 / 376, R-MAT 2^18 K = 52 127 / 117 / 115 / 116, grid of 4M nodes K
+    // = 41 699 / 700 / 717 / 682)
     // pipelined stream for narrow groups with long tasks (same-box A/B: R-MAT K=32/64
     // -9%/-12%; K=128 +8%, grid+hubs K=32 (32-entry tasks, 4 lanes) +6%), and for 8-lane groups
     // whatever the task length (grid+hubs K=64 0.620 -> 0.582 ms, K=8 0.251 -> 0.238)
@@ -1443,7 +1446,7 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     }
 #define TRS_TASKS(L)                                                                                      \
   case L: {                                                                                               \
-    constexpr int U = L >= 16 ? (VEC == 8 ? 3 : 4) : (L == 4 && VEC == 8) ? 32 : 8;                     \
+    constexpr int U = L >= 16 && VEC == 8 ? 3 : (L == 4 && VEC == 8) ? 32 : 8;                          \
     if constexpr (L <= 8) {                                                                               \
       if (pf) { TRS_TASKS_NT(L, U, true, false) } else { TRS_TASKS_NT(L, U, false, false) }               \
     } else if constexpr (L == 16) {                                                                       \
@@ -2140,19 +2143,19 @@ hipError_t launch_spmm(const DevicePlan& p, const uint16_t* B, int64_t ldb, int 
   // (us, narrow -> this): K = 5 310 -> 244, 7 336 -> 262, 13 348 -> 289, 17 580 -> 379, 18 385 ->
   // 312, 28 460 -> 371, 31 643 -> 458, 65 1755 -> 643, 97 2198 -> 724, 100 942 -> 644, 127 2425 -> 814,
   // 130 2122 -> 1333, 255 4436 -> 1618; SBM 250K nodes K = 17 76 -> 43, 65 169 -> 95, 127 240 -> 132.
-  // K = 33..64 off the 16-byte grid keep 8-byte loads in 16-lane groups, whose staged stream holds
-  // more entries in flight than 8-lane groups held to 2 waves: K = 33 595 (16-byte) / 454, 41 622 /
-  // 464, 52 568 / 442, 63 696 / 518 (2-byte loads before: 992, 1013, 440 with 8 bytes, 1130); grid of
-  // 4M nodes with hubs K = 41 760 / 700.  On the 16-byte grid they do so where the call's operands are
-  // well beyond the 256 MB MALL, where the gathers wait on HBM (R-MAT 2^20 with 31M entries K = 40 / 48
-  // / 56 / 64 505 / 507 / 564 / 459 -> 410 / 410 / 438 / 419 us, grid of 4M nodes K = 40 / 56 / 64 622 /
-  // 753 / 588 -> 606 / 735 / 572), and not below (grid of 640K nodes K = 48 / 64 74 / 71 -> 83 / 83,
-  // R-MAT 2^18 K = 64 112 -> 122).
+  // K = 33..64 take 8-byte loads in 16-lane groups, whose staged stream holds more entries in flight than
+  // 8-lane groups of 16-byte loads held to 2 waves (us, 16-byte / 8-byte, in batches of 8): R-MAT 2^20 K =
+  // 33 595 / 442, 41 622 / 453, 48 507 / 372, 64 457 / 376; R-MAT 2^18 K = 40 / 48 / 56 / 64 120 / 120 / 127 / 112,
+  // 110 / 110 / 115 / 109; R-MAT 2^14 K = 64 20.4 / 18.7; ER of 274K nodes K = 40 69.8 / 66.5; grid of 4M nodes
+  // with hubs K = 64 587 / 564.  On the 16-byte grid the 16-byte loads stay where pieces of a few hub rows are
+  // far longer than the packed tasks of a mesh and the operands fit the MALL: grid of 640K nodes (tasks of
+  // 32, pieces of 128) K = 40 / 48 / 64 73 / 74 / 71, 79 / 85 / 85; with 2M nodes, past it, both the same.
   // K = 5 and 7 stay on 8 lanes of 2 bytes over short rows (grid of 2M nodes K = 7: 109 us, 127 with 4-byte
   // loads; R-MAT, whose tasks are long, 336 / 262)
   const bool aligned = K % 8 == 0 && ldb % 8 == 0 && aligned16(B);
   const int64_t touched = p.nnz_csr * 6 + (int64_t)p.m * K * 4 + (int64_t)p.n * K * 2;
-  const bool v8 = K > 16 && (K <= 32 || K > 64 || (aligned && touched < kBeyondMall)), v4 = K > 8,
+  const bool hub_pieces = p.task_max > 3 * p.task_nnz && touched < kBeyondMall;
+  const bool v8 = K > 16 && (K <= 32 || K > 64 || (aligned && hub_pieces)), v4 = K > 8,
              v2 = K > 4 && (K % 2 == 0 || K > 8 || p.task_nnz >= 64);
   // (the staged hot rows need 16-byte aligned rows in the buffer too)
   if (hot != nullptr && !aligned16(hot)) hot = nullptr;
