@@ -99,6 +99,14 @@ def launched(kms, runs):
     return [v if r else None for v, r in zip(kms, runs)]
 
 
+def staged_row_bytes(K: int, sddmm: bool) -> int:
+    """Bytes of one staged hot row at width K, 0 where the width does not stage (widths that 8 does not
+    divide stage padded to whole cache lines)."""
+    if K % 8 == 0:
+        return 2 * K if K >= 128 else 0
+    return 2 * ((K + 63) // 64 * 64) if K >= (121 if sddmm else 65 if K % 2 else 104) else 0
+
+
 def dominant(kms) -> int:
     return max((i for i, v in enumerate(kms) if v is not None), key=lambda i: kms[i])
 
@@ -299,7 +307,7 @@ def bench_sddmm(args, workload, g, K):
         nr = st["csr_nnz"]
         bytes_k = 8 * nr + 4 * (M + 1) + 2 * M * K + 2 * N * K
         impl = (4 * nr if st["mfma_tiles"] else 0) + 16 * st["tasks"]   # output index, task descriptors
-        hot_bytes = 2 * K * st["hot_rows"] if need and K >= 128 and K % 8 == 0 else 0
+        hot_bytes = staged_row_bytes(K, True) * st["hot_rows"] if need else 0
         impl += 2 * hot_bytes                                           # staged hot rows: read + write
         impl += 3 * max(0, need - hot_bytes)                            # split-part merge: index, buffer, output (4 B each)
     else:
@@ -467,7 +475,7 @@ def main():
         rows_k = M - rows_w
         bytes_k = 6 * nnz_k + 4 * (rows_k + 1) + 2 * N * K + 4 * rows_k * K
         impl = 16 * st["tasks"] + 4 * K * st["partial_slots"]          # task descriptors, partial slots
-        impl += 4 * K * st["hot_rows"] if K >= 128 and K % 8 == 0 else 0  # staged hot rows: read + write
+        impl += 2 * staged_row_bytes(K, False) * st["hot_rows"]           # staged hot rows: read + write
     elif dom == 1:  # MFMA windows: tile entries + the windows' residual entries, their rows
         bytes_k = 6 * (st["mfma_nnz"] + nnz_w) + 4 * (rows_w + 1) + 2 * N * K + 4 * rows_w * K
         impl = st["mfma_tiles"] * (512 + 64) - 6 * st["mfma_nnz"]      # dense 16x16 tiles + column ids

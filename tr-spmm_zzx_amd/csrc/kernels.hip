@@ -2141,7 +2141,7 @@ hipError_t launch_spmm(const DevicePlan& p, const uint16_t* B, int64_t ldb, int 
   // lanes of 4 bytes: 0.545 -> 0.273; K = 4 as 4 lanes of 2 bytes: 0.233 -> 0.219).  With narrower
   // loads for the widths that 8, 4 or 2 do not divide, and 2-byte ones for odd ones, R-MAT 2^20 took
   // (us, narrow -> this): K = 5 310 -> 244, 7 336 -> 262, 13 348 -> 289, 17 580 -> 379, 18 385 ->
-  // 312, 28 460 -> 371, 31 643 -> 458, 65 1755 -> 643, 97 2198 -> 724, 100 942 -> 644, 127 2425 -> 814,
+  // 312, 28 460 -> 371, 31 643 -> 458, 65 1755 -> 643, 97 2198 -> 724, 100 942 -> 661, 127 2425 -> 814,
   // 130 2122 -> 1333, 255 4436 -> 1618; SBM 250K nodes K = 17 76 -> 43, 65 169 -> 95, 127 240 -> 132.
   // K = 33..64 take 8-byte loads in 16-lane groups, whose staged stream holds more entries in flight than
   // 8-lane groups of 16-byte loads held to 2 waves (us, 16-byte / 8-byte, in batches of 8): R-MAT 2^20 K =
