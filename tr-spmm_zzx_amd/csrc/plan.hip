@@ -73,9 +73,10 @@ constexpr int kLowerOnHost = -100;
 // Below kSplitSmall entries the SpMM splits from 512 entries on: a shorter row's eight sub-rows are then
 // a task and a slot each with a few tens of entries (R-MAT 2^16, K = 32 / 64 / 128: 256 entries 35.1 /
 // 46.6 / 58.9 us, 512 31.8 / 40.6 / 57.1, no split 36.2 / 44.6 / 59.8; R-MAT 2^14 20.8 / 22.8 / 28.6,
-// 19.3 / 20.1 / 26.2, 20.0 / 23.2 / 26.8; R-MAT 2^18, 7.9M entries: the same within 1%).
+// 19.3 / 20.1 / 26.2, 20.0 / 23.2 / 26.8; R-MAT 2^18, 7.9M entries: the same within 1%; with 3.9M
+// entries the 256 are better: K = 80 90 / 100).  Tasks shrink below the same line (build_tasks).
 constexpr int32_t kSpmmSplitMin = 256;
-constexpr int64_t kSplitSmall = 1 << 22;
+constexpr int64_t kSplitSmall = 3 << 20;
 constexpr int32_t kSddmmSplitMin = 512;
 // ... and only when those rows' entries are at least this many times their distinct columns:
 // R-MAT's rows of >= 256 entries gather 20.0M times from 0.60M columns (33x), the 64 hubs of the
@@ -809,7 +810,7 @@ Tasks build_tasks(const Placement& P, const std::vector<int32_t>& rowptr, int32_
   // entries K = 64 / 128 / 200: tasks of 32 25.2 / 41.9 / 82.5, 64 26.6 / 36.1 / 78.4), those of narrower
   // groups, which walk a list of their own, do not (K = 32: 21 with 32, 28 with 60).
   int S_narrow = S;
-  if (opt.task_nnz <= 0) {
+  if (opt.task_nnz <= 0 && nent < kSplitSmall) {   // (R-MAT 2^18 with 3.9M entries K = 16: 60 entries 64 us, 128 57)
     const bool tiny = nent < kTinyEntries;
     S_narrow = (int)std::min<int64_t>(S, std::max<int64_t>(tiny ? 16 : 32, nent / kMinTasks));
     S = with_fixup || tiny ? S_narrow : (int)std::min<int64_t>(S, std::max<int64_t>(64, nent / kMinTasks));
