@@ -12,10 +12,13 @@ import trspmm
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("K", [130, 136, 160, 192, 193, 264])
-def test_narrow_last_pass_adds_to_the_merged_outputs(K):
-    print("sddmm narrow last pass", K, flush=True)
-    g = graphs.rmat(scale=13, edge_factor=16, seed=9)
+# 2^13 columns: one pass of 32 lanes to K = 256, passes of 128 above.  2^16 and 2^18 columns: Y beyond the
+# size to which one pass is taken (odd widths 16 MB, even ones 64 MB), so passes of 128 from K = 129 on.
+@pytest.mark.parametrize("K, scale", [(130, 13), (136, 13), (160, 13), (192, 13), (193, 13), (256, 13), (257, 13),
+                                      (264, 13), (145, 16), (129, 16), (130, 18)])
+def test_narrow_last_pass_adds_to_the_merged_outputs(K, scale):
+    print("sddmm narrow last pass", K, scale, flush=True)
+    g = graphs.rmat(scale=scale, edge_factor=16 if scale == 13 else 1, seed=9)
     f = trspmm.build_format(g.rowptr, g.col, g.val)
     plan = trspmm.Plan.for_sddmm(f, g.m, g.n, mfma_tc=False, mfma_sptc=False, xcd_split=64, task_nnz=16)
     assert plan.stats()["split_rows"] > 0 and plan.sddmm_workspace_bytes(K) > 0
