@@ -1,0 +1,34 @@
+"""GPU format builder: windows at the edges of its routing rule (1024, 2048 and 8192 distinct columns; 9/8
+entries a column), bit for bit against the host builder."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import same_array
+import trspmm
+
+pytestmark = pytest.mark.gpu
+
+
+def _window(U, extra, rng, n):
+    """16 rows over U distinct columns of n: two rows share them out, a third repeats `extra` of them."""
+    cols = np.sort(rng.choice(n, size=U, replace=False))
+    first = rng.random(U) < 0.5
+    return [cols[first], cols[~first], np.sort(rng.choice(cols, size=extra, replace=False))] + [cols[:0]] * 13
+
+
+@pytest.mark.parametrize("U", [1024, 1025, 2048, 2049, 3001, 8192, 8193])
+def test_windows_at_the_routing_edges(U):
+    rng = np.random.default_rng(U)
+    n = 20000
+    rows = []
+    for extra in (0, (U - 1) // 8, U // 8 + 1, U):   # below, just below, just above 9/8 entries a column; 2
+        print("window of", U, "columns", U + extra, "entries", flush=True)
+        rows += _window(U, extra, rng, n)
+    rowptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    col = np.concatenate(rows).astype(np.int32)
+    val = rng.integers(1, 16, size=len(col)).astype(np.float32)
+    hf = trspmm.build_format(rowptr, col, val)
+    f = trspmm.build_format_device(*(torch.from_numpy(a).cuda() for a in (rowptr, col, val))).download()
+    bad = [trspmm.ops.SLOT_NAMES[i] for i in range(32) if not same_array(f.slot(i), hf.slot(i))]
+    assert not bad, bad

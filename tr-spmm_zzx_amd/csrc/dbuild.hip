@@ -22,8 +22,8 @@
 // Stages (one pass each over device arrays, prefix sums between them):
 //   A  every entry's position in its window sorted by (column, local row): ranks from binary
 //      searches in the window's other rows, no sort; distinct columns with 16-bit row masks;
-//   B  per window (a wave for windows of <= kSmallU distinct columns, a workgroup of 16 waves
-//      otherwise): TC chunks, units, the introsort, the greedy matching, groups;
+//   B  per window (a wave, or a workgroup of 8 waves for wide ones: wave_window; the same results
+//      either way): TC chunks, units, the introsort, the greedy matching, groups;
 //   C  counts per window and per row, prefix sums;
 //   D  the format arrays.
 #include <hip/hip_runtime.h>
@@ -45,7 +45,8 @@ namespace {
 
 using u64 = unsigned long long;
 
-constexpr int kSmallU = 2048;       // windows with more distinct columns take the workgroup kernel
+constexpr int kSmallU = 8192;       // windows with more distinct columns take the workgroup kernel
+constexpr int kMidU = 2048;         // ... and those with more than this many that share them (wave_window)
 constexpr int kNarrowU = 1024;      // windows of at most this many, the narrow launch of the wave kernel
 constexpr int kBlockWaves = 8;      // waves of that kernel
 constexpr int kLdsUnits = 65536;    // most units whose order it keeps in LDS (16-bit indices; the
@@ -917,14 +918,27 @@ __device__ void plan_window(const Build& B, int32_t w, P* perm, uint32_t* taken,
   }
 }
 
+// Whether window w of U distinct columns is routed by one wave.  Past kMidU columns a workgroup sorts
+// the units of a window faster where rows share columns, 1.22 to 2.8 entries a column (format, plan and
+// product, wave / workgroup: R-MAT 2^13 2546 / 2247 us, 2^14 3419 / 2948, 2^16 5441 / 4842, 2^17 6860 / 6308), and
+// slower where nearly every column holds one entry and nearly all units tie (grid of 223^2 nodes, two hub
+// rows in a window: 1729 / 2296).  The line is at 9/8 entries a column.
+__device__ __forceinline__ bool wave_window(const Build& B, int32_t w, int32_t U) {
+  if (U <= kMidU || U > kSmallU) return U <= kMidU;
+  const int64_t r0 = (int64_t)w * B.ws;
+  const int64_t r1 = r0 + B.ws < B.rows ? r0 + B.ws : B.rows;
+  return (int64_t)(B.rowptr[r1] - B.rowptr[r0]) * 8 < (int64_t)U * 9;
+}
+
 // Windows of (LO, CAP] distinct columns, CAP <= kSmallU, one wave each (workgroups of one wave); matched
 // pairs go to the window's part of B.pairs.  The LDS is sized by CAP, so that the many narrow windows
-// run 32 to a CU, not the 8 that kSmallU leaves room for (R-MAT 2^18: 1200 us in one launch -> 325 in two).
+// run 32 to a CU, not the 8 that kSmallU leaves room for (R-MAT 2^18: 1200 us in one launch -> 325 in two,
+// the windows past kMidU routed by workgroups).
 template <int LO, int CAP>
 __global__ __launch_bounds__(64) void k_plan_small(Build B) {
   const int32_t w = blockIdx.x;
   const int32_t ub = B.ubase[w], U = B.ubase[w + 1] - ub;
-  if ((LO > 0 && U <= LO) || U > CAP) return;
+  if ((LO > 0 && U <= LO) || U > CAP || (CAP > kMidU && !wave_window(B, w, U))) return;
   __shared__ uint16_t perm[CAP / 2 + 1];
   __shared__ uint8_t unnz[CAP / 2 + 1];
   __shared__ uint8_t leaf[CAP / 2 + 1];
@@ -980,7 +994,7 @@ __global__ __launch_bounds__(256) void k_list_large(Build B, int32_t* big, int32
   const int32_t w = (int32_t)(blockIdx.x * 256 + threadIdx.x);
   if (w >= B.nwin) return;
   const int32_t U = B.ubase[w + 1] - B.ubase[w];
-  if (U <= kSmallU) return;
+  if (wave_window(B, w, U)) return;
   const int32_t i = atomicAdd(nbig, 1);
   big[2 * i] = U;
   big[2 * i + 1] = w;
@@ -1516,7 +1530,8 @@ int trs_build_online_device(const int32_t* rowptr, const int32_t* col, const flo
     return fail(TRS_EDEVICE, "hipMemsetAsync failed");
   if (W > 0) {
     hipLaunchKernelGGL(k_list_large, dim3(grid_of(W)), dim3(256), 0, s, B, big, nbig_d);
-    hipLaunchKernelGGL((k_plan_small<kNarrowU, kSmallU>), dim3(W), dim3(64), 0, s, B);
+    hipLaunchKernelGGL((k_plan_small<kMidU, kSmallU>), dim3(W), dim3(64), 0, s, B);
+    hipLaunchKernelGGL((k_plan_small<kNarrowU, kMidU>), dim3(W), dim3(64), 0, s, B);
     hipLaunchKernelGGL((k_plan_small<0, kNarrowU>), dim3(W), dim3(64), 0, s, B);
     int32_t nbig = 0;
     if (hipMemcpyAsync(&nbig, nbig_d, 4, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
