@@ -728,6 +728,7 @@ struct Tasks {
 // Residual tasks and pieces of long rows a plan aims at when the automatic sizes leave fewer (see
 // build_tasks).
 constexpr int64_t kMinTasks = 65536;
+constexpr int64_t kMinTasksEven = 16384;
 constexpr int64_t kMinPieces = 32768;
 constexpr int64_t kTinyEntries = 3 << 18;
 // Rows per chunk of the main part's task packing (a multiple of 16: MFMA windows stay whole).
@@ -809,10 +810,18 @@ Tasks build_tasks(const Placement& P, const std::vector<int32_t>& rowptr, int32_
   // SDDMM tasks of 16-lane groups hold twice that (no row is written per task; R-MAT 2^16 with 983K
   // entries K = 64 / 128 / 200: tasks of 32 25.2 / 41.9 / 82.5, 64 26.6 / 36.1 / 78.4), those of narrower
   // groups, which walk a list of their own, do not (K = 32: 21 with 32, 28 with 60).
+  // An SpMM no row of which fills a task has no long chain to shorten: from kTinyEntries on its tasks shrink
+  // only to kMinTasksEven of them (ER of 60,000 nodes, 17 entries a row, K = 32 / 64 / 128 / 256, tasks of 48:
+  // 18.3 / 22.5 / 39.8 / 71.8 us, of 62: 20.7 / 26.1 / 35.6 / 68.9, of 32 at K = 128 39.1; ER of 100,000 nodes
+  // K = 16, of 48 25.4, of 68 21.3).
+  int32_t longest = 0;
+  for (int32_t q = 0; q < m; ++q) longest = std::max(longest, rowptr[q + 1] - rowptr[q]);
   int S_narrow = S;
   if (opt.task_nnz <= 0 && nent < kSplitSmall) {   // (R-MAT 2^18 with 3.9M entries K = 16: 60 entries 64 us, 128 57)
     const bool tiny = nent < kTinyEntries;
     S_narrow = (int)std::min<int64_t>(S, std::max<int64_t>(tiny ? 16 : 32, nent / kMinTasks));
+    if (with_fixup && !tiny && longest <= S)
+      S_narrow = (int)std::min<int64_t>(S, std::max<int64_t>(32, nent / kMinTasksEven));
     S = with_fixup || tiny ? S_narrow : (int)std::min<int64_t>(S, std::max<int64_t>(64, nent / kMinTasks));
   }
   T.task_nnz = S;
@@ -822,8 +831,6 @@ Tasks build_tasks(const Placement& P, const std::vector<int32_t>& rowptr, int32_
   // ... but a longest row of at most two pieces stays whole: the chain it saves is shorter than the
   // fixup launch that cutting it asks for (ER of 4096 nodes, 17 entries a row, longest 40: 9.7 us with no
   // row cut, 13.2 with a few)
-  int32_t longest = 0;
-  for (int32_t q = 0; q < m; ++q) longest = std::max(longest, rowptr[q + 1] - rowptr[q]);
   while (piece_auto < 256 && longest <= 2 * piece_auto) piece_auto *= 2;
   const int piece_max = std::max(S, opt.piece_nnz > 0 ? opt.piece_nnz : piece_auto);
   const int rows_cap = trs::kTaskRows;
