@@ -34,7 +34,8 @@ def inside(rows, K, off, pad, seed):
 
 # edges of every load width (2 | 4 | 8 | 16 bytes), of the 4-, 8- and 16-lane groups, of the widths that
 # stage hot rows, and of a second feature pass
-WIDTHS = [4, 5, 7, 8, 9, 13, 16, 17, 23, 31, 33, 40, 47, 63, 65, 96, 103, 104, 106, 119, 121, 127, 129, 130, 135, 255]
+WIDTHS = [4, 5, 7, 8, 9, 13, 16, 17, 23, 31, 33, 40, 47, 63, 65, 72, 96, 103, 104, 106, 119, 121, 127, 129, 130, 135, 136,
+          200, 255]
 
 
 @pytest.mark.parametrize("K", WIDTHS)
@@ -65,10 +66,10 @@ def test_sddmm_any_width_and_alignment(K, off, pad):
         plan = trspmm.Plan.for_sddmm(f, g.m, g.n, **opts)
         X, Xh = inside(g.m, K, off, pad, seed=K)
         Y, Yh = inside(g.n, K, off + 1, pad, seed=K + 1)
-        # an Inf in one X row and one Y row: only their own entries are not finite.  (In Y behind the first
-        # vector: lanes past K multiply zeros with that one, which makes 0 x Inf there.)
+        # an Inf in one X row and one Y row: only their own entries are not finite, and they are +-Inf.  (In Y
+        # among the features that lanes past K read, to no effect.)
         X[5, K - 1] = float("inf")
-        Y[9, K - 8 if K >= 16 else K - 1] = float("inf")
+        Y[9, 0] = float("inf")
         Xh, Yh = X.cpu().numpy(), Y.cpu().numpy()
         S = plan.sddmm(X, Y)
         torch.cuda.synchronize()

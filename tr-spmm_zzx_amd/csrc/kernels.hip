@@ -1063,8 +1063,9 @@ __device__ __forceinline__ void sddmm_tasks_run(const DevicePlan& P, int block, 
       const int w = RAG ? row_window<VEC>(f < K ? f : 0, K) : f < K ? f : 0;
       const OwnElements<VEC> own(f < K ? f - w : VEC);
       // all Y gathers first, unconditional so they issue back to back (lanes past K read features
-      // [0, VEC) and padded slots repeat the last entry; both are discarded), then one X fetch per
-      // distinct row of the chunk; the fragment each entry uses is selected in registers
+      // [0, VEC) and padded slots repeat the last entry; both are discarded, the former by leaving out
+      // their sums: an Inf among those features would make 0 x Inf of a zero X fragment), then one X
+      // fetch per distinct row of the chunk; the fragment each entry uses is selected in registers
       BFrag<VEC> x[U], y[U];
       const uint16_t* __restrict__ Yf = Y + w;
       const uint16_t* __restrict__ Hf = HOT ? P.hot_b + w : nullptr;
@@ -1100,7 +1101,8 @@ __device__ __forceinline__ void sddmm_tasks_run(const DevicePlan& P, int block, 
 #pragma unroll
       for (int i = 0; i < U; ++i) {
         if (i > 0 && rr[i] != rr[i - 1]) xe = x[i];
-        s[i] += xe.dot(y[i]);
+        const float d = xe.dot(y[i]);
+        s[i] += RAG || f < K ? d : 0.f;   // (RAG: both operands are zero there)
       }
       if (carry) {
         xc = xe;
