@@ -357,3 +357,18 @@ def test_hot_selection_equals_brute_force(name, gen, want):
     rows, entries = _brute_force_hot(g.col[:nnz], g.n, w)
     say("hot selection", name, s["hot_rows"], s["hot_entries"], rows, entries)
     assert (s["hot_rows"], s["hot_entries"]) == (rows, entries)
+
+
+@pytest.mark.parametrize("n", [32767, 32768, 32769, 65537, 1 << 20, (1 << 20) + 1])
+def test_hot_selection_at_the_edges_of_the_column_ranges(n):
+    """The counts are taken range by range of 32,768 columns in LDS, past 2^20 columns with global atomics."""
+    rng = np.random.default_rng(n)
+    m, per = 2048, 160
+    cols = np.concatenate([rng.integers(0, n, (m, per - 8)), n - 1 - rng.integers(0, 40, (m, 4)), rng.integers(0, 40, (m, 4))], 1)
+    rows = [np.unique(c) for c in cols]
+    rowptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    col = np.concatenate(rows).astype(np.int32)
+    f = trspmm.build_format(rowptr, col, np.ones(len(col), np.float32))
+    say("hot selection over", n, "columns")
+    s = trspmm.Plan.from_format(f, m, n, mfma_tc=False, mfma_sptc=False, xcd_split=-1, hot_rows=100).stats()
+    assert (s["hot_rows"], s["hot_entries"]) == _brute_force_hot(col, n, 100)

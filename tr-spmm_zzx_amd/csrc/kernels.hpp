@@ -156,11 +156,19 @@ constexpr int32_t kCountSpan = 32768;
 constexpr int kCountRanges = 32;
 inline bool counts_in_lds(int32_t n) { return n <= kCountSpan * kCountRanges; }
 // Copies for a list of `total` entries over n columns counted in LDS: a workgroup to every CU, of at least
-// 8192 entries each.
+// 8192 entries each, within a buffer of 2 MB, or of 8 copies where that is more (16 past 2^16 columns).  The
+// kernel alone would take more copies, but the buffer lives for one plan, and what it costs to get and to give
+// back more than that is not won back (us per plan, 73 / 8 copies: ER of 60,000 nodes 1340 / 1016; 120 / 9,
+// grid of 223^2 nodes with hubs 1096 / 782, and 280 of the next format build; 128 / 8, R-MAT 2^16 2430 / 2133;
+// 32 / 16 / 8, ER of 250,000 nodes 2305 / 2331 / 2657).
 inline int lds_count_copies(int64_t total, int32_t n) {
   const int64_t ranges = (n + kCountSpan - 1) / kCountSpan;
-  const int64_t most = 256 / ranges, fit = total / 8192;
-  return (int)(fit < 1 ? 1 : fit < most ? fit : most);
+  const int64_t held = (int64_t)(2 << 20) / ((int64_t)n * 4), least = n > 1 << 16 ? 16 : 8;
+  int64_t copies = held > least ? held : least;
+  if (copies > 256 / ranges) copies = 256 / ranges;
+  const int64_t fit = total / 8192;
+  if (copies > fit) copies = fit;
+  return (int)(copies < 1 ? 1 : copies);
 }
 hipError_t launch_count_columns(const int32_t* col, int64_t total, int32_t n, int32_t* counts, int copies,
                                 hipStream_t stream);
