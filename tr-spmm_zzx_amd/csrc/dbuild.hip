@@ -48,6 +48,7 @@ using u64 = unsigned long long;
 constexpr int kSmallU = 8192;       // windows with more distinct columns take the workgroup kernel
 constexpr int kMidU = 2048;         // ... and those with more than this many that share them (wave_window)
 constexpr int kNarrowU = 1024;      // windows of at most this many, the narrow launch of the wave kernel
+constexpr int kFewWide = 1024;      // at most this many wider ones share one launch of the wave kernel
 constexpr int kBlockWaves = 8;      // waves of that kernel
 constexpr int kLdsUnits = 65536;    // most units whose order it keeps in LDS (16-bit indices; the
                                     // device's LDS per workgroup may allow fewer)
@@ -933,12 +934,20 @@ __device__ __forceinline__ bool wave_window(const Build& B, int32_t w, int32_t U
 // Windows of (LO, CAP] distinct columns, CAP <= kSmallU, one wave each (workgroups of one wave); matched
 // pairs go to the window's part of B.pairs.  The LDS is sized by CAP, so that the many narrow windows
 // run 32 to a CU, not the 8 that kSmallU leaves room for (R-MAT 2^18: 1200 us in one launch -> 325 in two,
-// the windows past kMidU routed by workgroups).
+// the windows past kMidU routed by workgroups).  One launch waits for the longest window of the one before,
+// so where the windows past kNarrowU are few (kFewWide; *wide of them) the widest launch takes them all: the chip
+// holds 1792 of its workgroups at once (grid of 223^2 nodes, 64 windows of a hub row: 255 us in three launches, 161
+// in two, 136 in the one of all windows).
 template <int LO, int CAP>
-__global__ __launch_bounds__(64) void k_plan_small(Build B) {
+__global__ __launch_bounds__(64) void k_plan_small(Build B, const int32_t* __restrict__ wide) {
   const int32_t w = blockIdx.x;
   const int32_t ub = B.ubase[w], U = B.ubase[w + 1] - ub;
-  if ((LO > 0 && U <= LO) || U > CAP || (CAP > kMidU && !wave_window(B, w, U))) return;
+  if (U > CAP || (LO == 0 ? false : CAP > kMidU ? U <= kNarrowU : U <= LO)) return;
+  if constexpr (CAP > kMidU) {
+    if (!wave_window(B, w, U) || (U <= LO && *wide > kFewWide)) return;
+  } else if constexpr (LO > 0) {
+    if (*wide <= kFewWide) return;
+  }
   __shared__ uint16_t perm[CAP / 2 + 1];
   __shared__ uint8_t unnz[CAP / 2 + 1];
   __shared__ uint8_t leaf[CAP / 2 + 1];
@@ -989,12 +998,16 @@ __global__ __launch_bounds__(kBlockWaves * 64) void k_plan_huge(Build B, const i
 }
 
 // Windows for the workgroup kernels: (distinct columns, window) of each, big[0, nbig) (the host
-// orders them, largest first, and splits them between the two kernels).
+// orders them, largest first, and splits them between the two kernels).  nbig[1] counts the windows
+// past kNarrowU of the wave kernel.
 __global__ __launch_bounds__(256) void k_list_large(Build B, int32_t* big, int32_t* nbig) {
   const int32_t w = (int32_t)(blockIdx.x * 256 + threadIdx.x);
   if (w >= B.nwin) return;
   const int32_t U = B.ubase[w + 1] - B.ubase[w];
-  if (wave_window(B, w, U)) return;
+  if (wave_window(B, w, U)) {
+    if (U > kNarrowU) atomicAdd(nbig + 1, 1);
+    return;
+  }
   const int32_t i = atomicAdd(nbig, 1);
   big[2 * i] = U;
   big[2 * i + 1] = w;
@@ -1530,9 +1543,9 @@ int trs_build_online_device(const int32_t* rowptr, const int32_t* col, const flo
     return fail(TRS_EDEVICE, "hipMemsetAsync failed");
   if (W > 0) {
     hipLaunchKernelGGL(k_list_large, dim3(grid_of(W)), dim3(256), 0, s, B, big, nbig_d);
-    hipLaunchKernelGGL((k_plan_small<kMidU, kSmallU>), dim3(W), dim3(64), 0, s, B);
-    hipLaunchKernelGGL((k_plan_small<kNarrowU, kMidU>), dim3(W), dim3(64), 0, s, B);
-    hipLaunchKernelGGL((k_plan_small<0, kNarrowU>), dim3(W), dim3(64), 0, s, B);
+    hipLaunchKernelGGL((k_plan_small<kMidU, kSmallU>), dim3(W), dim3(64), 0, s, B, nbig_d + 1);
+    hipLaunchKernelGGL((k_plan_small<kNarrowU, kMidU>), dim3(W), dim3(64), 0, s, B, nbig_d + 1);
+    hipLaunchKernelGGL((k_plan_small<0, kNarrowU>), dim3(W), dim3(64), 0, s, B, nbig_d + 1);
     int32_t nbig = 0;
     if (hipMemcpyAsync(&nbig, nbig_d, 4, hipMemcpyDeviceToHost, s) != hipSuccess || hipStreamSynchronize(s) != hipSuccess)
       return fail(TRS_EDEVICE, std::string("trs_build_online_device: ") + hipGetErrorString(hipGetLastError()));
