@@ -19,6 +19,7 @@ def rules(tmp_path_factory):
                            "-I", INC, SRC, "-o", so])
     lib = ctypes.CDLL(so)
     lib.rule_lds_count_copies.argtypes = [ctypes.c_int64, ctypes.c_int32]
+    lib.rule_task_sizes.argtypes = [ctypes.c_int64, ctypes.c_int64] + [ctypes.c_int32] * 5 + [ctypes.c_void_p]
     return lib
 
 
@@ -31,3 +32,62 @@ def test_column_count_copies_stay_in_a_small_buffer(rules, total, n):
     # a buffer of 2 MB, or of 8 copies (16 past 2^16 columns)
     assert c * n * 4 <= max(2 << 20, (8 if n <= 1 << 16 else 16) * n * 4)
     assert rules.rule_counts_in_lds(n) == 1 and rules.rule_counts_in_lds((1 << 20) + 1) == 0
+
+
+def sizes(rules, entries, nonempty, longest, spmm, split=False, task=0, piece=0):
+    out = (ctypes.c_int32 * 7)()
+    rules.rule_task_sizes(entries, nonempty, longest, int(spmm), int(split), task, piece, out)
+    return dict(zip(("task", "narrow", "piece", "full_task", "full_piece", "row_task", "even"), out))
+
+
+TINY, SMALL = 3 << 18, 3 << 20
+
+
+@pytest.mark.parametrize("spmm", [True, False])
+def test_task_sizes_of_even_rows(rules, spmm):
+    """Rows no longer than a packed task: 16,384 tasks below 786,432 entries, and no row is cut."""
+    for entries, rows, longest in ((278_000, 16384, 42), (483_463, 28439, 40), (552_000, 42440, 32), (740_053, 52861, 36)):
+        z = sizes(rules, entries, rows, longest, spmm)
+        want = min(z["row_task"], max(16, entries // 16384 if spmm else entries // 16384 // 4 * 4))
+        assert z["even"] and z["task"] == want and z["piece"] >= longest, (entries, z)
+        assert z["narrow"] == (want if spmm else 16 if want < 24 else 24), (entries, z)
+    for entries, rows in ((TINY, 46000), (1_020_000, 60000), (SMALL - 1, 180_000)):
+        z = sizes(rules, entries, rows, 40, spmm)
+        assert z["task"] == (min(z["row_task"], max(32, entries // 16384)) if spmm else 64), (entries, z)
+    assert sizes(rules, SMALL, 180_000, 40, spmm)["task"] == 4 * SMALL // 180_000
+
+
+def test_task_and_piece_sizes_of_uneven_rows(rules):
+    # SpMM: tasks of 16 and pieces of 32 (tiny), 32 and 64 (small)
+    z = sizes(rules, TINY - 1, 40_000, 4000, True, split=True)
+    assert not z["even"] and (z["task"], z["piece"]) == (16, 32)
+    z = sizes(rules, TINY, 40_000, 4000, True, split=True)
+    assert (z["task"], z["piece"]) == (32, 64)
+    assert sizes(rules, SMALL - 1, 90_000, 4000, True, split=True)["task"] == 47
+    # SDDMM: 16-lane groups take 16,384 tasks (tiny) or tasks of 64, pieces of 64 from 393,216 entries on
+    z = sizes(rules, 491_520, 12_000, 4000, False, split=True)
+    assert (z["task"], z["narrow"], z["piece"], z["full_task"], z["full_piece"]) == (16, 16, 32, 28, 64)
+    z = sizes(rules, 491_520, 12_000, 4000, False)
+    assert (z["task"], z["piece"]) == (28, 64)
+    z = sizes(rules, (3 << 17) - 1, 12_000, 4000, False)
+    assert (z["piece"], z["full_piece"]) == (32, 32)
+    z = sizes(rules, 983_040, 40_000, 4000, False, split=True)
+    assert (z["task"], z["narrow"], z["piece"], z["full_piece"]) == (64, 32, 64, 128)
+    # past 3,145,728 entries: pieces of 128 of short rows up to 5M entries (6,291,456 with split rows), else 256
+    for entries, mean, split, want in ((3_194_880, 36, True, 256), (3_932_160, 26, True, 256), (4_915_200, 19.8, True, 128),
+                                       (5_898_240, 14.7, True, 128), (5_898_240, 22.5, True, 256), (6 << 20, 15, True, 256),
+                                       (4_990_000, 5.5, False, 128), (5_000_000, 5.5, False, 256)):
+        z = sizes(rules, entries, int(entries / mean), 20_000, True, split=split)
+        assert z["piece"] == want and z["task"] == z["row_task"], (entries, mean, z)
+    assert sizes(rules, 3_194_880, 87_000, 14_000, False, split=True)["piece"] == 128
+    # a longest row of at most two pieces stays whole
+    assert sizes(rules, 200_000, 40_000, 64, True)["piece"] >= 64
+    assert sizes(rules, 200_000, 40_000, 65, True)["piece"] == 32
+
+
+def test_asked_sizes_are_taken(rules):
+    for spmm in (True, False):
+        z = sizes(rules, 500_000, 20_000, 4000, spmm, task=24, piece=100)
+        assert (z["task"], z["narrow"], z["piece"], z["full_piece"]) == (24, 24, 100, 100)
+        z = sizes(rules, 2_000_000, 40_000, 4000, spmm, task=512)
+        assert (z["task"], z["piece"]) == (512, 512) and z["full_piece"] >= 512

@@ -119,6 +119,92 @@ struct DevicePlan {
   int32_t out_off = 0;   // set in the view that writes xbuf: entry q writes out[q - out_off]
 };
 
+// Sizes of residual tasks and pieces.
+// A plan of fewer entries than this is small: it splits rows over the XCDs from 512 entries on, not 256, and its
+// tasks and pieces shrink (see task_sizes).
+constexpr int64_t kSmallEntries = 3 << 20;
+// ... and of fewer than this, tiny.
+constexpr int64_t kTinyEntries = 3 << 18;
+// Tasks that tiny and even plans aim at, and the uneven small ones of SpMM.
+constexpr int64_t kMinTasks = 16384;
+constexpr int64_t kMinTasksUneven = 65536;
+
+struct TaskSizes {
+  int32_t task = 0;     // entries per task of packed rows
+  int32_t narrow = 0;   // the same in the list of SDDMM lane groups of <= 8 lanes
+  int32_t piece = 0;    // longest piece of a row
+  int32_t full_task = 0, full_piece = 0;   // both in the unsplit list of an SDDMM plan with a split part
+  int32_t row_task = 0;     // automatic entries per task of a large matrix
+  bool even = false;        // no row is longer than such a task
+};
+
+// Sizes for `entries` residual entries in `nonempty` rows, the longest row that tasks walk being `longest`; split:
+// the long rows are cut by XCD; task_opt, piece_opt: sizes that the caller asks for (0 = automatic).
+// Entries per task: about four mean rows, 32 .. 128 (MI355X: 32 for a degree-4 mesh, 128 for R-MAT).  Short rows
+// want small tasks (more lane groups in flight, fewer row flushes per group), long rows larger ones.
+// Small matrices are bound by the longest chain of batches any lane group walks, one memory round trip after
+// another, while the chip has lane groups to spare: their tasks hold 16 entries (tiny) or 32, and pieces of long
+// rows 32 or 64.  Measured, us per call at K = 32 / 64 / 128, pieces of 32 / 64 / 128 / 256 entries: R-MAT 2^12
+// (123K entries) 18 / 17 / 21, 22 / 23 / 28, 29 / 31 / 42; R-MAT 2^14 (491K) 19 / 20 / 26, 22 / 23 / 33, 36 / 38 /
+// 52; R-MAT 2^16 (2.0M; tasks of 32) 32 / 43 / 65, 32 / 41 / 57, 42 / 54 / 66; grid of 800^2 nodes with hubs (3.5M)
+// 51 / 80 / 191, 47 / 72 / 177, 50 / 71 / 168, 61 / 73 / 177.
+// Where no row is longer than a task (even) there is no long chain to shorten: tasks shrink to 16,384 of them (ER of
+// 52,861 nodes, 740K entries, K = 16 / 36 / 80 / 128, tasks of 16 10.7 / 20.7 / 25.2 / 30.1, of 45 10.5 / 14.5 / 21.0
+// / 26.8; ER of 60,000 nodes, 1.0M, K = 32 / 64 / 128 / 256, of 48 18.3 / 22.5 / 39.8 / 71.8, of 62 20.7 / 26.1 /
+// 35.6 / 68.9).
+// SDDMM lane groups of 16 lanes take larger tasks than narrower ones (no row is written per task), which walk a list
+// of their own: tiny plans 16,384 tasks, in steps of 4 (17 entries are three batches of 8, 16 two: ER of 40,000 nodes,
+// 280K, K = 16 8.8, 7.6) (R-MAT 2^14, K = 48 / 64, tasks of 16 19.3 / 19.6, of 30 17.1 / 17.6; ER of
+// 42,440 nodes, 552K, 19.3 / 19.2, of 33 17.8 / 17.9), small ones 64 (R-MAT 2^16 with 983K entries K = 64 / 128 / 200:
+// of 32 25.2 / 41.9 / 82.5, of 64 26.6 / 36.1 / 78.4); K <= 32 those of SpMM, even tiny plans at most 24 (ER of 28,439
+// nodes K = 16 / 32, of 16 9.7 / 10.8, 22 8.0 / 8.5, 30 9.6 / 9.9; of 60,000 nodes, 10 a row 12.3 / 14.2, 11.9 / 13.7,
+// 11.2 / 14.0, of 45 13.2 / 18.1).  With a split part that is for those who walk whole rows, K < 128; K >=
+// 128 take 16 (R-MAT 2^14 K = 128, of 16 22.4, of 28 27.8).  From 393K on the pieces of those who walk whole rows hold 64 (R-MAT 2^14 K = 80 / 96 22.3 / 23.0 with 32, 20.1 / 20.6 with 64; R-MAT 2^13, 150K, K = 64 8.7, 12.1).
+// Past kSmallEntries pieces of 128 pay where rows are short, and up to 5M entries, or 6M where the long rows are
+// split: a piece is a partial slot, written and summed again at every width (SpMM us, K = 16 / 64 / 128 / 200, pieces
+// of 128 / 256: R-MAT 2^19 with 4.9M entries, 20 a row 66 / 98 / 155 / 345, 90 / 106 / 168 / 354, with 5.9M, 22 a row 72
+// / 111 / 171 / 380, 80 / 106 / 164 / 369; R-MAT 2^17 with 3.2M, 36 a row 43 / 61 / 85 / 160, 47 / 55 / 72 / 150; R-MAT
+// 2^18 with 4.4M 63 / 79 / 117 / 237, 54 / 78 / 112 / 231; grid of 900^2 nodes, 4.5M 54 / - / 221 / 493, 60 / - / 232 /
+// 497, of 1000^2, 5.5M 66 / 133 / 247 / 598, 63 / 125 / 241 / 575).  The SDDMM writes no slots: 128 to 6M.
+inline TaskSizes task_sizes(int64_t entries, int64_t nonempty, int32_t longest, bool spmm, bool split, bool auto_split,
+                            int32_t task_opt, int32_t piece_opt) {
+  TaskSizes t;
+  const double mean = nonempty > 0 ? (double)entries / (double)nonempty : 1.0;
+  t.row_task = (int32_t)(4.0 * mean < 32.0 ? 32.0 : 4.0 * mean > 128.0 ? 128.0 : 4.0 * mean);
+  t.even = longest <= t.row_task;
+  const bool tiny = entries < kTinyEntries, small = entries < kSmallEntries;
+  auto at_most = [](int64_t v, int64_t hi) { return (int32_t)(v < hi ? v : hi); };
+  t.task = t.narrow = task_opt > 0 ? task_opt : t.row_task;
+  if (task_opt <= 0 && small) {
+    const int64_t least = tiny ? 16 : 32, uneven = entries / kMinTasksUneven;
+    const int64_t shared = spmm ? entries / kMinTasks : entries / kMinTasks / 4 * 4;
+    t.narrow = at_most(t.even && (spmm || tiny) ? (shared > least ? shared : least) : uneven > least ? uneven : least,
+                       t.row_task);
+    if (!spmm && tiny && t.narrow > 16) t.narrow = t.narrow < 24 ? 16 : 24;
+    t.task = spmm ? t.narrow : tiny ? at_most(shared > 16 ? shared : 16, t.row_task) : at_most(64, t.row_task);
+  }
+  t.full_task = t.task;
+  if (task_opt <= 0 && tiny && split && !spmm) t.task = 16;
+  // (pieces of 32 only with the automatic split threshold, which they were measured with)
+  int32_t piece = tiny && auto_split && (spmm || split || entries < 3 << 17) ? 32 : 64;
+  if (!small) {
+    const int64_t line = split || !spmm ? 6ll << 20 : 5'000'000;
+    piece = entries < line && (!spmm || 3 * t.row_task <= 2 * 128) ? 128 : 256;
+  }
+  // ... but a longest row of at most two pieces stays whole: the chain it saves is shorter than the fixup launch that
+  // cutting it asks for (ER of 4096 nodes, 17 entries a row, longest 40: 9.7 us with no row cut, 13.2 with a few)
+  while (piece < 256 && longest <= 2 * piece) piece *= 2;
+  if (piece_opt > 0) piece = piece_opt;
+  t.piece = piece > t.task ? piece : t.task;
+  // (no slots, no fixups to repeat; pieces twice as long where they were shortened: R-MAT 2^16 with 983K entries
+  // K = 64 26.6 -> 23.9 us, 2^17 with 2.9M 56.5 -> 52.6)
+  t.full_piece = t.piece;
+  const int32_t full = tiny ? 64 : 256;
+  if (piece_opt <= 0 && t.piece < full && (!tiny || entries >= 3 << 17)) t.full_piece = at_most(2 * t.piece, full);
+  if (t.full_piece < t.full_task) t.full_piece = t.full_task;
+  return t;
+}
+
 // Hot-row staging applies to 16-byte gathers of at least this many features (one 16-lane group,
 // 256-byte rows: R-MAT 2^20 K = 128 -6%, K = 256 -5%; K = 32 and 64 unchanged or slower).
 constexpr int kHotMinK = 128;

@@ -70,13 +70,12 @@ constexpr int kLowerOnHost = -100;
 // 2^20 step at K = 32 / 64 / 128 / 256: -16% / -6% / -18% / -19% against no split (128 and 512
 // entries measured slower at K = 128).  SDDMM, K = 128 / 256: -14% / -20% (its launcher keeps the
 // unsplit layout below K = 128, where the split measured slower: K = 32 / 64 / 96 +65% / +20% / +8%).
-// Below kSplitSmall entries the SpMM splits from 512 entries on: a shorter row's eight sub-rows are then
+// Below kSmallEntries entries the SpMM splits from 512 entries on: a shorter row's eight sub-rows are then
 // a task and a slot each with a few tens of entries (R-MAT 2^16, K = 32 / 64 / 128: 256 entries 35.1 /
 // 46.6 / 58.9 us, 512 31.8 / 40.6 / 57.1, no split 36.2 / 44.6 / 59.8; R-MAT 2^14 20.8 / 22.8 / 28.6,
 // 19.3 / 20.1 / 26.2, 20.0 / 23.2 / 26.8; R-MAT 2^18, 7.9M entries: the same within 1%; with 3.9M
-// entries the 256 are better: K = 80 90 / 100).  Tasks shrink below the same line (build_tasks).
+// entries the 256 are better: K = 80 90 / 100).  Tasks shrink below the same line (task_sizes).
 constexpr int32_t kSpmmSplitMin = 256;
-constexpr int64_t kSplitSmall = 3 << 20;
 constexpr int32_t kSddmmSplitMin = 512;
 // ... and only when those rows' entries are at least this many times their distinct columns:
 // R-MAT's rows of >= 256 entries gather 20.0M times from 0.60M columns (33x), the 64 hubs of the
@@ -725,12 +724,6 @@ struct Tasks {
   Status st;
 };
 
-// Residual tasks and pieces of long rows a plan aims at when the automatic sizes leave fewer (see
-// build_tasks).
-constexpr int64_t kMinTasks = 65536;
-constexpr int64_t kMinTasksEven = 16384;
-constexpr int64_t kMinPieces = 32768;
-constexpr int64_t kTinyEntries = 3 << 18;
 // Rows per chunk of the main part's task packing (a multiple of 16: MFMA windows stay whole).
 constexpr int64_t kPackRows = 1 << 16;
 
@@ -786,56 +779,21 @@ Tasks build_tasks(const Placement& P, const std::vector<int32_t>& rowptr, int32_
                   bool with_fixup, const trs_plan_options& opt) {
   Tasks T;
   const int64_t nent = rowptr[m];
-  // Entries per packed task: short rows want small tasks (more lane groups in flight, fewer row
-  // flushes per group), long rows want larger ones.  Measured on MI355X: 32 for a degree-4 mesh,
-  // 128 for R-MAT (mean non-empty row ~49) -- about four mean rows per task.
-  int S = opt.task_nnz;
-  if (S <= 0) {
-    int64_t nonempty = 0;
-    for (int32_t q = 0; q < m; ++q) nonempty += rowptr[q + 1] > rowptr[q];
-    const double mean = nonempty ? (double)nent / (double)nonempty : 1.0;
-    S = (int)std::min(128.0, std::max(32.0, 4.0 * mean));
-  }
-  // Small matrices are bound by the longest chain of batches any lane group walks, one memory round
-  // trip after another, while the chip has lane groups to spare: the automatic sizes shrink so that
-  // there are kMinTasks tasks (of at least 16 entries, 32 from kTinyEntries on, where every SIMD has
-  // its waves already: ER of 274K nodes K = 32 44 us with 32, 50 with 16) and pieces of long rows
-  // about as long as the entries divided by kMinPieces (a power of two from 64, or 32 below
-  // kTinyEntries, to 256).  Measured, us
-  // per call at K = 32 / 64 / 128, pieces of 32 / 64 / 128 / 256 entries: R-MAT 2^12 (123K entries) 18
-  // / 17 / 21, 22 / 23 / 28, 29 / 31 / 42; R-MAT 2^14 (491K) 19 / 20 / 26, 22 / 23 / 33, 36 / 38 / 52;
-  // R-MAT 2^16 (2.0M; tasks of 32) 32 / 43 / 65, 32 / 41 / 57, 42 / 54 / 66; grid of 800^2 nodes with
-  // hubs (3.5M) 51 / 80 / 191, 47 / 72 / 177, 50 / 71 / 168, 61 / 73 / 177; R-MAT 2^18 (7.9M) at 128
-  // and 256: 78 / 116 / 161, 95 / 112 / 155.
-  // SDDMM tasks of 16-lane groups hold twice that (no row is written per task; R-MAT 2^16 with 983K
-  // entries K = 64 / 128 / 200: tasks of 32 25.2 / 41.9 / 82.5, 64 26.6 / 36.1 / 78.4), those of narrower
-  // groups, which walk a list of their own, do not (K = 32: 21 with 32, 28 with 60).
-  // An SpMM no row of which fills a task has no long chain to shorten: from kTinyEntries on its tasks shrink
-  // only to kMinTasksEven of them (ER of 60,000 nodes, 17 entries a row, K = 32 / 64 / 128 / 256, tasks of 48:
-  // 18.3 / 22.5 / 39.8 / 71.8 us, of 62: 20.7 / 26.1 / 35.6 / 68.9, of 32 at K = 128 39.1; ER of 100,000 nodes
-  // K = 16, of 48 25.4, of 68 21.3).
-  int32_t longest = 0;
-  for (int32_t q = 0; q < m; ++q) longest = std::max(longest, rowptr[q + 1] - rowptr[q]);
-  int S_narrow = S;
-  if (opt.task_nnz <= 0 && nent < kSplitSmall) {   // (R-MAT 2^18 with 3.9M entries K = 16: 60 entries 64 us, 128 57)
-    const bool tiny = nent < kTinyEntries;
-    S_narrow = (int)std::min<int64_t>(S, std::max<int64_t>(tiny ? 16 : 32, nent / kMinTasks));
-    if (with_fixup && !tiny && longest <= S)
-      S_narrow = (int)std::min<int64_t>(S, std::max<int64_t>(32, nent / kMinTasksEven));
-    S = with_fixup || tiny ? S_narrow : (int)std::min<int64_t>(S, std::max<int64_t>(64, nent / kMinTasks));
-  }
-  T.task_nnz = S;
-  // (pieces of 32 only with the automatic split threshold, which they were measured with)
-  int piece_auto = nent >= kTinyEntries || opt.xcd_split != 0 ? 64 : 32;
-  while (piece_auto < 256 && nent / kMinPieces * 2 >= piece_auto * 3) piece_auto *= 2;
-  // ... but a longest row of at most two pieces stays whole: the chain it saves is shorter than the
-  // fixup launch that cutting it asks for (ER of 4096 nodes, 17 entries a row, longest 40: 9.7 us with no
-  // row cut, 13.2 with a few)
-  while (piece_auto < 256 && longest <= 2 * piece_auto) piece_auto *= 2;
-  const int piece_max = std::max(S, opt.piece_nnz > 0 ? opt.piece_nnz : piece_auto);
-  const int rows_cap = trs::kTaskRows;
+  // sizes by the entries, the rows that hold them, and the longest row that a task walks
   auto is_owned = [&](int32_t r) { return !owned.empty() && owned[r / 16]; };
   const int32_t J = P.J();
+  int64_t nonempty = 0;
+  int32_t longest = 0;
+  for (int32_t q = 0; q < m; ++q) {
+    const int32_t len = rowptr[q + 1] - rowptr[q];
+    nonempty += len > 0;
+    if (len > longest && !is_owned(q)) longest = len;
+  }
+  const trs::TaskSizes Z = trs::task_sizes(nent, nonempty, longest, with_fixup, J > 0, opt.xcd_split == 0, opt.task_nnz,
+                                           opt.piece_nnz);
+  const int S = Z.task, S_narrow = Z.narrow, piece_max = Z.piece;
+  T.task_nnz = S;
+  const int rows_cap = trs::kTaskRows;
   if (with_fixup) T.slots = J;   // sub-row j sums into slot j; piece slots follow
 
   // equal pieces of at most piece_max entries of [b, e) of (sub-)row r
@@ -860,7 +818,7 @@ Tasks build_tasks(const Placement& P, const std::vector<int32_t>& rowptr, int32_
     ++T.split_rows;
   };
   // runs of whole (sub-)rows [r, r1) of rp, row r1 - r <= rows_cap, entries <= run_max (S, or the
-  // narrow list's), none longer than piece_max; stop(r) ends a run before row r
+  // unsplit or narrow list's), none longer than piece_max; stop(r) ends a run before row r
   int run_max = S;
   auto pack = [&](const std::vector<int32_t>& rp, int32_t r, int32_t end, auto&& stop) {
     int32_t r1 = r + 1;
@@ -918,16 +876,18 @@ Tasks build_tasks(const Placement& P, const std::vector<int32_t>& rowptr, int32_
     sort_longest_first(outv.begin(), outv.end());
   };
   build_main(true, T.tasks, piece_max);
-  // (SDDMM: no slots, no fixups to repeat; its unsplit list in pieces twice as long where they were
-  // shortened: R-MAT 2^16 with 983K entries K = 64 26.6 -> 23.9 us, 2^17 with 2.9M 56.5 -> 52.6)
-  if (!with_fixup && J > 0)
-    build_main(false, T.full, opt.piece_nnz <= 0 && nent >= kTinyEntries ? std::min(256, 2 * piece_max) : piece_max);
+  if (!with_fixup && J > 0) {   // SDDMM: no slots, no fixups to repeat
+    run_max = Z.full_task;
+    build_main(false, T.full, Z.full_piece);
+    run_max = S;
+  }
   // SDDMM lane groups of <= 8 lanes walk the unsplit layout in pieces of S entries: with 8 lanes
   // to a group a wave holds 8 tasks, and the long rows' pieces should not hold them for 256
   // entries (same-box A/B on R-MAT 2^20, pieces of 128 against 256: K = 16 0.302 -> 0.288 ms, K =
   // 32 0.359 -> 0.337; 16-lane groups lose with them, K = 64 0.443 -> 0.454, K = 96 0.651 ->
   // 0.668, and keep the 256-entry pieces)
-  if (!with_fixup && opt.piece_nnz <= 0 && piece_max > S_narrow) {
+  // (compared with the pieces of the list that they would walk otherwise)
+  if (!with_fixup && opt.piece_nnz <= 0 && (J > 0 ? Z.full_piece : piece_max) > S_narrow) {
     bool longer = false;
     for (int32_t r = 0; r < m && !longer; ++r) longer = !is_owned(r) && rp[r + 1] - rp[r] > S_narrow;
     if (longer) {
@@ -1686,7 +1646,7 @@ Status finalize(Lowering& L, const trs_plan_options& opt, trs_plan** out, const 
   // residual tasks over rows not owned by an MFMA window
   // XCD column split for SpMM (each sub-row costs a partial slot of 4 K bytes written and read back)
   const int32_t split_min = opt.xcd_split < 0 ? 0 : opt.xcd_split > 0 ? opt.xcd_split
-                            : nent < kSplitSmall ? 2 * kSpmmSplitMin : kSpmmSplitMin;
+                            : nent < trs::kSmallEntries ? 2 * kSpmmSplitMin : kSpmmSplitMin;
   const int32_t reuse = opt.xcd_split == 0 ? kSplitMinReuse : 0;
   Status pst;
   const Placement PL =
