@@ -11,6 +11,27 @@ void rule_task_sizes(int64_t entries, int64_t nonempty, int32_t longest, int32_t
   const int32_t v[7] = {t.task, t.narrow, t.piece, t.full_task, t.full_piece, t.row_task, t.even ? 1 : 0};
   for (int i = 0; i < 7; ++i) out[i] = v[i];
 }
+// plan fields: entries, columns, rows cut into pieces, split part's tasks, task_nnz, row_task, even_rows, staged rows,
+// feature_lanes; out: features per lane, lanes per group (0: as many as the width needs)
+static trs::DevicePlan plan_of(const int64_t* f) {
+  trs::DevicePlan p;
+  p.nnz_csr = f[0];
+  p.m = p.n = (int32_t)f[1];
+  p.nfixups = (int32_t)f[2];
+  p.x_ntasks = (int32_t)f[3];
+  p.task_nnz = (int32_t)f[4];
+  p.row_task = (int32_t)f[5];
+  p.even_rows = (int32_t)f[6];
+  p.nhot = (int32_t)f[7];
+  p.feature_lanes = (int32_t)f[8];
+  return p;
+}
+void rule_spmm_route(const int64_t* f, int32_t K, int32_t aligned, int32_t* out) {
+  const trs::Route r = trs::spmm_route(plan_of(f), K, aligned != 0);
+  out[0] = r.vec;
+  out[1] = r.lanes;
+}
+int64_t rule_hot_bytes(const int64_t* f, int32_t K, int32_t sddmm) { return trs::hot_buffer_bytes(plan_of(f), K, sddmm != 0); }
 int32_t rule_counts_in_lds(int32_t n) { return trs::counts_in_lds(n) ? 1 : 0; }
 
 }

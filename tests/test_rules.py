@@ -19,6 +19,9 @@ def rules(tmp_path_factory):
                            "-I", INC, SRC, "-o", so])
     lib = ctypes.CDLL(so)
     lib.rule_lds_count_copies.argtypes = [ctypes.c_int64, ctypes.c_int32]
+    lib.rule_spmm_route.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]
+    lib.rule_hot_bytes.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32]
+    lib.rule_hot_bytes.restype = ctypes.c_int64
     lib.rule_task_sizes.argtypes = [ctypes.c_int64, ctypes.c_int64] + [ctypes.c_int32] * 5 + [ctypes.c_void_p]
     return lib
 
@@ -91,3 +94,39 @@ def test_asked_sizes_are_taken(rules):
         assert (z["task"], z["narrow"], z["piece"], z["full_piece"]) == (24, 24, 100, 100)
         z = sizes(rules, 2_000_000, 40_000, 4000, spmm, task=512)
         assert (z["task"], z["piece"]) == (512, 512) and z["full_piece"] >= 512
+
+
+def plan(entries, n, cut=0, split=0, task=64, row_task=64, even=0, hot=0, lanes=0):
+    return (ctypes.c_int64 * 9)(entries, n, cut, split, task, row_task, even, hot, lanes)
+
+
+def spmm(rules, p, K, aligned=True):
+    out = (ctypes.c_int32 * 2)()
+    rules.rule_spmm_route(p, K, int(aligned), out)
+    return tuple(out)
+
+
+RMAT = dict(entries=7_900_000, n=1 << 18, cut=9000, split=20_000, task=128, row_task=128, hot=16384)
+
+
+def test_spmm_one_pass_widths(rules):
+    short = plan(3_496_630, 349_663, task=44, row_task=44, even=1)
+    long_rows = plan(2_400_000, 142_496, task=68, row_task=68, even=1)
+    for K in range(100, 257, 4):
+        if K % 8 == 0:
+            assert spmm(rules, plan(**RMAT), K) == spmm(rules, short, K) == (8, 0)
+        elif K < 128:
+            assert spmm(rules, short, K) == (4, 32) and spmm(rules, long_rows, K) == spmm(rules, plan(**RMAT), K) == (8, 0)
+        else:
+            assert spmm(rules, short, K) == (4, 64) and spmm(rules, long_rows, K) == spmm(rules, plan(**RMAT), K) == (8, 32)
+            # no staged rows, and no bytes for them
+            assert rules.rule_hot_bytes(plan(**RMAT), K, 0) == 0 and rules.rule_hot_bytes(plan(**RMAT), K + 1, 0) > 0
+            # a plan that asks for fewer lanes keeps its passes
+            assert spmm(rules, plan(**{**RMAT, "lanes": 16}), K) == (8, 0)
+            assert rules.rule_hot_bytes(plan(**{**RMAT, "lanes": 16}), K, 0) > 0
+    assert spmm(rules, plan((1 << 17) - 1, 20_000, task=16, row_task=36, even=1), 180) == (8, 32)
+    assert spmm(rules, plan(TINY - 1, 140_000, cut=64, task=16, row_task=32), 180) == (8, 32)
+    assert spmm(rules, plan(TINY, 140_000, cut=64, task=32, row_task=32), 180) == (4, 64)
+    assert spmm(rules, short, 260) == (4, 64) and spmm(rules, long_rows, 388) == (8, 32) and spmm(rules, plan(**RMAT), 260) == (8, 0)
+    for K in (129, 130, 131, 254, 255, 258, 264):
+        assert spmm(rules, short, K) == (8, 0)

@@ -1368,17 +1368,17 @@ void launch_windows_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, int
 
 template <int VEC>
 hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
-                           float* partial, uint16_t* hot, hipStream_t s, hipEvent_t* ev) {
+                           float* partial, uint16_t* hot, int lanes, hipStream_t s, hipEvent_t* ev) {
   if (ev) (void)hipEventRecord(ev[0], s);
-  int lpg = lanes_for(K, VEC);
+  int lpg = lanes > 0 ? lanes : lanes_for(K, VEC);
   // a plan may ask for fewer lanes per group: several feature passes, each gathering a narrower
   // slice of B (smaller working set per pass)
   while (p.feature_lanes > 0 && lpg > p.feature_lanes && lpg > 1) lpg >>= 1;
   // passes of at most 128 features for 16-byte loads: each pass gathers 256-byte slices of B
   // rows, twice as many of which fit an XCD's L2 as whole 512-byte rows (R-MAT 2^20, K = 256:
   // 1.730 ms in one pass of 32 lanes, 1.522 in two of 16, 1.837 in four of 8; K = 128 in two
-  // passes of 64 features: 0.748 -> 0.910)
-  if (p.feature_lanes <= 0 && VEC == 8 && lpg > 16) lpg = 16;
+  // passes of 64 features: 0.748 -> 0.910), but for the widths of spmm_one_pass
+  if (p.feature_lanes <= 0 && VEC == 8 && lpg > 16 && lanes <= 0) lpg = 16;
   // at least 4 lanes, whose column/value loads are shared, also where K < 4 leaves lanes idle
   // (same-box A/B: R-MAT K=1 0.316 -> 0.183 ms, K=2 0.255 -> 0.201; grid+hubs K=1 0.201 -> 0.122,
   // K=2 0.237 -> 0.175; 8 lanes at K=3: R-MAT 0.214 -> 0.258)
@@ -1459,11 +1459,11 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     }                                                                                                     \
     break;                                                                                                \
   }
-    // 4- and 2-byte loads serve K <= 8 in groups of 4 or 8 lanes, 8-byte ones K <= 64 in 4 or 16 lanes
+    // 4- and 2-byte loads serve K <= 8 in groups of 4 or 8 lanes
     if constexpr (VEC < 4) {
       switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) }
     } else if constexpr (VEC < 8) {
-      switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) TRS_TASKS(16) }
+      switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) TRS_TASKS(16) TRS_TASKS(32) TRS_TASKS(64) }
     } else {
       switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) TRS_TASKS(16) TRS_TASKS(32) TRS_TASKS(64) }
     }
@@ -1490,7 +1490,7 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     if constexpr (VEC < 4) {
       switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) }
     } else if constexpr (VEC < 8) {
-      switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) TRS_FIX(16) }
+      switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) TRS_FIX(16) TRS_FIX(32) TRS_FIX(64) }
     } else {
       switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) TRS_FIX(16) TRS_FIX(32) TRS_FIX(64) }
     }
@@ -1986,7 +1986,7 @@ __global__ __launch_bounds__(256) void k_zero_fill(float* __restrict__ out, int6
 // their own (this file with TRS_KERNEL_PART = the width), part 0 holds the rest and calls them.
 template <int VEC>
 hipError_t spmm_width(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
-                      float* partial, uint16_t* hot, hipStream_t s, hipEvent_t* ev);
+                      float* partial, uint16_t* hot, int lanes, hipStream_t s, hipEvent_t* ev);
 template <int VEC>
 void windows_width(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc, hipStream_t s);
 template <int VEC>
@@ -1995,8 +1995,8 @@ hipError_t sddmm_width(const DevicePlan& p, const uint16_t* X, int64_t ldx, cons
 #if TRS_KERNEL_PART > 0
 template <int VEC>
 hipError_t spmm_width(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
-                      float* partial, uint16_t* hot, hipStream_t s, hipEvent_t* ev) {
-  return launch_spmm_vec<VEC>(p, B, ldb, K, C, ldc, partial, hot, s, ev);
+                      float* partial, uint16_t* hot, int lanes, hipStream_t s, hipEvent_t* ev) {
+  return launch_spmm_vec<VEC>(p, B, ldb, K, C, ldc, partial, hot, lanes, s, ev);
 }
 template <int VEC>
 void windows_width(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc, hipStream_t s) {
@@ -2010,7 +2010,7 @@ hipError_t sddmm_width(const DevicePlan& p, const uint16_t* X, int64_t ldx, cons
 #endif
 #define TRS_WIDTH_INSTANCES(PREFIX, V)                                                                       \
   PREFIX template hipError_t spmm_width<V>(const DevicePlan&, const uint16_t*, int64_t, int, float*, int64_t, \
-                                           float*, uint16_t*, hipStream_t, hipEvent_t*);                      \
+                                           float*, uint16_t*, int, hipStream_t, hipEvent_t*);                 \
   PREFIX template void windows_width<V>(const DevicePlan&, const uint16_t*, int64_t, int, float*, int64_t,    \
                                         hipStream_t);                                                         \
   PREFIX template hipError_t sddmm_width<V>(const DevicePlan&, const uint16_t*, int64_t, const uint16_t*,     \
@@ -2134,45 +2134,15 @@ void launch_spmm_windows(const DevicePlan& p, const uint16_t* B, int64_t ldb, in
   else windows_width<1>(p, B, ldb, K, C, ldc, stream);
 }
 
-// Bytes a call reads and writes at least (entries, B, C) past which its gathers wait on HBM.
-constexpr int64_t kBeyondMall = 320'000'000;
-
 hipError_t launch_spmm(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
                        float* partial, uint16_t* hot, hipStream_t stream, hipEvent_t* ev) {
-  // wide loads only where they leave at least 4 lanes per group (whose column/value loads are
-  // shared): with K <= 8 one or two lanes would stream a task alone (R-MAT K=8: 0.545 ms with one
-  // 16-byte load per entry, 0.348 with two lanes of 8-byte loads, 0.283 with eight lanes of 2-byte
-  // loads, 0.273 with four lanes of 4-byte loads (below); K=4 0.515 -> 0.220), and K=16 runs best
-  // as 4 lanes of 8-byte loads (R-MAT 0.436 ms with 2 lanes of 16-byte loads, 0.324; grid+hubs
-  // 0.368 -> 0.307)
-  // Load width by K alone: a row of any alignment is read with whole vectors (see half8_u), the last
-  // lane taking the row's last VEC features.  16-byte loads from K = 17 on, where 3 lanes of a group
-  // have work (K = 16 is faster as 4 lanes of 8 bytes: R-MAT 2^20 0.436 -> 0.324 ms, and K = 8 as 4
-  // lanes of 4 bytes: 0.545 -> 0.273; K = 4 as 4 lanes of 2 bytes: 0.233 -> 0.219).  With narrower
-  // loads for the widths that 8, 4 or 2 do not divide, and 2-byte ones for odd ones, R-MAT 2^20 took
-  // (us, narrow -> this): K = 5 310 -> 244, 7 336 -> 262, 13 348 -> 289, 17 580 -> 379, 18 385 ->
-  // 312, 28 460 -> 371, 31 643 -> 458, 65 1755 -> 643, 97 2198 -> 724, 100 942 -> 661, 127 2425 -> 814,
-  // 130 2122 -> 1333, 255 4436 -> 1618; SBM 250K nodes K = 17 76 -> 43, 65 169 -> 95, 127 240 -> 132.
-  // K = 33..64 take 8-byte loads in 16-lane groups, whose staged stream holds more entries in flight than
-  // 8-lane groups of 16-byte loads held to 2 waves (us, 16-byte / 8-byte, in batches of 8): R-MAT 2^20 K =
-  // 33 595 / 442, 41 622 / 453, 48 507 / 372, 64 457 / 376; R-MAT 2^18 K = 40 / 48 / 56 / 64 120 / 120 / 127 / 112,
-  // 110 / 110 / 115 / 109; R-MAT 2^14 K = 64 20.4 / 18.7; ER of 274K nodes K = 40 69.8 / 66.5; grid of 4M nodes
-  // with hubs K = 64 587 / 564.  On the 16-byte grid the 16-byte loads stay where pieces of a few hub rows are
-  // far longer than the packed tasks of a mesh and the operands fit the MALL: grid of 640K nodes (tasks of
-  // 32, pieces of 128) K = 40 / 48 / 64 73 / 74 / 71, 79 / 85 / 85; with 2M nodes, past it, both the same.
-  // K = 5 and 7 stay on 8 lanes of 2 bytes over short rows (grid of 2M nodes K = 7: 109 us, 127 with 4-byte
-  // loads; R-MAT, whose tasks are long, 336 / 262)
-  const bool aligned = K % 8 == 0 && ldb % 8 == 0 && aligned16(B);
-  const int64_t touched = p.nnz_csr * 6 + (int64_t)p.m * K * 4 + (int64_t)p.n * K * 2;
-  const bool hub_pieces = p.task_max > 3 * p.task_nnz && touched < kBeyondMall;
-  const bool v8 = K > 16 && (K <= 32 || K > 64 || (aligned && hub_pieces)), v4 = K > 8,
-             v2 = K > 4 && (K % 2 == 0 || K > 8 || p.task_nnz >= 64);
+  const Route r = spmm_route(p, K, ldb % 8 == 0 && aligned16(B));
   // (the staged hot rows need 16-byte aligned rows in the buffer too)
   if (hot != nullptr && !aligned16(hot)) hot = nullptr;
-  return v8 ? spmm_width<8>(p, B, ldb, K, C, ldc, partial, hot, stream, ev)
-       : v4 ? spmm_width<4>(p, B, ldb, K, C, ldc, partial, nullptr, stream, ev)
-       : v2 ? spmm_width<2>(p, B, ldb, K, C, ldc, partial, nullptr, stream, ev)
-            : spmm_width<1>(p, B, ldb, K, C, ldc, partial, nullptr, stream, ev);
+  return r.vec == 8 ? spmm_width<8>(p, B, ldb, K, C, ldc, partial, hot, r.lanes, stream, ev)
+       : r.vec == 4 ? spmm_width<4>(p, B, ldb, K, C, ldc, partial, nullptr, r.lanes, stream, ev)
+       : r.vec == 2 ? spmm_width<2>(p, B, ldb, K, C, ldc, partial, nullptr, r.lanes, stream, ev)
+                    : spmm_width<1>(p, B, ldb, K, C, ldc, partial, nullptr, r.lanes, stream, ev);
 }
 
 hipError_t launch_sddmm(const DevicePlan& p, const uint16_t* X, int64_t ldx, const uint16_t* Y, int64_t ldy,

@@ -76,6 +76,8 @@ struct DevicePlan {
   int32_t sddmm_unroll = 0;    // SDDMM residual entries in flight per lane group (4, 8; 0 automatic)
   int32_t split_dispatch = 0;  // 1: main part and XCD split part as two launches (profiling)
   int32_t task_nnz = 0;        // entries per packed residual task
+  int32_t row_task = 0;        // ... of a large matrix with these rows (see task_sizes)
+  int32_t even_rows = 0;       // 1: no row that tasks walk is longer than that
   int32_t task_max = 0;        // most entries of any residual task (packed rows or a piece)
   const int32_t* slot_list = nullptr;   // partial slots of the split rows, in summation order
   // XCD column split: sub-rows (pieces of long rows by column range, laid out range-major in
@@ -205,6 +207,72 @@ inline TaskSizes task_sizes(int64_t entries, int64_t nonempty, int32_t longest, 
   return t;
 }
 
+// How a width is run: features per lane (16-, 8-, 4- or 2-byte loads) and lanes per group (0: as many as the width
+// needs, at most 16 of 16-byte loads).
+struct Route { int vec, lanes; };
+
+// SpMM widths K = 132, 140, .. 252, that 4 divides and 8 does not, in one feature pass: two passes of rows off the
+// 16-byte grid cost more than the narrower slices save (us, two passes of 16 lanes of 16 bytes / one of 32 / one of
+// 64 lanes of 8 bytes: ER of 907,888 nodes K = 132 / 180 / 244 1458 / 1646 / 1935, 854 / 1071 / 1362, 908 / 1132 /
+// 1374; ER of 150,000 nodes, 9 a row 126 / 151 / 182, 86 / 105 / 136, 82 / 100 / 127; R-MAT 2^18 with 7.9M entries 309
+// / 306 / 358, 263 / 277 / 321, 384 / 384 / 409; grid of 1300^2 nodes 810 / 1025 / 1264, 691 / 811 / 1013, 726 / 800
+// / 917).
+// The staged rows serve passes of 16 lanes only.
+inline bool spmm_one_pass(int K) { return K > 128 && K <= 256 && K % 4 == 0 && K % 8 != 0; }
+// 8-byte loads serve those widths, and K = 100 .. 124, where rows are short and nothing is staged, but for the
+// smallest plans (K = 100 / 124, 16 lanes of 16 bytes / 32 of 8: ER of 349,663 nodes, 11 a row 191 / 222, 185 / 218; of
+// 80,000 nodes, 9 a row 38.4 / 44.2, 34.7 / 40.3; grid of 1300^2 nodes 454 / 545, 450 / 510; longer rows lose, ER of
+// 142,496 nodes, 17 a row 102 / 121, 105 / 124).
+inline bool unstaged(const DevicePlan& p) { return p.x_ntasks == 0 && p.nhot == 0; }
+// Uneven rows from 786K entries on only (grid of 300^2 nodes with hubs, 495K entries, K = 132 / 244, 32 lanes / 64: 39.6
+// / 54.1, 42.7 / 56.5).
+inline bool short_rows(const DevicePlan& p) {
+  return p.row_task < 64 && unstaged(p) && p.nnz_csr >= (p.even_rows ? 1 << 17 : kTinyEntries);
+}
+
+// The route of an SpMM (aligned: rows of B on the 16-byte grid).
+// wide loads only where they leave at least 4 lanes per group (whose column/value loads are
+// shared): with K <= 8 one or two lanes would stream a task alone (R-MAT K=8: 0.545 ms with one
+// 16-byte load per entry, 0.348 with two lanes of 8-byte loads, 0.283 with eight lanes of 2-byte
+// loads, 0.273 with four lanes of 4-byte loads (below); K=4 0.515 -> 0.220), and K=16 runs best
+// as 4 lanes of 8-byte loads (R-MAT 0.436 ms with 2 lanes of 16-byte loads, 0.324; grid+hubs
+// 0.368 -> 0.307)
+// Load width by K alone: a row of any alignment is read with whole vectors (see half8_u), the last
+// lane taking the row's last VEC features.  16-byte loads from K = 17 on, where 3 lanes of a group
+// have work (K = 16 is faster as 4 lanes of 8 bytes: R-MAT 2^20 0.436 -> 0.324 ms, and K = 8 as 4
+// lanes of 4 bytes: 0.545 -> 0.273; K = 4 as 4 lanes of 2 bytes: 0.233 -> 0.219).  With narrower
+// loads for the widths that 8, 4 or 2 do not divide, and 2-byte ones for odd ones, R-MAT 2^20 took
+// (us, narrow -> this): K = 5 310 -> 244, 7 336 -> 262, 13 348 -> 289, 17 580 -> 379, 18 385 ->
+// 312, 28 460 -> 371, 31 643 -> 458, 65 1755 -> 643, 97 2198 -> 724, 100 942 -> 661, 127 2425 -> 814,
+// 130 2122 -> 1333, 255 4436 -> 1618; SBM 250K nodes K = 17 76 -> 43, 65 169 -> 95, 127 240 -> 132.
+// K = 33..64 take 8-byte loads in 16-lane groups, whose staged stream holds more entries in flight than
+// 8-lane groups of 16-byte loads held to 2 waves (us, 16-byte / 8-byte, in batches of 8): R-MAT 2^20 K =
+// 33 595 / 442, 41 622 / 453, 48 507 / 372, 64 457 / 376; R-MAT 2^18 K = 40 / 48 / 56 / 64 120 / 120 / 127 / 112,
+// 110 / 110 / 115 / 109; R-MAT 2^14 K = 64 20.4 / 18.7; ER of 274K nodes K = 40 69.8 / 66.5; grid of 4M nodes
+// with hubs K = 64 587 / 564.  On the 16-byte grid the 16-byte loads stay where pieces of a few hub rows are
+// far longer than the packed tasks of a mesh and the operands fit the MALL: grid of 640K nodes (tasks of
+// 32, pieces of 128) K = 40 / 48 / 64 73 / 74 / 71, 79 / 85 / 85; with 2M nodes, past it, both the same.
+// K = 5 and 7 stay on 8 lanes of 2 bytes over short rows (grid of 2M nodes K = 7: 109 us, 127 with 4-byte
+// loads; R-MAT, whose tasks are long, 336 / 262)
+inline Route spmm_route(const DevicePlan& p, int K, bool aligned) {
+  const bool any_lanes = p.feature_lanes <= 0;   // (a plan may ask for fewer lanes)
+  if (K <= 8) return {K > 4 && (K % 2 == 0 || p.task_nnz >= 64) ? 2 : 1, 0};
+  if (K <= 16) return {4, 0};
+  if (K <= 32) return {8, 0};
+  if (K <= 64) {
+    const int64_t touched = p.nnz_csr * 6 + (int64_t)p.m * K * 4 + (int64_t)p.n * K * 2;
+    const bool hub_pieces = p.task_max > 3 * p.task_nnz && touched < 320'000'000;   // (past that, gathers wait on HBM)
+    return {aligned && K % 8 == 0 && hub_pieces ? 8 : 4, 0};
+  }
+  if (any_lanes && K % 4 == 0 && K % 8 != 0) {
+    if (K > 96 && K <= 128 && short_rows(p)) return {4, 32};
+    // (past 256 features passes of 256, where nothing is staged: ER of 150,000 nodes K = 300 / 388 231 / 292 us in passes of
+    // 128, 203 / 233)
+    if (spmm_one_pass(K) || (K > 256 && unstaged(p))) return short_rows(p) ? Route{4, 64} : Route{8, 32};
+  }
+  return {8, 0};
+}
+
 // Hot-row staging applies to 16-byte gathers of at least this many features (one 16-lane group,
 // 256-byte rows: R-MAT 2^20 K = 128 -6%, K = 256 -5%; K = 32 and 64 unchanged or slower).
 constexpr int kHotMinK = 128;
@@ -230,6 +298,7 @@ inline int hot_row_stride(int K) { return K % 8 == 0 ? K : (K + 63) / 64 * 64; }
 // Bytes of the staged-row buffer of plan p at width K (0 when the plan or K does not stage).
 inline int64_t hot_buffer_bytes(const DevicePlan& p, int K, bool sddmm) {
   if (p.nhot <= 0 || !stages_hot_rows(K, sddmm)) return 0;
+  if (!sddmm && p.feature_lanes <= 0 && spmm_one_pass(K)) return 0;
   return (int64_t)p.nhot * hot_row_stride(K) * 2;
 }
 // Column histogram of col[0, total) into counts[n] (ids outside [0, n) are skipped), counted in

@@ -720,6 +720,7 @@ struct Tasks {
   int32_t slots = 0;
   int64_t split_rows = 0;
   int32_t task_nnz = 0;              // entries per packed task (S)
+  int32_t row_task = 0, even = 0;    // see TaskSizes
   int32_t task_max = 0, xtask_max = 0;
   Status st;
 };
@@ -793,6 +794,8 @@ Tasks build_tasks(const Placement& P, const std::vector<int32_t>& rowptr, int32_
                                            opt.piece_nnz);
   const int S = Z.task, S_narrow = Z.narrow, piece_max = Z.piece;
   T.task_nnz = S;
+  T.row_task = Z.row_task;
+  T.even = Z.even;
   const int rows_cap = trs::kTaskRows;
   if (with_fixup) T.slots = J;   // sub-row j sums into slot j; piece slots follow
 
@@ -1734,6 +1737,8 @@ Status finalize(Lowering& L, const trs_plan_options& opt, trs_plan** out, const 
   // default: non-temporal C stores only (measured +3%); non-temporal A loads cost ~60% because
   // consecutive iterations re-read the same col/val cache lines
   d.task_nnz = T.task_nnz;
+  d.row_task = T.row_task;
+  d.even_rows = T.even;
   d.task_max = T.task_max;
   d.streaming = opt.streaming < 0 ? 2 : opt.streaming;
   d.xcd_run = opt.xcd_run > 0 ? opt.xcd_run : 16;
@@ -1961,6 +1966,8 @@ Status finalize_sddmm(Lowering& L, const trs_plan_options& opt, bool keep_order,
   d.stage = opt.stage < 0 ? -1 : 0;
   d.occupancy = opt.occupancy < 0 ? -1 : opt.occupancy == 0 ? 0 : std::min(8, std::max(2, opt.occupancy));
   d.task_nnz = T.task_nnz;
+  d.row_task = T.row_task;
+  d.even_rows = T.even;
   d.task_max = T.task_max;
   P->csr_only = true;
   trs_plan_stats& s = P->stats;
