@@ -130,3 +130,18 @@ def test_spmm_one_pass_widths(rules):
     assert spmm(rules, short, 260) == (4, 64) and spmm(rules, long_rows, 388) == (8, 32) and spmm(rules, plan(**RMAT), 260) == (8, 0)
     for K in (129, 130, 131, 254, 255, 258, 264):
         assert spmm(rules, short, K) == (8, 0)
+
+
+def test_spmm_even_rows_of_narrow_widths(rules):
+    big = dict(entries=2_400_000, n=142_496, task=68, row_task=68, even=1)
+    for K in range(9, 33):
+        assert spmm(rules, plan(**big), K) == ((1, 16) if K <= 16 else (2, 16))
+        # a cut row, a split part or fewer lanes asked for: as any plan
+        for other in (dict(cut=1), dict(split=8), dict(lanes=8), dict(even=0)):
+            assert spmm(rules, plan(**{**big, **other}), K) == ((4, 0) if K <= 16 else (8, 0))
+        # operands within half an L2, and tiny plans
+        small = plan(**{**big, "n": 2_000_000 // (2 * K) - 1})
+        tiny = plan(**{**big, "entries": TINY - 1})
+        for p in (small, tiny):
+            assert spmm(rules, p, K) == ((4, 0) if K <= 16 else (4, 8) if K % 2 else (8, 0))
+        assert spmm(rules, plan(**{**big, "entries": (1 << 18) - 1}), K) == ((4, 0) if K <= 16 else (4, 8))

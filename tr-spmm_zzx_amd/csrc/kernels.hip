@@ -1459,9 +1459,9 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     }                                                                                                     \
     break;                                                                                                \
   }
-    // 4- and 2-byte loads serve K <= 8 in groups of 4 or 8 lanes
+    // 4- and 2-byte loads: groups of 4 or 8 lanes to K = 8, of 16 lanes to K = 32
     if constexpr (VEC < 4) {
-      switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) }
+      switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) TRS_TASKS(16) }
     } else if constexpr (VEC < 8) {
       switch (lpg) { TRS_TASKS(1) TRS_TASKS(2) TRS_TASKS(4) TRS_TASKS(8) TRS_TASKS(16) TRS_TASKS(32) TRS_TASKS(64) }
     } else {
@@ -1488,7 +1488,7 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     dim3 grid(p.nwfixups + (p.nfixups + gpb - 1) / gpb, passes);
 #define TRS_FIX(L) case L: hipLaunchKernelGGL((k_spmm_fixup<VEC, L>), grid, dim3(256), 0, s, p, K, C, ldc, partial); break;
     if constexpr (VEC < 4) {
-      switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) }
+      switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) TRS_FIX(16) }
     } else if constexpr (VEC < 8) {
       switch (lpg) { TRS_FIX(1) TRS_FIX(2) TRS_FIX(4) TRS_FIX(8) TRS_FIX(16) TRS_FIX(32) TRS_FIX(64) }
     } else {

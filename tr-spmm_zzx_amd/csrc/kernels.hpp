@@ -230,6 +230,8 @@ inline bool short_rows(const DevicePlan& p) {
   return p.row_task < 64 && unstaged(p) && p.nnz_csr >= (p.even_rows ? 1 << 17 : kTinyEntries);
 }
 
+// Even rows, none of them cut into pieces.
+inline bool uncut(const DevicePlan& p) { return p.even_rows && p.nfixups + p.nwfixups == 0 && p.x_ntasks == 0; }
 // The route of an SpMM (aligned: rows of B on the 16-byte grid).
 // wide loads only where they leave at least 4 lanes per group (whose column/value loads are
 // shared): with K <= 8 one or two lanes would stream a task alone (R-MAT K=8: 0.545 ms with one
@@ -256,6 +258,17 @@ inline bool short_rows(const DevicePlan& p) {
 // loads; R-MAT, whose tasks are long, 336 / 262)
 inline Route spmm_route(const DevicePlan& p, int K, bool aligned) {
   const bool any_lanes = p.feature_lanes <= 0;   // (a plan may ask for fewer lanes)
+  if (any_lanes && K > 8 && K <= 32 && uncut(p)) {
+    // Rows of one length, none cut: past 2 MB of B (half an XCD's L2) the gathers miss and no hot rows serve them,
+    // which the many lanes and uncapped waves of narrow loads in 16-lane groups with a staged stream stand best (us,
+    // K = 9 / 16 / 18 / 24 / 31, 4-lane groups of 8 (K <= 16) or 16 bytes / this: ER of 142,496 nodes 35.9 / 37.7 / 43.2
+    // / 47.3 / 62.5, 31.7 / 29.6 / 35.3 / 34.6 / 46.5; of 907,888 nodes 308 / 297 / 361 / 363 / 447, 256 / 255 / 324 / 332
+    // / 407).  Below, and in tiny plans, 8-lane groups of 8-byte loads for odd widths, and for all in the smallest plans
+    // (K = 17 / 24 / 31: ER of 28,439 nodes 12.7 / 9.1 / 12.9, 11.6 / 10.1 / 11.7; of 30,000 nodes, 180K entries 9.7 / 8.0 /
+    // 9.8, 7.2 / 6.7 / 7.2).
+    if (p.nnz_csr >= kTinyEntries && (int64_t)p.n * K * 2 >= 2'000'000) return {K <= 16 ? 1 : 2, 16};
+    if (K > 16 && (K % 2 != 0 || p.nnz_csr < 1 << 18)) return {4, 8};
+  }
   if (K <= 8) return {K > 4 && (K % 2 == 0 || p.task_nnz >= 64) ? 2 : 1, 0};
   if (K <= 16) return {4, 0};
   if (K <= 32) return {8, 0};
