@@ -145,3 +145,27 @@ def test_spmm_even_rows_of_narrow_widths(rules):
         for p in (small, tiny):
             assert spmm(rules, p, K) == ((4, 0) if K <= 16 else (4, 8) if K % 2 else (8, 0))
         assert spmm(rules, plan(**{**big, "entries": (1 << 18) - 1}), K) == ((4, 0) if K <= 16 else (4, 8))
+
+
+MESH = dict(entries=3_500_000, n=640_000, cut=64, task=32, row_task=32)
+
+
+def test_spmm_meshes_with_a_few_long_rows(rules):
+    for K in range(9, 33):
+        small = {**MESH, "entries": (1 << 18) - 1, "n": 47_000}
+        assert spmm(rules, plan(**small), K) == ((1, 16) if K <= 16 else (2, 16))
+        for n in (640_000, 1_690_000, 4_194_304):
+            want = (4, 0) if K <= 16 else (4, 8) if K % 8 and 32 << 20 <= n * K * 2 < 128 << 20 else (8, 0)
+            assert spmm(rules, plan(**{**MESH, "n": n}), K) == want
+        assert spmm(rules, plan(**{**MESH, "entries": TINY - 1, "n": 140_000}), K) == ((4, 0) if K <= 16 else (4, 8) if K % 2 else (8, 0))
+        # long rows that are split, or rows that are not short: no mesh
+        for other in (dict(split=9), dict(row_task=40)):
+            assert spmm(rules, plan(**{**MESH, **other}), K) == ((4, 0) if K <= 16 else (8, 0))
+        assert spmm(rules, plan(**{**small, "split": 9, "row_task": 60}), K) == ((4, 0) if K <= 16 else (4, 8))
+    for K in (40, 48, 56, 64):
+        assert spmm(rules, plan(**MESH), K) == (8, 0) and spmm(rules, plan(**MESH), K, aligned=False) == (4, 0)
+        assert spmm(rules, plan(**MESH), K + 4 if K < 64 else 60) == (4, 0)
+        # no cut row (an even graph of short tasks, whatever its longest row), few entries, far past the caches
+        for other in (dict(cut=0), dict(cut=0, even=1, task=16), dict(entries=(1 << 18) - 1), dict(n=100_000_000 // K + 1)):
+            assert spmm(rules, plan(**{**MESH, **other}), K) == (4, 0)
+        assert spmm(rules, plan(**{**MESH, "n": 99_999_999 // K}), K) == (8, 0)

@@ -232,6 +232,9 @@ inline bool short_rows(const DevicePlan& p) {
 
 // Even rows, none of them cut into pieces.
 inline bool uncut(const DevicePlan& p) { return p.even_rows && p.nfixups + p.nwfixups == 0 && p.x_ntasks == 0; }
+// Short rows and a few long ones that are cut into pieces.
+inline bool mesh(const DevicePlan& p) { return p.row_task <= 32 && p.nfixups + p.nwfixups > 0 && p.x_ntasks == 0; }
+
 // The route of an SpMM (aligned: rows of B on the 16-byte grid).
 // wide loads only where they leave at least 4 lanes per group (whose column/value loads are
 // shared): with K <= 8 one or two lanes would stream a task alone (R-MAT K=8: 0.545 ms with one
@@ -251,9 +254,10 @@ inline bool uncut(const DevicePlan& p) { return p.even_rows && p.nfixups + p.nwf
 // 8-lane groups of 16-byte loads held to 2 waves (us, 16-byte / 8-byte, in batches of 8): R-MAT 2^20 K =
 // 33 595 / 442, 41 622 / 453, 48 507 / 372, 64 457 / 376; R-MAT 2^18 K = 40 / 48 / 56 / 64 120 / 120 / 127 / 112,
 // 110 / 110 / 115 / 109; R-MAT 2^14 K = 64 20.4 / 18.7; ER of 274K nodes K = 40 69.8 / 66.5; grid of 4M nodes
-// with hubs K = 64 587 / 564.  On the 16-byte grid the 16-byte loads stay where pieces of a few hub rows are
-// far longer than the packed tasks of a mesh and the operands fit the MALL: grid of 640K nodes (tasks of
-// 32, pieces of 128) K = 40 / 48 / 64 73 / 74 / 71, 79 / 85 / 85; with 2M nodes, past it, both the same.
+// with hubs K = 64 587 / 564.  On the 16-byte grid the 16-byte loads stay for a mesh whose pieces of a few hub rows are
+// far longer than its packed tasks, up to 200 MB of B (K = 40 / 48 / 64, 16-byte / 8-byte: grid of 300^2 nodes, 495K
+// entries 17.1 / 17.6 / 17.6, 19.4 / 19.2 / 19.9, of 640K nodes 73 / 74 / 71, 79 / 85 / 85; of 1300^2 nodes K = 48 / 64,
+// 162 / 216 MB 200 / 233, 225 / 217; of 145^2 nodes, 115K entries, K = 48 / 64 16.2 / 16.5, 15.6 / 15.8).
 // K = 5 and 7 stay on 8 lanes of 2 bytes over short rows (grid of 2M nodes K = 7: 109 us, 127 with 4-byte
 // loads; R-MAT, whose tasks are long, 336 / 262)
 inline Route spmm_route(const DevicePlan& p, int K, bool aligned) {
@@ -269,12 +273,28 @@ inline Route spmm_route(const DevicePlan& p, int K, bool aligned) {
     if (p.nnz_csr >= kTinyEntries && (int64_t)p.n * K * 2 >= 2'000'000) return {K <= 16 ? 1 : 2, 16};
     if (K > 16 && (K % 2 != 0 || p.nnz_csr < 1 << 18)) return {4, 8};
   }
+  if (any_lanes && K > 8 && K <= 32) {
+    // The smallest meshes, whose time is the chain of one hub row's pieces and their sum, take narrow loads in 16-lane
+    // groups (us, K = 9 / 16 / 17 / 24 / 31, 4-lane groups / this: grid of 120^2 nodes 13.7 / 13.9 / 17.2 / 15.3 / 17.6, 11.8
+    // / 11.9 / 12.6 / 12.6 / 13.0; of 200^2, 220K entries 10.9 / 10.6 / 13.5 / 11.8 / 13.7, 10.8 / 10.2 / 11.1 / 10.9 / 11.4;
+    // of 250^2, 344K 11.1 / 10.7 / 16.3 / 12.6 / 17.1, 13.3 / 12.2 / 14.1 / 12.8 / 14.6).  Off the 16-byte grid, 8-lane groups
+    // of 8-byte loads at odd widths of other tiny ones, and where B is past all L2s (32 MB) and within half the MALL
+    // (K = 17 / 28 / 31, 16 bytes / 8: 250^2 16.3 / 13.1 / 17.1, 13.6 / 12.8 / 13.6; 1300^2 169 / 187 / 227, 160 / 172 / 196;
+    // 800^2, K = 18 / 22 / 28, 23 / 28 / 36 MB 51 / 57 / 64, 56 / 59 / 62; 2048^2, K = 17 / 20 / 28, 143 .. 235 MB 405 / 381 /
+    // 465, 450 / 434 / 508).
+    if (mesh(p) && p.nnz_csr < 1 << 18) return {K <= 16 ? 1 : 2, 16};
+    const int64_t bytes = (int64_t)p.n * K * 2;
+    if (K > 16 && mesh(p) && ((K % 2 != 0 && p.nnz_csr < kTinyEntries) || (K % 8 != 0 && bytes >= 32 << 20 && bytes < 128 << 20)))
+      return {4, 8};
+    // Tiny plans with split rows are chains of few batches: more lanes with narrower loads (K = 17 / 24 / 32: R-MAT 2^14
+    // 22.1 / 19.9 / 20.0, 18.8 / 17.4 / 17.4; R-MAT 2^16 with 614K entries 28.8 / 24.8 / 24.8, 23.2 / 22.8 / 23.1).
+    if (K > 16 && p.x_ntasks > 0 && p.nnz_csr < kTinyEntries) return {4, 8};
+  }
   if (K <= 8) return {K > 4 && (K % 2 == 0 || p.task_nnz >= 64) ? 2 : 1, 0};
   if (K <= 16) return {4, 0};
   if (K <= 32) return {8, 0};
   if (K <= 64) {
-    const int64_t touched = p.nnz_csr * 6 + (int64_t)p.m * K * 4 + (int64_t)p.n * K * 2;
-    const bool hub_pieces = p.task_max > 3 * p.task_nnz && touched < 320'000'000;   // (past that, gathers wait on HBM)
+    const bool hub_pieces = mesh(p) && p.nnz_csr >= 1 << 18 && (int64_t)p.n * K * 2 < 200'000'000;
     return {aligned && K % 8 == 0 && hub_pieces ? 8 : 4, 0};
   }
   if (any_lanes && K % 4 == 0 && K % 8 != 0) {
