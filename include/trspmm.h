@@ -227,7 +227,10 @@ typedef struct trs_plan_options {
                              rows); 0 plain; -1 automatic (bit 1) */
   int32_t window_row_cap; /* longest residual row an MFMA window may carry before its tiles go
                              back to the residual path, when that row is also more than twice
-                             its window's mean residual row (0 = automatic: 128) */
+                             its window's mean residual row (0 = automatic: 128, and SpMM plans
+                             whose windows hold less than a sixteenth of the entries, and less than
+                             262,144, in their tiles keep none; a value > 0 asks for them all the
+                             same) */
   int32_t xcd_run;        /* workgroups are remapped so each of the 8 XCDs (own L2) runs this many
                              consecutive work items in a row; 1 = hardware round robin,
                              0 = automatic */

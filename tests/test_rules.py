@@ -22,6 +22,7 @@ def rules(tmp_path_factory):
     lib.rule_spmm_route.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]
     lib.rule_hot_bytes.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32]
     lib.rule_hot_bytes.restype = ctypes.c_int64
+    lib.rule_windows_pay.argtypes = [ctypes.c_int64, ctypes.c_int64]
     lib.rule_task_sizes.argtypes = [ctypes.c_int64, ctypes.c_int64] + [ctypes.c_int32] * 5 + [ctypes.c_void_p]
     return lib
 
@@ -169,3 +170,9 @@ def test_spmm_meshes_with_a_few_long_rows(rules):
         for other in (dict(cut=0), dict(cut=0, even=1, task=16), dict(entries=(1 << 18) - 1), dict(n=100_000_000 // K + 1)):
             assert spmm(rules, plan(**{**MESH, **other}), K) == (4, 0)
         assert spmm(rules, plan(**{**MESH, "n": 99_999_999 // K}), K) == (8, 0)
+
+
+def test_windows_with_few_entries_in_tiles_are_dropped(rules):
+    for tiles, entries, want in ((100, 1600, 1), (100, 1601, 0), (161, 491_520, 0), (16_384, 262_144, 1), ((1 << 18) - 1, 30_000_000, 0),
+                                 (1 << 18, 30_000_000, 1), (1_030_000, 19_000_000, 1)):
+        assert rules.rule_windows_pay(tiles, entries) == want, (tiles, entries)

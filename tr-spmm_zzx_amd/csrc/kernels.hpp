@@ -121,6 +121,18 @@ struct DevicePlan {
   int32_t out_off = 0;   // set in the view that writes xbuf: entry q writes out[q - out_off]
 };
 
+// Whether MFMA windows with `in_tiles` entries in their tiles, of `entries` in all, stay on MFMA: their launch, and
+// the residual rows of those windows, each walked by one lane group, cost 8 to 25 us a call whatever their number, and
+// an entry in a tile saves as little as 17 us a million at K = 32 and 40 at K = 128.  Kept minus dropped, us at K = 32 /
+// 64 / 128 / 256: R-MAT 2^14, 216 of 492K entries in tiles 17 / 18 / 24 / 27; blocks added to R-MAT 2^17, 145K of 3.1M
+// (4.6%) 20 / 19 / 20 / 19; to ER of 131,072 nodes, 62K of 2.3M (2.7%) 8 / 8 / 7 / 5, 128K of 2.4M (5.4%) 7 / 7 / 5 / 4, 671K
+// of 3.0M (23%) -3 / -1 / -14 / -32; of 524,288 nodes, 249K of 9.2M (2.7%) 0 / 2 / -4 / -15, 513K of 9.5M (5.4%) 4 / -2 /
+// -11 / -28; of 2^20 nodes, 498K of 18.4M (2.7%) -2 / - / -13 / -.  Block graphs hold 36% and more of theirs.
+constexpr int64_t kMinTileShare = 16, kEnoughTileEntries = 1 << 18;
+inline bool windows_pay(int64_t in_tiles, int64_t entries) {
+  return in_tiles >= kEnoughTileEntries || in_tiles * kMinTileShare >= entries;
+}
+
 // Sizes of residual tasks and pieces.
 // A plan of fewer entries than this is small: it splits rows over the XCDs from 512 entries on, not 256, and its
 // tasks and pieces shrink (see task_sizes).

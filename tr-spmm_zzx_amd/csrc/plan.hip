@@ -97,12 +97,6 @@ constexpr int32_t kWindowRowRatio = 2;
 // kept; the task kernel cuts those rows into pieces and XCD sub-rows instead).
 constexpr int64_t kWindowRowHardFactor = 4;
 
-// Windows stay on MFMA only where their tiles hold at least one in this many of all entries: fewer do
-// not pay for the window kernel's launch and for the windows' residual rows, which it walks with one
-// lane group each (R-MAT 2^14, 19 windows with 161 tile entries of 491K, K = 32 / 64 / 128: 43.3 / 45.8
-// / 58.2 -> 24.1 / 27.1 / 34.2 us; block graphs hold 36% and more of their entries in tiles).
-constexpr int64_t kMinTileShare = 16;
-
 // Hot-row staging (option hot_rows = 0): the kHotRows most gathered columns of the task kernels,
 // at most one in kHotColumnShare of all columns, and only when they take at least
 // kHotMinShare10 / 10 of the gathers.  R-MAT 2^20 (16,384 rows, 56.7% of the entries), K = 128:
@@ -1571,7 +1565,7 @@ Status finalize(Lowering& L, const trs_plan_options& opt, trs_plan** out, const 
       in_tiles += k;
       if (!demote[t.row0 / 16]) in_kept += k;
     }
-    if (opt.window_row_cap <= 0 && in_kept * kMinTileShare < total + in_tiles) {
+    if (opt.window_row_cap <= 0 && in_kept > 0 && !trs::windows_pay(in_kept, total + in_tiles)) {
       std::fill(demote.begin(), demote.end(), 1);
       any_demote = true;
     }
