@@ -176,3 +176,8 @@ def test_windows_with_few_entries_in_tiles_are_dropped(rules):
     for tiles, entries, want in ((100, 1600, 1), (100, 1601, 0), (161, 491_520, 0), (16_384, 262_144, 1), ((1 << 18) - 1, 30_000_000, 0),
                                  (1 << 18, 30_000_000, 1), (1_030_000, 19_000_000, 1)):
         assert rules.rule_windows_pay(tiles, entries) == want, (tiles, entries)
+
+
+def test_window_loads(rules):
+    want = {4: 1, 5: 2, 8: 2, 9: 4, 16: 4, 17: 8, 23: 8, 25: 4, 28: 8, 32: 8, 33: 4, 34: 8, 36: 4, 40: 8, 44: 4, 48: 8, 52: 8, 63: 4, 65: 8}
+    assert {K: rules.rule_window_vec(K) for K in want} == want

@@ -2125,13 +2125,12 @@ hipError_t launch_place_entries(const PlaceEntries& a, hipStream_t stream) {
 void launch_spmm_windows(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
                          hipStream_t stream) {
   if (p.nmwin <= 0) return;
-  // B rows are staged with 16-byte loads where the task kernel takes 8-byte ones (K = 40 / 50 / 64 on SBM of
-  // 250K nodes: 59 / 70 / 56 us, 62 / 74 / 65 with 8-byte loads), but for odd rows of about that width (K =
-  // 31 / 33 / 41: 57 / 65 / 69, 55 / 62 / 66)
-  if (K > 16 && !(K % 2 != 0 && K > 24 && K <= 64)) windows_width<8>(p, B, ldb, K, C, ldc, stream);
-  else if (K > 8) windows_width<4>(p, B, ldb, K, C, ldc, stream);
-  else if (K > 4) windows_width<2>(p, B, ldb, K, C, ldc, stream);
-  else windows_width<1>(p, B, ldb, K, C, ldc, stream);
+  switch (window_vec(K)) {
+    case 8: windows_width<8>(p, B, ldb, K, C, ldc, stream); break;
+    case 4: windows_width<4>(p, B, ldb, K, C, ldc, stream); break;
+    case 2: windows_width<2>(p, B, ldb, K, C, ldc, stream); break;
+    default: windows_width<1>(p, B, ldb, K, C, ldc, stream);
+  }
 }
 
 hipError_t launch_spmm(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,

@@ -219,6 +219,15 @@ inline TaskSizes task_sizes(int64_t entries, int64_t nonempty, int32_t longest, 
   return t;
 }
 
+// Features per load that stages B rows for the MFMA windows: 16 bytes from K = 17 on, also where the task kernel takes
+// 8-byte loads (K = 40 / 50 / 64 on SBM of 250K nodes: 59 / 70 / 56 us, 62 / 74 / 65 with 8-byte loads), but for odd rows
+// of about that width (K = 31 / 33 / 41: 57 / 65 / 69, 55 / 62 / 66) and rows of 33 to 48 features on the 8-byte grid only
+// (K = 28 / 36 / 44 / 52, SBM of 20,000 nodes 8.8 / 10.4 / 10.5 / 9.7, 9.1 / 9.2 / 9.3 / 10.4).
+inline int window_vec(int K) {
+  if (K > 16) return (K % 2 != 0 && K > 24 && K <= 64) || (K > 32 && K <= 48 && K % 8 == 4) ? 4 : 8;
+  return K > 8 ? 4 : K > 4 ? 2 : 1;
+}
+
 // How a width is run: features per lane (16-, 8-, 4- or 2-byte loads) and lanes per group (0: as many as the width
 // needs, at most 16 of 16-byte loads).
 struct Route { int vec, lanes; };
