@@ -104,7 +104,14 @@ def staged_row_bytes(K: int, sddmm: bool) -> int:
     divide stage padded to whole cache lines)."""
     if K % 8 == 0:
         return 2 * K if K >= 128 else 0
+    if not sddmm and 128 < K <= 256 and K % 4 == 0:   # one pass of 32 lanes
+        return 0
     return 2 * ((K + 63) // 64 * 64) if K >= (121 if sddmm else 65 if K % 2 else 104) else 0
+
+
+def sddmm_one_pass(n: int, K: int) -> bool:
+    """Whether a call on a plan with staged rows takes one pass of 32 lanes, which does not use them."""
+    return 128 < K <= 256 and n * K * 2 <= (128 if K % 8 == 0 else 64 if K % 2 == 0 else 16) << 20
 
 
 def dominant(kms) -> int:
@@ -307,9 +314,10 @@ def bench_sddmm(args, workload, g, K):
         nr = st["csr_nnz"]
         bytes_k = 8 * nr + 4 * (M + 1) + 2 * M * K + 2 * N * K
         impl = (4 * nr if st["mfma_tiles"] else 0) + 16 * st["tasks"]   # output index, task descriptors
-        hot_bytes = staged_row_bytes(K, True) * st["hot_rows"] if need else 0
-        impl += 2 * hot_bytes                                           # staged hot rows: read + write
-        impl += 3 * max(0, need - hot_bytes)                            # split-part merge: index, buffer, output (4 B each)
+        held = staged_row_bytes(K, True) * st["hot_rows"] if need else 0
+        one_pass = not args.feature_lanes and sddmm_one_pass(N, K)
+        impl += 0 if one_pass else 2 * held                             # staged hot rows: read + write
+        impl += 3 * max(0, need - held)                                 # split-part merge: index, buffer, output (4 B each)
     else:
         bytes_k = 8 * st["mfma_nnz"] + 2 * M * K + 2 * N * K
         impl = st["mfma_tiles"] * (64 + 1024) - 4 * st["mfma_nnz"]      # column ids, dense output slots

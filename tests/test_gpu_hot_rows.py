@@ -372,3 +372,23 @@ def test_hot_selection_at_the_edges_of_the_column_ranges(n):
     say("hot selection over", n, "columns")
     s = trspmm.Plan.from_format(f, m, n, mfma_tc=False, mfma_sptc=False, xcd_split=-1, hot_rows=100).stats()
     assert (s["hot_rows"], s["hot_entries"]) == _brute_force_hot(col, n, 100)
+
+
+@pytest.mark.parametrize("K, taken", [(128, False), (136, True), (200, True), (256, True), (264, False)])
+def test_sddmm_of_one_pass_takes_a_workspace_without_staged_rows(K, taken):
+    """K = 129 .. 256 in one pass stages nothing: a workspace of the split part's buffer is enough there, and too small
+    where rows are staged."""
+    g, f = rmat()
+    plan = trspmm.Plan.for_sddmm(f, g.m, g.n)
+    base = trspmm.Plan.for_sddmm(f, g.m, g.n, hot_rows=-1).sddmm_workspace_bytes(K)
+    assert plan.stats()["hot_rows"] > 0 and 0 < base < plan.sddmm_workspace_bytes(K)
+    X, Y = (torch.from_numpy(graphs.dense_operand(r, K, seed=K + i)).cuda() for i, r in enumerate((g.m, g.n)))
+    say("sddmm workspace", K)
+    out = torch.full((plan.stats()["nnz"],), float("nan"), device="cuda")
+    ws = torch.empty(base, dtype=torch.uint8, device="cuda")
+    rc = nat.lib().trs_sddmm_f16_ws(plan.handle, X.data_ptr(), K, Y.data_ptr(), K, K, out.data_ptr(), ws.data_ptr(), base,
+                                    int(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert rc == (0 if taken else 1)
+    if taken:
+        assert torch.equal(out, plan.sddmm(X, Y))

@@ -22,6 +22,7 @@ def rules(tmp_path_factory):
     lib.rule_spmm_route.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p]
     lib.rule_hot_bytes.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32]
     lib.rule_hot_bytes.restype = ctypes.c_int64
+    lib.rule_sddmm_one_pass.argtypes = [ctypes.c_void_p, ctypes.c_int32]
     lib.rule_windows_pay.argtypes = [ctypes.c_int64, ctypes.c_int64]
     lib.rule_task_sizes.argtypes = [ctypes.c_int64, ctypes.c_int64] + [ctypes.c_int32] * 5 + [ctypes.c_void_p]
     return lib
@@ -181,3 +182,17 @@ def test_windows_with_few_entries_in_tiles_are_dropped(rules):
 def test_window_loads(rules):
     want = {4: 1, 5: 2, 8: 2, 9: 4, 16: 4, 17: 8, 23: 8, 25: 4, 28: 8, 32: 8, 33: 4, 34: 8, 36: 4, 40: 8, 44: 4, 48: 8, 52: 8, 63: 4, 65: 8}
     assert {K: rules.rule_window_vec(K) for K in want} == want
+
+
+def test_sddmm_one_pass(rules):
+    one = lambda p, K: rules.rule_sddmm_one_pass(p, K) == 1
+    er = dict(entries=15_000_000, n=907_888, task=68, row_task=68, even=1)
+    for K in (129, 132, 200, 255, 256):
+        assert one(plan(**er), K) and not one(plan(**{**er, "lanes": 16}), K)
+        # staged rows or a split part: as long as Y comes from the caches
+        mb = 128 if K % 8 == 0 else 64 if K % 2 == 0 else 16
+        fits, past = (mb << 20) // (2 * K), (mb << 20) // (2 * K) + 1
+        for more in (dict(hot=100), dict(split=100)):
+            assert one(plan(**{**er, **more, "n": fits}), K) and not one(plan(**{**er, **more, "n": past}), K)
+    for K in (64, 128, 257, 384):
+        assert not one(plan(**er), K)

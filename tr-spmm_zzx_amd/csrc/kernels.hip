@@ -1504,16 +1504,9 @@ template <int VEC>
 hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx, const uint16_t* Y, int64_t ldy,
                             int K, float* out, uint16_t* hot, float* xbuf, hipStream_t s, hipEvent_t* ev) {
   if (ev) (void)hipEventRecord(ev[0], s);
-  // K = 129..256 in one pass of 32 lanes where the Y rows come from the caches anyway: the pass saves a
-  // launch, a walk of the entries and the outputs' read and write (us, two passes / one: ER of 6558 nodes K =
-  // 256 16.5 / 7.2, R-MAT 2^14 K = 200 47 / 36, R-MAT 2^16 K = 200 / 256 123 / 99, 108 / 99, R-MAT 2^18 400 /
-  // 331, 357 / 357).  Rows off the 16-byte grid gain from the staged rows of two passes sooner: even
-  // widths to 64 MB of Y (R-MAT 2^17 K = 222 174 / 149, 2^18 K = 130 308 / 344), odd ones to 16 MB (R-MAT
-  // 2^14 K = 145 45 / 44, 2^16 109 / 117).
-  const int64_t one_pass_y = (int64_t)(K % 8 == 0 ? 128 : K % 2 == 0 ? 64 : 16) << 20;
-  const bool one_pass = K <= 256 && (int64_t)p.n * K * 2 <= one_pass_y;
+  const bool one_pass = sddmm_one_pass(p, K);
   // staged hot Y rows (all K features, once per call) for the passes run by 16-lane groups
-  const bool hot_on = VEC == 8 && hot != nullptr && hot_buffer_bytes(p, K, true) > 0 && (K <= 128 || !one_pass);
+  const bool hot_on = VEC == 8 && hot != nullptr && hot_buffer_bytes(p, K, true) > 0 && !one_pass;
   const DevicePlan hp = hot_on ? hot_view(p, Y, ldy, K, hot, s) : p;
   // the split part writes its own buffer (then merged) where the workspace holds one
   bool merge_on = p.x_ntasks > 0 && xbuf != nullptr && merge_buffer_bytes(p, K) > 0;

@@ -348,6 +348,18 @@ inline bool stages_hot_rows(int K, bool sddmm) {
   if (K % 8 == 0) return K >= kHotMinK;
   return K >= (sddmm ? 121 : K % 2 != 0 ? 65 : 104);
 }
+// SDDMM K = 129..256 in one pass of 32 lanes where no long rows' columns are there to be read again from the L2s (no
+// split part, no staged rows), or the Y rows come from the caches anyway: the pass saves a launch, a walk of the
+// entries and the outputs' read and write (us, two passes / one: ER of 907,888 nodes K = 132 / 180 / 256 1283 / 1461 / 1235,
+// 871 / 1055 / 1137; of 150,000 nodes K = 228 159 / 116; grid of 1300^2 nodes K = 130 / 244 / 256 696 / 1041 / 765, 556 / 744 /
+// 706; SBM of 250,000 nodes K = 180 286 / 207; ER of 6558 nodes K = 256 16.5 / 7.2; R-MAT 2^14 K = 200 47 / 36, 2^16 K = 200
+// / 256 123 / 99, 108 / 99, 2^18 400 / 331, 357 / 357).  Rows off the 16-byte grid gain from the staged rows of two passes
+// sooner: even widths to 64 MB of Y (R-MAT 2^17 K = 222 174 / 149, 2^18 K = 130 308 / 344), odd ones to 16 MB (R-MAT 2^14 K =
+// 145 45 / 44, 2^16 109 / 117).  The staged rows serve two passes only.
+inline bool sddmm_one_pass(const DevicePlan& p, int K) {
+  if (K <= 128 || K > 256 || p.feature_lanes > 0) return false;
+  return unstaged(p) || (int64_t)p.n * K * 2 <= (int64_t)(K % 8 == 0 ? 128 : K % 2 == 0 ? 64 : 16) << 20;
+}
 inline int hot_row_stride(int K) { return K % 8 == 0 ? K : (K + 63) / 64 * 64; }
 // Bytes of the staged-row buffer of plan p at width K (0 when the plan or K does not stage).
 inline int64_t hot_buffer_bytes(const DevicePlan& p, int K, bool sddmm) {

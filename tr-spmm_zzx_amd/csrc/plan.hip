@@ -2527,7 +2527,8 @@ static int sddmm_impl(const trs_plan* p, const uint16_t* X, int64_t ldx, const u
     return report(fail(TRS_EINVAL, "trs_sddmm_f16: NULL operand or leading dimension < K"));
   if (ldy > INT32_MAX) return report(fail(TRS_ERANGE, "trs_sddmm_f16: leading dimension of Y beyond 2^31 - 1"));
   const int64_t full = trs_sddmm_workspace_bytes(p, K);
-  const int64_t need = staging_is_optional(K) ? trs::merge_buffer_bytes(p->dp, K) : full;
+  // (one pass stages no rows, whatever the size that trs_sddmm_workspace_bytes names)
+  const int64_t need = staging_is_optional(K) || trs::sddmm_one_pass(p->dp, K) ? trs::merge_buffer_bytes(p->dp, K) : full;
   if (ws && ws_bytes < need)
     return report(fail(TRS_EINVAL, "trs_sddmm_f16_ws: workspace smaller than trs_sddmm_workspace_bytes"));
   float* xbuf = ws && trs::merge_buffer_bytes(p->dp, K) > 0 ? static_cast<float*>(ws) : nullptr;
