@@ -34,6 +34,11 @@ void rule_spmm_route(const int64_t* f, int32_t K, int32_t aligned, int32_t* out)
 int64_t rule_hot_bytes(const int64_t* f, int32_t K, int32_t sddmm) { return trs::hot_buffer_bytes(plan_of(f), K, sddmm != 0); }
 int32_t rule_windows_pay(int64_t in_tiles, int64_t entries) { return trs::windows_pay(in_tiles, entries) ? 1 : 0; }
 int32_t rule_sddmm_one_pass(const int64_t* f, int32_t K) { return trs::sddmm_one_pass(plan_of(f), K) ? 1 : 0; }
+void rule_sddmm_route(const int64_t* f, int32_t K, int32_t* out) {
+  const trs::Route r = trs::sddmm_route(plan_of(f), K);
+  out[0] = r.vec;
+  out[1] = r.lanes;
+}
 int32_t rule_window_vec(int32_t K) { return trs::window_vec(K); }
 int32_t rule_counts_in_lds(int32_t n) { return trs::counts_in_lds(n) ? 1 : 0; }
 

@@ -62,3 +62,28 @@ def test_spmm_routes(name, off, pad):
         # sum is many times their spread
         assert np.max(np.abs(C - R)) <= 1e-5 * max(1.0, float(np.max(np.abs(R)))), (name, K)
         assert torch.all(full[:, :1] == 7.0) and torch.all(full[:, 1 + K:] == 7.0), (name, K)
+
+
+SDDMM_GRAPHS = {
+    # even rows, Y past the lines of the narrow routes
+    "even_wide_y": lambda: graphs.erdos_renyi_gcn(nodes=700_000, edges=700_000, seed=8),
+    "even": GRAPHS["even"],
+    # blocks: tiles whose widths 16 and 32 do not divide
+    "sbm": lambda: graphs.sbm(communities=64, seed=5, val_seed=6),
+}
+
+
+@pytest.mark.parametrize("off,pad", [(0, 0), (1, 1)])
+@pytest.mark.parametrize("name", list(SDDMM_GRAPHS))
+def test_sddmm_routes(name, off, pad):
+    g = SDDMM_GRAPHS[name]()
+    plan = trspmm.Plan.for_sddmm(trspmm.build_format_device(*(torch.from_numpy(a).cuda() for a in (g.rowptr, g.col, g.val))), g.m, g.n)
+    for K in (9, 12, 15, 16, 17, 24, 31, 32, 100, 124, 244):
+        print("sddmm route", name, K, off, pad, flush=True)
+        X, Xh = inside(g.m, K, off, pad, seed=K)
+        Y, Yh = inside(g.n, K, off, pad, seed=K + 1)
+        S = plan.sddmm(X, Y)
+        torch.cuda.synchronize()
+        R = osp.csr_sddmm(g.rowptr[: g.m + 1], g.col, Xh, Yh)
+        # per-entry dot of K fp16 products, fp32 accumulation
+        assert np.max(np.abs(S.cpu().numpy() - R)) <= (1e-5 * np.sqrt(K) * 4 + 1e-6) * max(1.0, float(np.max(np.abs(R)))), (name, K)

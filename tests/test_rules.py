@@ -23,6 +23,7 @@ def rules(tmp_path_factory):
     lib.rule_hot_bytes.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_int32]
     lib.rule_hot_bytes.restype = ctypes.c_int64
     lib.rule_sddmm_one_pass.argtypes = [ctypes.c_void_p, ctypes.c_int32]
+    lib.rule_sddmm_route.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p]
     lib.rule_windows_pay.argtypes = [ctypes.c_int64, ctypes.c_int64]
     lib.rule_task_sizes.argtypes = [ctypes.c_int64, ctypes.c_int64] + [ctypes.c_int32] * 5 + [ctypes.c_void_p]
     return lib
@@ -196,3 +197,19 @@ def test_sddmm_one_pass(rules):
             assert one(plan(**{**er, **more, "n": fits}), K) and not one(plan(**{**er, **more, "n": past}), K)
     for K in (64, 128, 257, 384):
         assert not one(plan(**er), K)
+
+
+def test_sddmm_routes(rules):
+    def route(K, **more):
+        out = (ctypes.c_int32 * 2)()
+        rules.rule_sddmm_route(plan(**{**dict(entries=15_000_000, n=907_888, task=68, row_task=68, even=1), **more}), K, out)
+        return tuple(out)
+
+    for K in (4, 8, 9, 15, 16, 17, 24, 31, 32, 33, 64, 65, 98, 100, 104, 124, 128, 132, 256):
+        plain = (1, 0) if K <= 8 else (2, 0) if K <= 16 else (4, 0) if K <= 64 else (8, 0)
+        wide = (4, 32) if K in (100, 124) else plain
+        assert route(K) == ((1, 16) if 8 < K <= 16 else (2, 16) if 16 < K <= 32 else wide)
+        assert route(K, n=11_999_999 // (2 * K) if K <= 16 else 5_999_999 // (2 * K)) == wide
+        assert route(K, entries=TINY - 1) == ((1, 16) if 8 < K <= 16 else plain)
+        for other in (dict(even=0), dict(split=4), dict(lanes=8)):
+            assert route(K, **other) == plain

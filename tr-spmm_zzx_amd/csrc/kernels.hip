@@ -1502,7 +1502,7 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
 
 template <int VEC>
 hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx, const uint16_t* Y, int64_t ldy,
-                            int K, float* out, uint16_t* hot, float* xbuf, hipStream_t s, hipEvent_t* ev) {
+                            int K, float* out, uint16_t* hot, float* xbuf, int lanes, hipStream_t s, hipEvent_t* ev) {
   if (ev) (void)hipEventRecord(ev[0], s);
   const bool one_pass = sddmm_one_pass(p, K);
   // staged hot Y rows (all K features, once per call) for the passes run by 16-lane groups
@@ -1521,7 +1521,7 @@ hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx,
     const uint16_t* Yp = Y + f0;
     const int acc = f0 > 0 ? 1 : 0;
     DevicePlan pp = p;
-    int lpg = lanes_for(Kp, VEC);
+    int lpg = lanes > 0 ? lanes : lanes_for(Kp, VEC);
     // a plan may ask for fewer lanes: the kernel then loops over feature chunks per batch
     while (p.feature_lanes > 0 && lpg > p.feature_lanes && lpg > 1) lpg >>= 1;
     // at least 8 lanes, so that a group writes 8 consecutive sums (32 bytes) per store and the
@@ -1588,11 +1588,11 @@ hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx,
       TRS_SD_U(L, 8)                                                                                       \
     }                                                                                                      \
     break;
-    // loads narrower than 16 bytes serve K <= 64, at most 16 lanes of 8 bytes, 8 of 4 or 2 bytes
+    // loads narrower than 16 bytes: groups of 8 or 16 lanes, of 8-byte ones to 32
     if constexpr (VEC < 4) {
-      switch (lpg) { TRS_SD(1) TRS_SD(2) TRS_SD(4) TRS_SD(8) }
-    } else if constexpr (VEC < 8) {
       switch (lpg) { TRS_SD(1) TRS_SD(2) TRS_SD(4) TRS_SD(8) TRS_SD(16) }
+    } else if constexpr (VEC < 8) {
+      switch (lpg) { TRS_SD(1) TRS_SD(2) TRS_SD(4) TRS_SD(8) TRS_SD(16) TRS_SD(32) }
     } else {
       switch (lpg) { TRS_SD(1) TRS_SD(2) TRS_SD(4) TRS_SD(8) TRS_SD(16) TRS_SD(32) TRS_SD(64) }
     }
@@ -1984,7 +1984,7 @@ template <int VEC>
 void windows_width(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc, hipStream_t s);
 template <int VEC>
 hipError_t sddmm_width(const DevicePlan& p, const uint16_t* X, int64_t ldx, const uint16_t* Y, int64_t ldy, int K,
-                       float* out, uint16_t* hot, float* xbuf, hipStream_t s, hipEvent_t* ev);
+                       float* out, uint16_t* hot, float* xbuf, int lanes, hipStream_t s, hipEvent_t* ev);
 #if TRS_KERNEL_PART > 0
 template <int VEC>
 hipError_t spmm_width(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, float* C, int64_t ldc,
@@ -1997,8 +1997,8 @@ void windows_width(const DevicePlan& p, const uint16_t* B, int64_t ldb, int K, f
 }
 template <int VEC>
 hipError_t sddmm_width(const DevicePlan& p, const uint16_t* X, int64_t ldx, const uint16_t* Y, int64_t ldy, int K,
-                       float* out, uint16_t* hot, float* xbuf, hipStream_t s, hipEvent_t* ev) {
-  return launch_sddmm_vec<VEC>(p, X, ldx, Y, ldy, K, out, hot, xbuf, s, ev);
+                       float* out, uint16_t* hot, float* xbuf, int lanes, hipStream_t s, hipEvent_t* ev) {
+  return launch_sddmm_vec<VEC>(p, X, ldx, Y, ldy, K, out, hot, xbuf, lanes, s, ev);
 }
 #endif
 #define TRS_WIDTH_INSTANCES(PREFIX, V)                                                                       \
@@ -2007,7 +2007,7 @@ hipError_t sddmm_width(const DevicePlan& p, const uint16_t* X, int64_t ldx, cons
   PREFIX template void windows_width<V>(const DevicePlan&, const uint16_t*, int64_t, int, float*, int64_t,    \
                                         hipStream_t);                                                         \
   PREFIX template hipError_t sddmm_width<V>(const DevicePlan&, const uint16_t*, int64_t, const uint16_t*,     \
-                                            int64_t, int, float*, uint16_t*, float*, hipStream_t, hipEvent_t*);
+                                            int64_t, int, float*, uint16_t*, float*, int, hipStream_t, hipEvent_t*);
 #if TRS_KERNEL_PART > 0
 TRS_WIDTH_INSTANCES(, TRS_KERNEL_PART)
 #else
@@ -2139,23 +2139,12 @@ hipError_t launch_spmm(const DevicePlan& p, const uint16_t* B, int64_t ldb, int 
 
 hipError_t launch_sddmm(const DevicePlan& p, const uint16_t* X, int64_t ldx, const uint16_t* Y, int64_t ldy,
                         int K, float* out, uint16_t* hot, float* xbuf, hipStream_t stream, hipEvent_t* ev) {
-  // K <= 8 takes 2-byte loads so that K lanes share a task (R-MAT K=8: 0.747 ms with one lane of
-  // 16-byte loads per task, 0.331), and up to K=64 8-byte loads are faster than 16-byte ones
-  // (same-box A/B on R-MAT: K=32 0.468 -> 0.430 ms, K=64 0.550 -> 0.503; K=128 1.038 vs 1.080
-  // with 8-byte loads, so 16-byte loads from K=72 on)
-  // Load width by K alone, as in launch_spmm: 8 lanes of 2 bytes to K = 8 and of 4 bytes to K = 16
-  // (outputs in 32-byte runs; R-MAT 2^20 K = 16 0.418 -> 0.334 ms, K = 12 0.408 -> 0.287), 8-byte loads
-  // to K = 64 (K = 32 0.468 -> 0.430 against 16-byte loads, K = 64 0.550 -> 0.503; K = 33 598 / 605 us, 52
-  // 477 / 582), 16-byte loads above.  With narrower loads for the widths that the vector does not
-  // divide the pattern took (us, narrow -> this): K = 9 393 -> 293, 13 396 -> 303, 17 706 -> 356, 31 712 ->
-  // 404, 33 702 -> 508, 63 1447 -> 567, 65 1173 -> 724, 97 2003 -> 779, 98 1508 -> 753, 100 905 -> 753,
-  // 127 2058 -> 944, 130 1657 -> 1484, 255 3692 -> 1809.
-  const bool v8 = K > 64, v4 = K > 16, v2 = K > 8;
+  const Route r = sddmm_route(p, K);
   if (hot != nullptr && !aligned16(hot)) hot = nullptr;
-  return v8 ? sddmm_width<8>(p, X, ldx, Y, ldy, K, out, hot, xbuf, stream, ev)
-       : v4 ? sddmm_width<4>(p, X, ldx, Y, ldy, K, out, nullptr, xbuf, stream, ev)
-       : v2 ? sddmm_width<2>(p, X, ldx, Y, ldy, K, out, nullptr, xbuf, stream, ev)
-            : sddmm_width<1>(p, X, ldx, Y, ldy, K, out, nullptr, xbuf, stream, ev);
+  return r.vec == 8 ? sddmm_width<8>(p, X, ldx, Y, ldy, K, out, hot, xbuf, r.lanes, stream, ev)
+       : r.vec == 4 ? sddmm_width<4>(p, X, ldx, Y, ldy, K, out, nullptr, xbuf, r.lanes, stream, ev)
+       : r.vec == 2 ? sddmm_width<2>(p, X, ldx, Y, ldy, K, out, nullptr, xbuf, r.lanes, stream, ev)
+                    : sddmm_width<1>(p, X, ldx, Y, ldy, K, out, nullptr, xbuf, r.lanes, stream, ev);
 }
 #endif  // TRS_KERNEL_PART == 0
 

@@ -327,6 +327,34 @@ inline Route spmm_route(const DevicePlan& p, int K, bool aligned) {
   return {8, 0};
 }
 
+// The route of an SDDMM.
+// K <= 8 takes 2-byte loads so that K lanes share a task (R-MAT K=8: 0.747 ms with one lane of
+// 16-byte loads per task, 0.331), and up to K=64 8-byte loads are faster than 16-byte ones
+// (same-box A/B on R-MAT: K=32 0.468 -> 0.430 ms, K=64 0.550 -> 0.503; K=128 1.038 vs 1.080
+// with 8-byte loads, so 16-byte loads from K=72 on)
+// Load width by K alone, as in launch_spmm: 8 lanes of 2 bytes to K = 8 and of 4 bytes to K = 16
+// (outputs in 32-byte runs; R-MAT 2^20 K = 16 0.418 -> 0.334 ms, K = 12 0.408 -> 0.287), 8-byte loads
+// to K = 64 (K = 32 0.468 -> 0.430 against 16-byte loads, K = 64 0.550 -> 0.503; K = 33 598 / 605 us, 52
+// 477 / 582), 16-byte loads above.  With narrower loads for the widths that the vector does not
+// divide the pattern took (us, narrow -> this): K = 9 393 -> 293, 13 396 -> 303, 17 706 -> 356, 31 712 ->
+// 404, 33 702 -> 508, 63 1447 -> 567, 65 1173 -> 724, 97 2003 -> 779, 98 1508 -> 753, 100 905 -> 753,
+// 127 2058 -> 944, 130 1657 -> 1484, 255 3692 -> 1809.
+// Even rows take narrower loads in more lanes where the gathers miss: 2-byte loads in 16 lanes at K = 9 .. 16 past 12 MB of
+// Y, 4-byte ones at K = 17 .. 32 past 6 MB (us, 8 lanes of 4 or 8 bytes / this: ER of 907,888 nodes K = 9 / 15 / 18 / 24 / 32
+// 321 / 376 / 378 / 404 / 352, 290 / 340 / 355 / 370 / 323; of 200,000 nodes K = 18 / 24 / 31 70 / 70 / 88, 65 / 67 / 80; of
+// 500,000 nodes K = 9 / 15, 9 / 15 MB 92 / 106, 97 / 103; of 142,496 nodes K = 18 / 22, 5.1 / 6.3 MB 44 / 47, 45 / 47), and 8-byte
+// ones in 32 lanes at K = 100 .. 124, which need no masks of a ragged tail, but for tiny plans (ER of 907,888 nodes K = 108
+// 765 / 737, of 349,663 K = 124 212 / 205, of 60,000 46.1 / 46.7, of 28,439 23.4 / 24.9).
+inline Route sddmm_route(const DevicePlan& p, int K) {
+  const int64_t bytes = (int64_t)p.n * K * 2;
+  const bool even = p.even_rows && p.x_ntasks == 0 && p.feature_lanes <= 0;
+  if (K <= 8) return {1, 0};
+  if (K <= 16) return even && bytes >= 12'000'000 ? Route{1, 16} : Route{2, 0};
+  if (K <= 32) return even && p.nnz_csr >= kTinyEntries && bytes >= 6'000'000 ? Route{2, 16} : Route{4, 0};
+  if (K <= 64) return {4, 0};
+  return even && p.nnz_csr >= kTinyEntries && K > 96 && K <= 128 && K % 8 == 4 ? Route{4, 32} : Route{8, 0};
+}
+
 // Hot-row staging applies to 16-byte gathers of at least this many features (one 16-lane group,
 // 256-byte rows: R-MAT 2^20 K = 128 -6%, K = 256 -5%; K = 32 and 64 unchanged or slower).
 constexpr int kHotMinK = 128;
