@@ -23,7 +23,7 @@
 //                   accumulated over K with gfx950's v_mfma_f32_16x16x32_f16 (both operands
 //                   contiguous in K, 16-byte loads straight from global), sampled at the tile's
 //                   stored entries; k_sddmm_mfma is the same with v_mfma_f32_16x16x16_f16 for
-//                   K < 8.
+//                   K < 16 (K = 8 aside).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -1213,8 +1213,8 @@ __global__ __launch_bounds__(256) void k_sddmm_mfma(DevicePlan P, const uint16_t
   }
 }
 
-// SDDMM over dense tiles with gfx950's v_mfma_f32_16x16x32_f16, K >= 8 and rows of any alignment: lane l supplies 8 consecutive features (one 16-byte load) of X row row0 + l % 16 as A and of
-// Y row col_{l % 16} as B, for the feature group 8 (l / 16) of each 32-feature step.  A and B use
+// SDDMM over dense tiles with gfx950's v_mfma_f32_16x16x32_f16, K >= 8 and rows of any alignment: lane l
+// supplies 8 consecutive features (one 16-byte load) of X row row0 + l % 16 as A and of Y row col_{l % 16} as B, for the feature group 8 (l / 16) of each 32-feature step.  A and B use
 // the same lane/element -> feature assignment, so D[r][c] = X[r] . Y[c] whatever order the
 // instruction sums its 32 products in.  The loads of up to 4 steps (128 features) are issued
 // before their MFMAs.  Features past K read feature 0 and are zeroed in both operands; the lane at the end of a
@@ -1650,7 +1650,9 @@ hipError_t launch_sddmm_vec(const DevicePlan& p, const uint16_t* X, int64_t ldx,
   if (p.ntiles > 0 && p.tile_pos) {
     const bool v4 = K % 4 == 0 && ldx % 4 == 0 && ldy % 4 == 0 && (reinterpret_cast<uintptr_t>(X) & 7) == 0 &&
                     (reinterpret_cast<uintptr_t>(Y) & 7) == 0;
-    const bool v8 = K >= 8;
+    // a step of 32 features, half idle, does not pay for its masks below K = 16 (SBM of 700,000 nodes, whole call, K = 9 / 11 /
+    // 15 268 / 278 / 299 us with steps of 16, 292 / 303 / 320 with one of 32)
+    const bool v8 = K == 8 || K >= 16;
     dim3 grid((p.ntiles + 3) / 4);
     // 16x16x32 with 16-byte loads issued ahead (same-box A/B on SBM 1M: K=128 0.174 -> 0.116 ms,
     // K=256 0.314 -> 0.205 ms; K=32 unchanged)
