@@ -1129,8 +1129,12 @@ __device__ __forceinline__ void sddmm_tasks_run(const DevicePlan& P, int block, 
 
 // Main part (Pm, the first gm workgroups, into out_m) and split part (Px, the rest, into out_x) in
 // one launch, as k_spmm_tasks (gm a multiple of kXcds where a split part follows).
+// Waves per SIMD that the registers must leave room for: the ragged form of 8-byte loads in 8-lane groups takes 130
+// registers by itself, which is 3 waves where the form of whole vectors has 4 (3 / 4 waves: SBM of 100,000 nodes K = 18 47.5 /
+// 36.9 us, R-MAT 2^18 with 3.9M entries K = 22 67.9 / 60.8, grid of 1300^2 nodes K = 17 141 / 128).
+constexpr int sddmm_min_waves(int vec, int lpg, int u, bool rag) { return vec == 4 && lpg == 8 && u == 8 && rag ? 4 : 1; }
 template <int VEC, int LPG, int U, bool LS, bool SPF, bool NTO, bool HOT, bool RAG>
-__global__ __launch_bounds__(256) void k_sddmm_tasks(DevicePlan Pm, DevicePlan Px, int gm,
+__global__ __launch_bounds__(256, sddmm_min_waves(VEC, LPG, U, RAG)) void k_sddmm_tasks(DevicePlan Pm, DevicePlan Px, int gm,
                                                      const uint16_t* __restrict__ X, int64_t ldx,
                                                      const uint16_t* __restrict__ Y, int64_t ldy, int K,
                                                      float* __restrict__ out_m, float* __restrict__ out_x, int acc) {
