@@ -171,10 +171,11 @@ def test_noalloc_with_staged_rows():
         assert np.array_equal(C.cpu().numpy(), run_spmm(p, Bh))
 
 
-@pytest.mark.parametrize("K", [128, 256, 200, 64, 136, 264])
+@pytest.mark.parametrize("K", [128, 256, 200, 64, 136, 264, 384])
 def test_sddmm_staged_equals_unstaged(K):
-    """K = 136 and 264 end in a feature pass of 8 features (under 16 lanes), which reads the plain
-    column ids while the earlier passes read the staged rows, accumulating into the same outputs."""
+    """K = 264 ends in a feature pass of 8 features (under 16 lanes), which reads the plain column ids while the
+    earlier passes read the staged rows, accumulating into the same outputs; K = 384 has three staged passes.  K = 136,
+    200 and 256 take one pass here (Y within 128 MB), which stages nothing, whatever the workspace holds."""
     g, f = rmat()
     hot = trspmm.Plan.for_sddmm(f, g.m, g.n)
     plain = trspmm.Plan.for_sddmm(f, g.m, g.n, hot_rows=-1)
@@ -392,3 +393,24 @@ def test_sddmm_of_one_pass_takes_a_workspace_without_staged_rows(K, taken):
     assert rc == (0 if taken else 1)
     if taken:
         assert torch.equal(out, plan.sddmm(X, Y))
+
+
+@pytest.mark.parametrize("K", [122, 127])
+def test_sddmm_ragged_staged_rows(K):
+    """K = 121 .. 127 stage padded rows from 48 MB of Y on: the same bits as without, and the oracle's values."""
+    rng = np.random.default_rng(K)
+    m, n = 1024, 220_000
+    rows = [np.unique(np.concatenate([rng.integers(0, n, 80), rng.integers(0, 60, 30)])) for _ in range(m)]
+    rowptr = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    col = np.concatenate(rows).astype(np.int32)
+    f = trspmm.build_format(rowptr, col, np.ones(len(col), np.float32))
+    hot, plain = (trspmm.Plan.for_sddmm(f, m, n, mfma_tc=False, mfma_sptc=False, hot_rows=h) for h in (100, -1))
+    assert hot.stats()["hot_rows"] > 0 and hot.sddmm_workspace_bytes(K) > plain.sddmm_workspace_bytes(K)
+    say("ragged staged sddmm", K)
+    Xh, Yh = graphs.dense_operand(m, K, seed=K), graphs.dense_operand(n, K, seed=K + 1)
+    X, Y = torch.from_numpy(Xh).cuda(), torch.from_numpy(Yh).cuda()
+    S = hot.sddmm(X, Y)
+    assert torch.equal(S, plain.sddmm(X, Y))
+    R = osp.csr_sddmm(rowptr, col, Xh, Yh)
+    tol = (1e-5 * np.sqrt(K) * 4 + 1e-6) * max(1.0, float(np.max(np.abs(R))))
+    assert np.max(np.abs(S.cpu().numpy() - R)) <= tol

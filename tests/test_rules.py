@@ -213,3 +213,11 @@ def test_sddmm_routes(rules):
         assert route(K, entries=TINY - 1) == ((1, 16) if 8 < K <= 16 else plain)
         for other in (dict(even=0), dict(split=4), dict(lanes=8)):
             assert route(K, **other) == plain
+
+
+def test_ragged_sddmm_rows_are_staged_past_48_mb(rules):
+    for K in (121, 124, 127):
+        fits, past = (48 << 20) // (2 * K), (48 << 20) // (2 * K) + 1
+        assert rules.rule_hot_bytes(plan(**{**RMAT, "n": fits - 1}), K, 1) == 0
+        assert rules.rule_hot_bytes(plan(**{**RMAT, "n": past}), K, 1) == 16384 * 128 * 2
+    assert rules.rule_hot_bytes(plan(**{**RMAT, "n": 4096}), 128, 1) == 16384 * 128 * 2

@@ -393,6 +393,9 @@ inline int hot_row_stride(int K) { return K % 8 == 0 ? K : (K + 63) / 64 * 64; }
 inline int64_t hot_buffer_bytes(const DevicePlan& p, int K, bool sddmm) {
   if (p.nhot <= 0 || !stages_hot_rows(K, sddmm)) return 0;
   if (!sddmm && p.feature_lanes <= 0 && spmm_one_pass(K)) return 0;
+  // (K = 121 .. 127: the copy and the renumbered walk pay once Y is past the L2s' reach, 48 MB: unstaged -> staged, R-MAT
+  // 2^16 with 614K entries K = 124 / 127 26 -> 31, 28 -> 32; 2^17, 33 MB, 84 -> 95, 90 -> 98; 2^18, 66 MB, K = 127 143 -> 123)
+  if (sddmm && K % 8 != 0 && K <= 128 && (int64_t)p.n * K * 2 < 48 << 20) return 0;
   return (int64_t)p.nhot * hot_row_stride(K) * 2;
 }
 // Column histogram of col[0, total) into counts[n] (ids outside [0, n) are skipped), counted in
