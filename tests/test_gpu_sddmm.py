@@ -68,9 +68,10 @@ def test_sddmm_long_rows_and_empty_rows(K):
     assert np.max(np.abs(out.cpu().numpy() - R)) < 1e-3
 
 
-@pytest.mark.parametrize("K", [72, 128, 256])
+@pytest.mark.parametrize("K", [72, 128, 256, 384])
 def test_staged_and_unstaged_sddmm_agree(K):
-    """16-lane groups (K = 65..128, and each 128-feature pass of K = 256) stage each task's column
+    """16-lane groups (K = 65..128, and each 128-feature pass of K = 384; K = 256 takes one pass of 32 lanes here,
+    which does not stage) stage each task's column
     ids in LDS (16-byte chunks from an 8-entry-aligned base).  Tasks here start at every offset mod 8 and hold
     up to 256 entries (rows of 100-256 entries, split rows beyond): staged and unstaged
     (stage = -1) plans against the closed form, and bitwise equal to each other (same summation
@@ -289,12 +290,13 @@ def test_sddmm_xcd_column_split_is_bitwise_equal():
     assert np.max(np.abs(outs[1].cpu().numpy() - R)) <= (1e-5 * np.sqrt(128) * 4 + 1e-6) * max(1.0, np.max(np.abs(R)))
 
 
-@pytest.mark.parametrize("K", [128, 136, 200, 256])
+@pytest.mark.parametrize("K", [128, 136, 200, 256, 257, 264, 384])
 def test_sddmm_split_part_merged_equals_in_place(K):
     """From K = 128 an SDDMM call with a workspace writes its split part (XCD sub-rows of the long
     rows) into a buffer of its own and merges the split rows' outputs into place afterwards; the
     call without a workspace writes them in place.  Same dot products, same outputs bitwise, and
-    against the closed form; both lowerings; feature passes (K > 128) accumulate in the buffer."""
+    against the closed form; both lowerings; the feature passes of K > 256 accumulate in the buffer (K = 136, 200 and
+    256 take one pass here)."""
     print("sddmm merge", K, flush=True)
     g = graphs.rmat(scale=16, edge_factor=16, seed=21)
     f = trspmm.build_format(g.rowptr, g.col, g.val)
