@@ -167,9 +167,9 @@ struct TaskSizes {
 // / 26.8; ER of 60,000 nodes, 1.0M, K = 32 / 64 / 128 / 256, of 48 18.3 / 22.5 / 39.8 / 71.8, of 62 20.7 / 26.1 /
 // 35.6 / 68.9).
 // SDDMM lane groups of 16 lanes take larger tasks than narrower ones (no row is written per task), which walk a list
-// of their own: tiny plans 16,384 tasks, in steps of 4 (17 entries are three batches of 8, 16 two: ER of 40,000 nodes,
-// 280K, K = 16 8.8, 7.6) (R-MAT 2^14, K = 48 / 64, tasks of 16 19.3 / 19.6, of 30 17.1 / 17.6; ER of
-// 42,440 nodes, 552K, 19.3 / 19.2, of 33 17.8 / 17.9), small ones 64 (R-MAT 2^16 with 983K entries K = 64 / 128 / 200:
+// of their own: tiny plans 16,384 tasks (R-MAT 2^14, K = 48 / 64, tasks of 16 19.3 / 19.6, of 30 17.1 / 17.6; ER of
+// 42,440 nodes, 552K, 19.3 / 19.2, of 33 17.8 / 17.9; not 17 to 19, three batches of 8 where 16 are two: ER of 40,000 nodes,
+// 280K, K = 16 8.8, 7.6), small ones 64 (R-MAT 2^16 with 983K entries K = 64 / 128 / 200:
 // of 32 25.2 / 41.9 / 82.5, of 64 26.6 / 36.1 / 78.4); K <= 32 those of SpMM, even tiny plans at most 24 (ER of 28,439
 // nodes K = 16 / 32, of 16 9.7 / 10.8, 22 8.0 / 8.5, 30 9.6 / 9.9; of 60,000 nodes, 10 a row 12.3 / 14.2, 11.9 / 13.7,
 // 11.2 / 14.0, of 45 13.2 / 18.1).  With a split part that is for those who walk whole rows, K < 128; K >=
@@ -191,7 +191,8 @@ inline TaskSizes task_sizes(int64_t entries, int64_t nonempty, int32_t longest, 
   t.task = t.narrow = task_opt > 0 ? task_opt : t.row_task;
   if (task_opt <= 0 && small) {
     const int64_t least = tiny ? 16 : 32, uneven = entries / kMinTasksUneven;
-    const int64_t shared = spmm ? entries / kMinTasks : entries / kMinTasks / 4 * 4;
+    int64_t shared = entries / kMinTasks;
+    if (!spmm && shared < 20) shared = 16;
     t.narrow = at_most(t.even && (spmm || tiny) ? (shared > least ? shared : least) : uneven > least ? uneven : least,
                        t.row_task);
     if (!spmm && tiny && t.narrow > 16) t.narrow = t.narrow < 24 ? 16 : 24;
@@ -408,14 +409,15 @@ constexpr int32_t kCountSpan = 32768;
 constexpr int kCountRanges = 32;
 inline bool counts_in_lds(int32_t n) { return n <= kCountSpan * kCountRanges; }
 // Copies for a list of `total` entries over n columns counted in LDS: a workgroup to every CU, of at least
-// 8192 entries each, within a buffer of 2 MB, or of 8 copies where that is more (16 past 2^16 columns).  The
+// 8192 entries each, within a buffer of 1.75 MB, or of 8 copies where that is more (16 past 2^16 columns).  The
 // kernel alone would take more copies, but the buffer lives for one plan, and what it costs to get and to give
 // back more than that is not won back (us per plan, 73 / 8 copies: ER of 60,000 nodes 1340 / 1016; 120 / 9,
 // grid of 223^2 nodes with hubs 1096 / 782, and 280 of the next format build; 128 / 8, R-MAT 2^16 2430 / 2133;
-// 32 / 16 / 8, ER of 250,000 nodes 2305 / 2331 / 2657).
+// 32 / 16 / 8, ER of 250,000 nodes 2305 / 2331 / 2657; 2 MB itself is where the steps begin: ER of 16,384 nodes, format,
+// plan and product, 32 / 16 copies 2027 / 1282).
 inline int lds_count_copies(int64_t total, int32_t n) {
   const int64_t ranges = (n + kCountSpan - 1) / kCountSpan;
-  const int64_t held = (int64_t)(2 << 20) / ((int64_t)n * 4), least = n > 1 << 16 ? 16 : 8;
+  const int64_t held = (int64_t)(7 << 18) / ((int64_t)n * 4), least = n > 1 << 16 ? 16 : 8;
   int64_t copies = held > least ? held : least;
   if (copies > 256 / ranges) copies = 256 / ranges;
   const int64_t fit = total / 8192;
