@@ -39,6 +39,7 @@ void rule_sddmm_route(const int64_t* f, int32_t K, int32_t* out) {
   out[0] = r.vec;
   out[1] = r.lanes;
 }
+uint32_t rule_entry_ahead(uint32_t p0, int32_t k, int32_t lane, uint32_t e) { return trs::entry_ahead(p0, k, lane, e); }
 int32_t rule_window_vec(int32_t K) { return trs::window_vec(K); }
 int32_t rule_counts_in_lds(int32_t n) { return trs::counts_in_lds(n) ? 1 : 0; }
 

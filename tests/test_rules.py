@@ -24,6 +24,8 @@ def rules(tmp_path_factory):
     lib.rule_hot_bytes.restype = ctypes.c_int64
     lib.rule_sddmm_one_pass.argtypes = [ctypes.c_void_p, ctypes.c_int32]
     lib.rule_sddmm_route.argtypes = [ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p]
+    lib.rule_entry_ahead.argtypes = [ctypes.c_uint32, ctypes.c_int32, ctypes.c_int32, ctypes.c_uint32]
+    lib.rule_entry_ahead.restype = ctypes.c_uint32
     lib.rule_windows_pay.argtypes = [ctypes.c_int64, ctypes.c_int64]
     lib.rule_task_sizes.argtypes = [ctypes.c_int64, ctypes.c_int64] + [ctypes.c_int32] * 5 + [ctypes.c_void_p]
     return lib
@@ -221,3 +223,12 @@ def test_ragged_sddmm_rows_are_staged_past_48_mb(rules):
         assert rules.rule_hot_bytes(plan(**{**RMAT, "n": fits - 1}), K, 1) == 0
         assert rules.rule_hot_bytes(plan(**{**RMAT, "n": past}), K, 1) == 16384 * 128 * 2
     assert rules.rule_hot_bytes(plan(**{**RMAT, "n": 4096}), 128, 1) == 16384 * 128 * 2
+
+
+@pytest.mark.parametrize("e", [1, 64, 513, (1 << 31) - 1])
+def test_entries_ahead_stay_in_the_row(rules, e):
+    """Also where the last row ends at the 2^31 - 1 entries that a plan may hold."""
+    for p0 in (max(e - 700, 0), max(e - 65, 0), e - 1):
+        for k in range(8):
+            for lane in (0, 63):
+                assert rules.rule_entry_ahead(p0, k, lane, e) == min(p0 + 64 * k + lane, e - 1)

@@ -1433,7 +1433,7 @@ hipError_t launch_spmm_vec(const DevicePlan& p, const uint16_t* B, int64_t ldb, 
     // capped (R-MAT K=128 with 2 entries per batch at 5 / 4 / 3 waves: 0.970 / 0.985 / 1.147 ms,
     // K=256 at 8 / 3 waves: 2.24 / 3.49; with 4 entries per batch, capped at 3 or 4 waves: slower
     // than uncapped at K = 128 and 256)
-    // (2-byte loads, used for K <= 8 and odd widths, stay uncapped: R-MAT K=8 0.293 ms uncapped,
+    // (2-byte loads, used for K <= 8, stay uncapped: R-MAT K=8 0.293 ms uncapped,
     // 0.326 at 2 waves)
     // (4-byte loads in 8-lane groups, K = 10 and 14: 4 waves; R-MAT K=10 0.358 ms uncapped, 0.346
     // at 4 waves, 0.396 at 2)
@@ -1721,24 +1721,24 @@ __global__ __launch_bounds__(256) void k_place_entries(const PlaceEntries a) {
   const int row = (int)(blockIdx.x * 4 + (threadIdx.x >> 6));
   const int lane = threadIdx.x & 63;
   if (row >= a.m) return;
-  const int b = a.rowptr[row], e = a.rowptr[row + 1];
+  const uint32_t b = (uint32_t)a.rowptr[row], e = (uint32_t)a.rowptr[row + 1];
   const int si = a.split_index[row];
   if (si >= 0) {
     int cur[kXcds];
 #pragma unroll
     for (int x = 0; x < kXcds; ++x) cur[x] = a.cursor[si * kXcds + x];
-    for (int p0 = b; p0 < e; p0 += 64 * kPlaceAhead) {
+    for (uint32_t p0 = b; p0 < e; p0 += 64 * kPlaceAhead) {
       int32_t cs[kPlaceAhead];
       float vs[kPlaceAhead];
 #pragma unroll
       for (int k = 0; k < kPlaceAhead; ++k) {   // steps past the row read its last entry
-        const int q = min(p0 + k * 64 + lane, e - 1);
+        const uint32_t q = entry_ahead(p0, k, lane, e);
         cs[k] = a.col[q];
         vs[k] = a.val_out ? a.val[q] : 0.f;
       }
 #pragma unroll
       for (int k = 0; k < kPlaceAhead; ++k) {
-        const int q = p0 + k * 64 + lane;
+        const uint32_t q = p0 + k * 64 + lane;
         if (p0 + k * 64 >= e) break;
         const bool in = q < e;
         const int32_t c = cs[k];
@@ -1753,7 +1753,7 @@ __global__ __launch_bounds__(256) void k_place_entries(const PlaceEntries a) {
         if (in) {
           a.col_out[dst] = c;
           if (a.val_out) a.val_out[dst] = half_bits_of(__builtin_bit_cast(uint32_t, vs[k]));
-          if (a.x_pos) a.x_pos[dst - a.x_base] = q;
+          if (a.x_pos) a.x_pos[dst - a.x_base] = (int32_t)q;
           if (a.x_src) a.x_src[a.merge_off[si] + (q - b)] = (int32_t)(dst - a.x_base);
         }
       }
@@ -1761,24 +1761,24 @@ __global__ __launch_bounds__(256) void k_place_entries(const PlaceEntries a) {
     if (a.compact) return;
   }
   int out = a.main_rowptr[row];
-  auto place = [&](int q, bool keep, int32_t c, float v) {
+  auto place = [&](uint32_t q, bool keep, int32_t c, float v) {
     const uint64_t mask = __ballot(keep);
     if (keep) {
       const int dst = out + lanes_below(mask);
       a.col_out[dst] = c;
       if (a.val_out) a.val_out[dst] = half_bits_of(__builtin_bit_cast(uint32_t, v));
-      if (a.res_pos) a.res_pos[dst] = q;
+      if (a.res_pos) a.res_pos[dst] = (int32_t)q;
     }
     out += __popcll(mask);
   };
-  int p0 = b;
-  for (; e - p0 > 64; p0 += 64 * kPlaceAhead) {
+  uint32_t p0 = b;
+  for (; p0 + 64 < e; p0 += 64 * kPlaceAhead) {
     int32_t cs[kPlaceAhead];
     float vs[kPlaceAhead];
     uint8_t fs[kPlaceAhead];
 #pragma unroll
     for (int k = 0; k < kPlaceAhead; ++k) {
-      const int q = min(p0 + k * 64 + lane, e - 1);
+      const uint32_t q = entry_ahead(p0, k, lane, e);
       cs[k] = a.col[q];
       vs[k] = a.val_out ? a.val[q] : 0.f;
       fs[k] = a.flag ? a.flag[q] : (uint8_t)0;
@@ -1786,12 +1786,12 @@ __global__ __launch_bounds__(256) void k_place_entries(const PlaceEntries a) {
 #pragma unroll
     for (int k = 0; k < kPlaceAhead; ++k) {
       if (p0 + k * 64 >= e) break;
-      const int q = p0 + k * 64 + lane;
+      const uint32_t q = p0 + k * 64 + lane;
       place(q, q < e && !fs[k], cs[k], vs[k]);
     }
   }
   if (p0 < e) {   // at most one step (most rows are no longer)
-    const int q = p0 + lane;
+    const uint32_t q = p0 + lane;
     const bool keep = q < e && !(a.flag && a.flag[q]);
     place(q, keep, keep ? a.col[q] : 0, keep && a.val_out ? a.val[q] : 0.f);
   }

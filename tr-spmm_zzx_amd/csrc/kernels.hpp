@@ -26,6 +26,13 @@ constexpr int kXcds = 8;
 // and cold columns evenly over the XCDs.
 __host__ __device__ inline int xcd_of_column(int32_t c) { return (int)(((uint32_t)c * 2654435761u) >> 29); }
 
+// Entry of lane `lane` in step k of a wave that walks a row from p0 on, 64 entries a step, or the row's last one past
+// its end e (entry indexes run to 2^31 - 1, the steps ahead past that: unsigned).
+__host__ __device__ inline uint32_t entry_ahead(uint32_t p0, int k, int lane, uint32_t e) {
+  const uint32_t q = p0 + (uint32_t)(k * 64 + lane);
+  return q < e ? q : e - 1;
+}
+
 // SDDMM split rows, merged: out[e] = xbuf[x_src[k_begin + e - e_begin]] for e in [e_begin, e_end),
 // at most kMergeTaskEntries indices per task (a multiple of 256).
 struct MergeTask { int32_t e_begin, e_end, k_begin, pad; };
