@@ -48,7 +48,7 @@ using u64 = unsigned long long;
 constexpr int kSmallU = 8192;       // windows with more distinct columns take the workgroup kernel
 constexpr int kMidU = 2048;         // ... and those with more than this many that share them (wave_window)
 constexpr int kNarrowU = 1024;      // windows of at most this many, the narrow launch of the wave kernel
-constexpr int kFewWide = 1024;      // at most this many wider ones share one launch of the wave kernel
+constexpr int kFewWide = 128;       // at most this many wider ones share one launch of the wave kernel
 constexpr int kBlockWaves = 8;      // waves of that kernel
 constexpr int kLdsUnits = 65536;    // most units whose order it keeps in LDS (16-bit indices; the
                                     // device's LDS per workgroup may allow fewer)
@@ -935,9 +935,9 @@ __device__ __forceinline__ bool wave_window(const Build& B, int32_t w, int32_t U
 // pairs go to the window's part of B.pairs.  The LDS is sized by CAP, so that the many narrow windows
 // run 32 to a CU, not the 8 that kSmallU leaves room for (R-MAT 2^18: 1200 us in one launch -> 325 in two,
 // the windows past kMidU routed by workgroups).  One launch waits for the longest window of the one before,
-// so where the windows past kNarrowU are few (kFewWide; *wide of them) the widest launch takes them all: the chip
-// holds 1792 of its workgroups at once (grid of 223^2 nodes, 64 windows of a hub row: 255 us in three launches, 161
-// in two, 136 in the one of all windows).
+// so where the windows past kNarrowU are few (kFewWide; *wide of them) the widest launch takes them all (grid of
+// 223^2 nodes, 64 windows of a hub row: 255 us in three launches, 161 in two, 136 in the one of all windows; R-MAT
+// 2^18, some hundreds of them: 332 in three, 543 in two).
 template <int LO, int CAP>
 __global__ __launch_bounds__(64) void k_plan_small(Build B, const int32_t* __restrict__ wide) {
   const int32_t w = blockIdx.x;
