@@ -214,11 +214,14 @@ typedef struct trs_plan_options {
   int32_t mfma_sptc;      /* 1: 2:4 group tiles whose fill >= sptc_min_fill run on MFMA */
   float sptc_min_fill;    /* fill threshold (nnz / 256 slots of a 16x16 tile) for mfma_sptc */
   int32_t task_nnz;       /* residual nnz per lane-group task packing short rows (0 = automatic:
-                             about four mean rows, 32..128, and smaller -- down to 16 -- where
-                             that leaves fewer than 16,384 tasks) */
+                             about four mean rows, 32..128, and smaller for plans of less than
+                             3,145,728 residual entries: 16 or 32, or 16,384 tasks where no row is
+                             longer than a task; larger ones for SDDMM lane groups of 16 lanes) */
   int32_t piece_nnz;      /* longest residual run one lane group walks; longer rows are split
-                             into pieces summed by the fixup kernel (0 = automatic: 256, or 64
-                             where the automatic task size leaves fewer than 16,384 tasks) */
+                             into pieces summed by the fixup kernel (0 = automatic: 32 below
+                             786,432 residual entries, 64 below 3,145,728, then 256, or 128 where
+                             rows are short and the entries less than 5 to 6 million; a longest row
+                             of at most two pieces stays whole) */
   int32_t feature_lanes;  /* lanes per lane group (power of two <= 64; each lane holds 8 features):
                              fewer lanes = several feature passes with a smaller B working set
                              per pass (0 = automatic) */
@@ -237,21 +240,23 @@ typedef struct trs_plan_options {
   int32_t sddmm_unroll;   /* SDDMM residual entries in flight per lane group: 4 or 8; 0 = automatic
                              (4 for passes of exactly 128 features with 16-byte loads, else 8) */
   int32_t stage;          /* a residual task's column ids (and values) are copied into LDS once
-                             before its gathers: 0 = automatic (16-lane groups, i.e. K = 65..128,
-                             and tasks of <= 256 entries), -1 = never */
+                             before its gathers: 0 = automatic (16-lane groups and
+                             tasks of <= 256 entries), -1 = never */
   int32_t occupancy;      /* waves per SIMD the residual task kernels may hold (2..8; values
                              outside are clamped): fewer concurrent tasks keep fewer gathered rows
-                             in flight.  0 = automatic (SpMM: 2 for K <= 64, uncapped above;
-                             SDDMM: uncapped), -1 = uncapped (as many as registers and LDS allow) */
+                             in flight.  0 = automatic (SpMM: 2 for lane groups of at most 8
+                             lanes of 8- or 16-byte loads, 4 of 4-byte loads, else uncapped -- so
+                             K <= 32 for the most part; SDDMM: uncapped), -1 = uncapped (as many
+                             as registers and LDS allow) */
   int32_t xcd_split;      /* XCD column split: the columns are divided among the 8 XCDs by a hash
                              and residual rows with at least this many entries are cut into one
                              sub-row per XCD, run by that XCD's workgroups (workgroup i runs on XCD
                              i mod 8), so each XCD's L2 holds B (or Y) rows of an eighth of the
                              columns; an SpMM sub-row costs a partial slot, an SDDMM sub-row entry
                              an output index (SDDMM uses the split from K = 128 on).
-                             0 = automatic (SpMM 256, SDDMM 512, and only when those rows read
-                             their columns at least 4 times each on average: no L2 reuse to gain
-                             otherwise), -1 = off */
+                             0 = automatic (SpMM 256, or 512 below 3,145,728 residual entries;
+                             SDDMM 512; and only when those rows read their columns at least 4
+                             times each on average: no L2 reuse to gain otherwise), -1 = off */
   int32_t host_lowering;  /* trs_plan_create only.  0: when the format holds its input CSR (a format
                              built in this process from canonical input), the MFMA tiles are cut
                              from the format on the host and the residual (the input CSR minus the
@@ -268,7 +273,10 @@ typedef struct trs_plan_options {
                              kernels gather most are copied into a dense buffer at the start of a
                              call (workspace), and the task kernels read them there; the plan keeps
                              a second copy of its column ids with those columns renumbered.  Used
-                             for K >= 128 (K % 8 == 0) on 16-byte aligned operands.  0 = automatic
+                             for K >= 128 (K % 8 == 0; SDDMM not where K = 129..256 takes one
+                             pass), and padded for widths that 8 does not divide: SpMM odd K >= 65
+                             and even K >= 104 but K = 132, 140..252, SDDMM K >= 121 (up to 127 from
+                             48 MB of Y on).  0 = automatic
                              (32768 rows, at most n / 16, and only when they take >= 30% of the
                              gathers), > 0 = that many rows, -1 = off.  Never for plans with more
                              than 4 columns per entry (n > 4 nnz) */
@@ -385,7 +393,7 @@ void trs_plan_free(trs_plan* p);
  * ------------------------------------------------------------------------------------------- */
 /* Bytes of device workspace trs_spmm_f16 needs for feature width K (0 when none): the partial
  * slots of split rows and, for K >= 128, the plan's staged hot B rows (option hot_rows).  For K that 8
- * does not divide the staged rows (odd K >= 65, even K >= 104) are optional: a workspace that only
+ * does not divide the staged rows (see hot_rows) are optional: a workspace that only
  * holds the partial slots is accepted, and the call then runs without them, the same bits. */
 int64_t trs_spmm_workspace_bytes(const trs_plan* p, int32_t K);
 
@@ -422,10 +430,13 @@ int trs_sddmm_f16(const trs_plan* p, const uint16_t* X, int64_t ldx, const uint1
  * buffer for the plan's split part (XCD sub-rows of its long rows, merged into place at the end of
  * the call) and the plan's staged hot Y rows (plan option hot_rows); 0 when the plan or K uses
  * neither.  For K that 8 does not divide the staged rows (K >= 121) are optional, as for the SpMM.
- * No reference counterpart. */
+ * Calls of one feature pass (K = 129..256 on plans without staged rows or split part, or within 16 to 128 MB of
+ * Y) use the output buffer only: they accept a workspace that holds no more, though the size named here for K
+ * that 8 divides has room for the staged rows.  No reference counterpart. */
 int64_t trs_sddmm_workspace_bytes(const trs_plan* p, int32_t K);
 
-/* trs_sddmm_f16 with a workspace of trs_sddmm_workspace_bytes(p, K) bytes (fewer: TRS_EINVAL):
+/* trs_sddmm_f16 with a workspace of trs_sddmm_workspace_bytes(p, K) bytes (fewer, but for what it calls
+ * optional or unused: TRS_EINVAL):
  * the call copies the plan's hot Y rows there before the dot products gather them, and its split
  * part writes its outputs there in its own order before a merge puts them in place.  The same
  * outputs, bitwise (only where rows are read from and sums written to changes); trs_sddmm_f16
