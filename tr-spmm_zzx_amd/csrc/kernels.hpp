@@ -180,7 +180,8 @@ struct TaskSizes {
 // of 32 25.2 / 41.9 / 82.5, of 64 26.6 / 36.1 / 78.4); K <= 32 those of SpMM, even tiny plans at most 24 (ER of 28,439
 // nodes K = 16 / 32, of 16 9.7 / 10.8, 22 8.0 / 8.5, 30 9.6 / 9.9; of 60,000 nodes, 10 a row 12.3 / 14.2, 11.9 / 13.7,
 // 11.2 / 14.0, of 45 13.2 / 18.1).  With a split part that is for those who walk whole rows, K < 128; K >=
-// 128 take 16 (R-MAT 2^14 K = 128, of 16 22.4, of 28 27.8).  From 393K on the pieces of those who walk whole rows hold 64 (R-MAT 2^14 K = 80 / 96 22.3 / 23.0 with 32, 20.1 / 20.6 with 64; R-MAT 2^13, 150K, K = 64 8.7, 12.1).
+// 128 take 16 (R-MAT 2^14 K = 128, of 16 22.4, of 28 27.8).  From 393K on the pieces of those who walk whole rows hold
+// 64 (R-MAT 2^14 K = 80 / 96 22.3 / 23.0 with 32, 20.1 / 20.6 with 64; R-MAT 2^13, 150K, K = 64 8.7, 12.1).
 // Past kSmallEntries pieces of 128 pay where rows are short, and up to 5M entries, or 6M where the long rows are
 // split: a piece is a partial slot, written and summed again at every width (SpMM us, K = 16 / 64 / 128 / 200, pieces
 // of 128 / 256: R-MAT 2^19 with 4.9M entries, 20 a row 66 / 98 / 155 / 345, 90 / 106 / 168 / 354, with 5.9M, 22 a row 72
